@@ -263,7 +263,7 @@ extern "C" int mcl_create(int device, mcl_ctx **out)
     int per_cu_m = 0;
     hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_m, (const void *)k_uzawa_mixed, MCL_BLOCK, 0);
     int per_cu = std::min(std::min(per_cu_u, per_cu_h), per_cu_m);
-    c->max_coop_blocks = std::min(std::max(1, per_cu) * c->num_cu, MCL_MAX_WG);
+    c->max_coop_blocks = std::min(std::max(1, per_cu) * c->num_cu, MCL_SYNC_WG);
     // grid barrier and reduction buffers
     unsigned *sync = nullptr;
     if (dev_alloc(c, c->owned, &sync, MCL_SYNC_WORDS)) { delete c; return MCL_E_DEVICE; }

@@ -307,7 +307,7 @@ __device__ double seq_dot(const double *__restrict__ x, const double *__restrict
 // Returns the iteration count; *ok is cleared if a barrier aborted.
 __device__ int pcg_persistent(const LevelDev &L, const EllMat &A, const double *__restrict__ b,
                               double *__restrict__ x, bool x_zero, double accu, int max_cycle, int precond,
-                              int kind, CgVecs v, const GridSync &gs, unsigned &gen, const RedBuf &rb,
+                              int kind, CgVecs v, const GridSync &gs, WaitState &ws, const RedBuf &rb,
                               dd (*lds)[MCL_BLOCK / MCL_WAVE], double *ldsm, bool &ok, long long &spmv,
                               bool exact)
 {
@@ -326,7 +326,7 @@ __device__ int pcg_persistent(const LevelDev &L, const EllMat &A, const double *
         if (!x_zero) spmv++;
         reduce_publish<1>(rb, 0, acc, lds);
     }
-    ok = ok && grid_sync(gs, gen);
+    ok = ok && grid_sync(gs, ws);
     double delta_new;
     {
         double o[1];
@@ -347,7 +347,7 @@ __device__ int pcg_persistent(const LevelDev &L, const EllMat &A, const double *
             spmv++;
             reduce_publish<1>(rb, 1, acc, lds);
         }
-        ok = ok && grid_sync(gs, gen);
+        ok = ok && grid_sync(gs, ws);
         double t1;
         {
             double o[1];
@@ -357,12 +357,12 @@ __device__ int pcg_persistent(const LevelDev &L, const EllMat &A, const double *
         const double alpha = delta_new / t1;
         for (int i = gtid; i < n; i += gsize) x[i] += alpha * v.d[i];
         if (L.nh > 0) {
-            ok = ok && grid_sync(gs, gen);
+            ok = ok && grid_sync(gs, ws);
             if (kind == 0) constrain_v(L, x, gtid, gsize);
             else constrain_T(L, x, gtid, gsize);
         }
         const bool recompute = (cycle % 50) == 0;
-        if (recompute) ok = ok && grid_sync(gs, gen);
+        if (recompute) ok = ok && grid_sync(gs, ws);
         double delta_old = delta_new;
         {
             dd acc[1] = {dd_zero()};
@@ -382,7 +382,7 @@ __device__ int pcg_persistent(const LevelDev &L, const EllMat &A, const double *
             double bm = block_max(mx, ldsm);
             if (threadIdx.x == 0) rb.pmax[0 * MCL_MAX_WG + blockIdx.x] = bm;
         }
-        ok = ok && grid_sync(gs, gen);
+        ok = ok && grid_sync(gs, ws);
         double res;
         {
             double o[1];
@@ -396,7 +396,7 @@ __device__ int pcg_persistent(const LevelDev &L, const EllMat &A, const double *
         for (int i = gtid; i < n; i += gsize) v.d[i] = v.s[i] + beta * v.d[i];
         cycle++;
         bool brk = precond ? (res < accu) : (kind == 0 ? res < accu : (res < accu && cycle > 10));
-        ok = ok && grid_sync(gs, gen);
+        ok = ok && grid_sync(gs, ws);
         if (brk) break;
     }
     return cycle;
@@ -413,7 +413,7 @@ __device__ int pcg_persistent(const LevelDev &L, const EllMat &A, const double *
 // between two reduction slots, so a workgroup writing a slot two sweeps later
 // cannot overtake a slower one still reading it.
 __device__ int jacobi_grid(const EllMat &A, const double *__restrict__ b, double *x, double *xt, double accu,
-                           int max_cycle, const GridSync &gs, unsigned &gen, const RedBuf &rb, double *ldsm, bool &ok,
+                           int max_cycle, const GridSync &gs, WaitState &ws, const RedBuf &rb, double *ldsm, bool &ok,
                            long long &spmv)
 {
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsize = gridDim.x * blockDim.x;
@@ -439,7 +439,7 @@ __device__ int jacobi_grid(const EllMat &A, const double *__restrict__ b, double
         const int slot = 4 + (cycle & 1);
         double bm = block_max(mx, ldsm);
         if (threadIdx.x == 0) rb.pmax[slot * MCL_MAX_WG + blockIdx.x] = bm;
-        ok = ok && grid_sync(gs, gen);
+        ok = ok && grid_sync(gs, ws);
         double m = 0.0;
         for (int bb = threadIdx.x; bb < (int)gridDim.x; bb += MCL_BLOCK) m = fmax(m, rb.pmax[slot * MCL_MAX_WG + bb]);
         const double diff = block_max(m, ldsm);
@@ -451,7 +451,7 @@ __device__ int jacobi_grid(const EllMat &A, const double *__restrict__ b, double
     }
     if (src != x) {
         for (int i = gtid; i < n; i += gsize) x[i] = src[i];
-        ok = ok && grid_sync(gs, gen);
+        ok = ok && grid_sync(gs, ws);
     }
     return cycle;
 }
@@ -559,25 +559,25 @@ __device__ int mg_block(const GsLevelDev *lv, int nl, const double *b, double *x
 
 // The inner solve of citcom_solver (Solver.c:82-89) for the chosen solver.
 __device__ int inner_solve(const UzawaParams &P, const LevelDev &L, const EllMat &K, const double *b, double *x,
-                           bool x_zero, CgVecs cv, unsigned &gen, dd (*lds)[MCL_BLOCK / MCL_WAVE], double *ldsm,
+                           bool x_zero, CgVecs cv, WaitState &ws, dd (*lds)[MCL_BLOCK / MCL_WAVE], double *ldsm,
                            bool &ok, long long &spmv)
 {
     switch (P.solver) {
     case MCL_INNER_JC:
-        return jacobi_grid(K, b, x, P.xt, P.accuracy, 1000, P.gs, gen, P.rb, ldsm, ok, spmv);
+        return jacobi_grid(K, b, x, P.xt, P.accuracy, 1000, P.gs, ws, P.rb, ldsm, ok, spmv);
     case MCL_INNER_GS: {
         const int c = gs_block(P.gsl[P.ngsl - 1], b, x, P.xt, P.accuracy, 1000, ldsm, spmv);
-        ok = ok && grid_sync(P.gs, gen);
+        ok = ok && grid_sync(P.gs, ws);
         return c;
     }
     case MCL_INNER_MG: {
         const int c = mg_block(P.gsl, P.ngsl, b, x, P.xt2, P.xt, P.accuracy, P.mg_cycle, P.mg_finest_iteration,
                                P.mg_coarse_iteration, ldsm, spmv);
-        ok = ok && grid_sync(P.gs, gen);
+        ok = ok && grid_sync(P.gs, ws);
         return c;
     }
     default:
-        return pcg_persistent(L, K, b, x, x_zero, P.accuracy, P.max_cg_cycle, P.cg_precondition, 0, cv, P.gs, gen,
+        return pcg_persistent(L, K, b, x, x_zero, P.accuracy, P.max_cg_cycle, P.cg_precondition, 0, cv, P.gs, ws,
                               P.rb, lds, ldsm, ok, spmv, P.exact_dots != 0);
     }
 }
@@ -591,8 +591,8 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsize = gridDim.x * blockDim.x;
     const int neq = L.neq, nel = L.nel;
     if (blockIdx.x == 0 && threadIdx.x == 0) P.stats->t_begin = wall_clock64();
-    unsigned gen = __hip_atomic_load(P.gs.gen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-    bool ok = true;
+    WaitState ws;
+    bool ok = sync_begin(P.gs, ws);
     long long spmv = 0, inner = 0;
     EllMat K{L.Kcol, L.Kncol, L.Kval, L.Kdiag, nullptr, neq};
     CgVecs cv{P.cg_r, P.cg_s, P.cg_d, P.cg_q};
@@ -616,10 +616,10 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
         P.Ahv[i] = L.F[i] - gp - u;
     }
     spmv++;
-    ok = ok && grid_sync(P.gs, gen);
-    inner += inner_solve(P, L, K, P.Ahv, P.u1, false, cv, gen, lds, ldsm, ok, spmv);
+    ok = ok && grid_sync(P.gs, ws);
+    inner += inner_solve(P, L, K, P.Ahv, P.u1, false, cv, ws, lds, ldsm, ok, spmv);
     for (int i = gtid; i < neq; i += gsize) P.d[i] += P.u1[i];
-    ok = ok && grid_sync(P.gs, gen);
+    ok = ok && grid_sync(P.gs, ws);
     double *r0 = P.r0, *r1 = P.r1, *r2 = P.r2, *z0 = P.z0, *z1 = P.z1, *s1 = P.s1, *s2 = P.s2;
     for (int e = gtid; e < nel; e += gsize) r1[e] = gt_elem(L, e, P.d);
     double dv = 1.0, dp = 1.0;
@@ -637,7 +637,7 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
             }
             reduce_publish<2>(P.rb, 4, acc, lds);
         }
-        ok = ok && grid_sync(P.gs, gen);
+        ok = ok && grid_sync(P.gs, ws);
         double r1z1, delta = 0.0;
         {
             double o[2];
@@ -651,14 +651,14 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
         }
         if (!(r1z1 == r1z1)) P.stats->nan_flag = 1;
         for (int e = gtid; e < nel; e += gsize) s2[e] = cycle == 0 ? z1[e] : z1[e] + delta * s1[e];
-        ok = ok && grid_sync(P.gs, gen);
+        ok = ok && grid_sync(P.gs, ws);
         // Ah = G s2 ; u1 = 0 ; K u1 = Ah
         for (int i = gtid; i < neq; i += gsize) {
             P.Ahv[i] = g_row(L, i, s2);
             P.u1[i] = 0.0;
         }
-        ok = ok && grid_sync(P.gs, gen);
-        inner += inner_solve(P, L, K, P.Ahv, P.u1, true, cv, gen, lds, ldsm, ok, spmv);
+        ok = ok && grid_sync(P.gs, ws);
+        inner += inner_solve(P, L, K, P.Ahv, P.u1, true, cv, ws, lds, ldsm, ok, spmv);
         // Ah = G^T u1 ; alpha = r1.z1 / s2.Ah
         {
             dd acc[1] = {dd_zero()};
@@ -669,7 +669,7 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
             }
             reduce_publish<1>(P.rb, 6, acc, lds);
         }
-        ok = ok && grid_sync(P.gs, gen);
+        ok = ok && grid_sync(P.gs, ws);
         double alpha;
         {
             double o[1];
@@ -695,7 +695,7 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
             }
             reduce_publish<4>(P.rb, 8, acc, lds);
         }
-        ok = ok && grid_sync(P.gs, gen);
+        ok = ok && grid_sync(P.gs, ws);
         {
             double o[4];
             reduce_collect<4>(P.rb, 8, gridDim.x, o, lds);
@@ -724,6 +724,7 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
         if (!(dv == dv) || !(dp == dp)) P.stats->nan_flag = 1;
         P.stats->t_end = wall_clock64();
     }
+    sync_end(P.gs, ws);
 }
 
 // Zero n 32-bit words (a kernel rather than hipMemsetAsync, so that a caller
@@ -931,8 +932,8 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_heat_fp64(HeatParams H)
     const LevelDev &L = H.L;
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsize = gridDim.x * blockDim.x;
     const int n = L.neqT, nel = L.nel;
-    unsigned gen = __hip_atomic_load(H.gs.gen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-    bool ok = true;
+    WaitState ws;
+    bool ok = sync_begin(H.gs, ws);
     long long spmv = 0;
     // tau per element and the advective dt bound
     double dtmin = 1e10;
@@ -960,7 +961,7 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_heat_fp64(HeatParams H)
         double bm = block_min(dtmin, ldsm);
         if (threadIdx.x == 0) H.rb.pmax[1 * MCL_MAX_WG + blockIdx.x] = bm;
     }
-    ok = ok && grid_sync(H.gs, gen);
+    ok = ok && grid_sync(H.gs, ws);
     for (int P = gtid; P < n; P += gsize) heat_assemble_row(L, H, P);
     double dt;
     {
@@ -973,7 +974,7 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_heat_fp64(HeatParams H)
         dt = dt < H.diff_dt ? dt : H.diff_dt;
         dt = dt * 0.75;
     }
-    ok = ok && grid_sync(H.gs, gen);
+    ok = ok && grid_sync(H.gs, ws);
     EllMat Kh{L.Tcol, L.Tncol, H.hK, nullptr, L.Tdiag_slot, n};
     EllMat Ch{L.Tcol, L.Tncol, H.hC, nullptr, L.Tdiag_slot, n};
     EllMat Ah{L.Tcol, L.Tncol, H.hA, nullptr, L.Tdiag_slot, n};
@@ -982,13 +983,13 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_heat_fp64(HeatParams H)
     if (H.first_call) {
         // initial_T_dot (:179-239)
         for (int i = gtid; i < n; i += gsize) H.hd[i] = H.T[L.heq_node[i]];
-        ok = ok && grid_sync(H.gs, gen);
+        ok = ok && grid_sync(H.gs, ws);
         for (int i = gtid; i < n; i += gsize) {
             H.B[i] = H.hF[i] - ell_row(L.Tcol, H.hK, L.Tncol[i], n, i, H.hd);
             H.hdd[i] = 0.0;
         }
-        ok = ok && grid_sync(H.gs, gen);
-        init_cycles = pcg_persistent(L, Ch, H.B, H.hdd, true, 1e-3, 400, H.cg_precondition, 1, cv, H.gs, gen,
+        ok = ok && grid_sync(H.gs, ws);
+        init_cycles = pcg_persistent(L, Ch, H.B, H.hdd, true, 1e-3, 400, H.cg_precondition, 1, cv, H.gs, ws,
                                      H.rb, lds, ldsm, ok, spmv, H.exact_dots != 0);
     }
     const double td = H.theta * dt;
@@ -998,8 +999,8 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_heat_fp64(HeatParams H)
         H.B[i] = H.hF[i] + ct / td;
         for (int s = 0; s < L.Tncol[i]; s++) H.hA[s * n + i] = H.hC[s * n + i] / td + H.hK[s * n + i];
     }
-    ok = ok && grid_sync(H.gs, gen);
-    int cycles = pcg_persistent(L, Ah, H.B, H.hd, false, 1e-3, 1000, H.cg_precondition, 1, cv, H.gs, gen, H.rb, lds,
+    ok = ok && grid_sync(H.gs, ws);
+    int cycles = pcg_persistent(L, Ah, H.B, H.hd, false, 1e-3, 1000, H.cg_precondition, 1, cv, H.gs, ws, H.rb, lds,
                                 ldsm, ok, spmv, H.exact_dots != 0);
     for (int i = gtid; i < L.nno; i += gsize) {
         int k = L.heat_id[i];
@@ -1014,4 +1015,5 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_heat_fp64(HeatParams H)
         H.stats->aborted = ok ? 0 : 1;
         *H.model_time += dt;
     }
+    sync_end(H.gs, ws);
 }

@@ -244,12 +244,9 @@ __device__ __forceinline__ MCL_G T *gp(T *p)
 
 // Vector accesses of the V-cycle.  CO = true for vectors of the grid levels
 // between neighbour waits: agent-scope atomic loads and stores (coherent
-// across the XCDs' L2 caches, see nbr_sync_coherent); CO = false for LDS
-// vectors and plain global accesses.
-#ifndef MCL_VCYCLE_COHERENT
-#define MCL_VCYCLE_COHERENT 1
-#endif
-constexpr bool kCO = MCL_VCYCLE_COHERENT != 0;
+// across the XCDs' L2 caches, see GridSync); CO = false for LDS vectors and
+// plain global accesses.
+constexpr bool kCO = true;
 
 template <bool CO, typename Ptr>
 __device__ __forceinline__ float vld(Ptr p)
@@ -877,14 +874,13 @@ __device__ __forceinline__ void deep_down_last(const GLevel &F, LB buf, float wf
 // (x_c the coarse result, CC its access mode), sweep 3 on W, sweep 4 on the
 // workgroup's own rows, written to F.x (the buffer of x_1/x_3: its
 // neighbours still read x_2 in this phase).  On the finest level sweep 4 is
-// z, zeroed on hanging equations, with sum r_i z_i published to `slot`.  The
+// z, zeroed on hanging equations, with sum r_i z_i added to rz.  The
 // operations and their order are those of prolong_add, jacobi and
 // last_sweep_rz.
 // deep_up for lists of at most MCL_BLOCK rows (false: not applicable)
 template <bool CC, typename XC, typename LB>
 __device__ __forceinline__ bool deep_up1(const GLevel &F, const Halo2 &h, XC xc, LB buf, float w, bool finest,
-                                         const MixedParams &P, const double *__restrict__ r, int slot,
-                                         dd (*lds)[MCL_BLOCK / MCL_WAVE])
+                                         const MixedParams &P, const double *__restrict__ r, dd &rz)
 {
     if (F.WK != 18 || h.nV > MCL_BLOCK) return false;
     const int t = threadIdx.x;
@@ -916,26 +912,24 @@ __device__ __forceinline__ bool deep_up1(const GLevel &F, const Halo2 &h, XC xc,
     __syncthreads();
     if (rv >= 0 && t < h.nW) xW[t] = xV[t] + w * dW * (bW - krow_dot(kw, xV));
     __syncthreads();
-    dd acc[1] = {dd_zero()};
     if (t < h.o.no) {
         float z = xW[t] + w * dW * (bW - krow_dot(kw, xW));
         if (finest) {
             const LevelDev &L = P.U.L;
             if (L.nh > 0 && L.hp_n[rv] != 0) z = 0.f;  // z lives in the constrained space
-            acc[0] = dd_add_prod(acc[0], r[rv], (double)z);
+            rz = dd_add_prod(rz, r[rv], (double)z);
         }
         vst<kCO>(F.x + rv, z);
     }
-    if (finest) reduce_publish<1>(P.U.rb, slot, acc, lds);
     return true;
 }
 
 template <bool CC, typename XC, typename LB>
 __device__ __forceinline__ void deep_up(const GLevel &F, XC xc, LB buf, float w, bool finest, const MixedParams &P,
-                                        const double *__restrict__ r, int slot, dd (*lds)[MCL_BLOCK / MCL_WAVE])
+                                        const double *__restrict__ r, dd &rz)
 {
     const Halo2 h = halo2(F);
-    if (deep_up1<CC>(F, h, xc, buf, w, finest, P, r, slot, lds)) return;
+    if (deep_up1<CC>(F, h, xc, buf, w, finest, P, r, rz)) return;
     const auto xV = buf;
     const auto xW = buf + h.nV;
     const auto x2 = sweep_buf(F, 2);
@@ -967,45 +961,31 @@ __device__ __forceinline__ void deep_up(const GLevel &F, XC xc, LB buf, float w,
     }
     __syncthreads();
     const LevelDev &L = P.U.L;
-    dd acc[1] = {dd_zero()};
     for (int i = h.o.b0 + (int)threadIdx.x; i < h.o.b0 + h.o.no; i += blockDim.x) {
         float z = xW[i - h.o.b0] + w * F.dinv[i] * (vld<kCO>(F.b + i) - ell32c<false>(F.WK, F.n, F.kl, F.val, i, xW));
         if (finest) {
             if (L.nh > 0 && L.hp_n[i] != 0) z = 0.f;  // z lives in the constrained space
-            acc[0] = dd_add_prod(acc[0], r[i], (double)z);
+            rz = dd_add_prod(rz, r[i], (double)z);
         }
         vst<kCO>(F.x + i, z);
     }
-    if (finest) reduce_publish<1>(P.U.rb, slot, acc, lds);
-}
-
-// Grid-wide wait between phases whose cross-workgroup data is accessed only
-// with agent-scope atomics (no cache maintenance), or a fenced grid barrier
-// when the V-cycle runs with plain accesses.
-__device__ __forceinline__ bool csync(const GridSync &gs, unsigned &gen, bool ok)
-{
-    if constexpr (kCO) return ok && grid_sync_coherent(gs, gen);
-    else return ok && grid_sync(gs, gen);
 }
 
 // Wait between two stencil phases of the V-cycle: only for the workgroups in
 // this workgroup's neighbour list (thread t polls neighbour t; nbr < 0: none),
 // or for the whole grid when the lists are off.
-__device__ __forceinline__ bool vsync(const GridSync &gs, unsigned &gen, bool ok, int nbr, bool use_nbr)
+__device__ __forceinline__ bool vsync(const GridSync &gs, WaitState &ws, bool ok, int nbr, bool use_nbr)
 {
+    if (!use_nbr) return ok && grid_wait(gs, ws);
 #if MCL_WAIT_TIMERS
     // split of the neighbour waits: work before the wait (12), the wait (13)
     MCL_PHASE(12);
-    bool r;
-    if (!use_nbr) r = ok && grid_sync(gs, gen);
-    else if constexpr (kCO) r = ok && nbr_sync_coherent(gs, gen, nbr);
-    else r = ok && nbr_sync(gs, gen, nbr);
+    const bool r = ok && nbr_sync(gs, ws, nbr);
     MCL_PHASE(13);
     return r;
+#else
+    return ok && nbr_sync(gs, ws, nbr);
 #endif
-    if (!use_nbr) return ok && grid_sync(gs, gen);
-    if constexpr (kCO) return ok && nbr_sync_coherent(gs, gen, nbr);
-    else return ok && nbr_sync(gs, gen, nbr);
 }
 
 // Copy of the LDS levels' matrices into the workgroup's LDS block.
@@ -1041,25 +1021,23 @@ __device__ __forceinline__ void coarse_solve(const MixedParams &P, const LdsLeve
 }
 
 // Finest level's last post-sweep z = x_{2 pre}, fused with sum r_i z_i
-// (published to reduction slot `slot`).
+// (added to rz).
 __device__ __forceinline__ void last_sweep_rz(const MixedParams &P, const MgLds &mgl, const double *__restrict__ r,
-                                              int slot, dd (*lds)[MCL_BLOCK / MCL_WAVE])
+                                              dd &rz)
 {
     const GLevel A = glevel(mgl.lev + P.nmg - 1);
     const float w = P.omega / mgl.lam[P.nmg - 1];
     const int kf = 2 * P.pre;
     const auto in = sweep_buf(A, kf - 1);
     const auto out = sweep_buf(A, kf);
-    dd acc[1] = {dd_zero()};
     const Ex ex = own_rows(A.n);
     const LevelDev &L = P.U.L;
     for (int i = ex.b; i < ex.e; i += ex.s) {
         float zi = vld<kCO>(in + i) + w * A.dinv[i] * (vld<kCO>(A.b + i) - ell32<kCO>(A, i, in));
         if (L.nh > 0 && L.hp_n[i] != 0) zi = 0.f;  // z lives in the constrained space
         vst<kCO>(out + i, zi);
-        acc[0] = dd_add_prod(acc[0], r[i], (double)zi);
+        rz = dd_add_prod(rz, r[i], (double)zi);
     }
-    reduce_publish<1>(P.U.rb, slot, acc, lds);
 }
 
 // Whether a grid level runs its two-sweep phases (needs pre = 2 and the lists).
@@ -1077,8 +1055,8 @@ __device__ __forceinline__ MCL_G float *level_result(const MixedParams &P, const
 
 // The V-cycle after the finest level's right-hand side and first sweep are in
 // place and synchronised, through the finest level's last post-sweep z with
-// sum r_i z_i published to reduction slot `slot` (the caller waits on the
-// grid before reading it or z).
+// this thread's part of sum r_i z_i in rz (the caller's grid wait reduces it
+// and completes z).
 //  * grid levels (lb+1 .. top): rows spread over the grid, neighbour waits;
 //    with pre = 2 each level's down leg (sweep 2, residual, restriction) and
 //    up leg (prolongation, sweeps 3 and 4) run as one phase each over the
@@ -1088,9 +1066,8 @@ __device__ __forceinline__ MCL_G float *level_result(const MixedParams &P, const
 //    identically, with its vectors and matrices in LDS and workgroup barriers
 //    only, so no workgroup waits on another and level lb+1 prolongates from
 //    its own LDS.
-__device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &mgl, const GridSync &gs, unsigned &gen,
-                                            bool &ok, int nbr, const double *__restrict__ r, int slot,
-                                            dd (*lds)[MCL_BLOCK / MCL_WAVE])
+__device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &mgl, const GridSync &gs, WaitState &ws,
+                                            bool &ok, int nbr, const double *__restrict__ r, dd &rz)
 {
     const int top = P.nmg - 1, pre = P.pre, kf = 2 * P.pre;
     const bool un = P.use_nbr != 0;
@@ -1105,17 +1082,17 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
         if (deep_down_on(P, A)) {
             if (l - 1 > lb) {
                 deep_down(A, glevel(mgl.lev + l - 1), mgl.halo, w, P.omega / lam[l - 1]);
-                ok = vsync(gs, gen, ok, nbr, un);
+                ok = vsync(gs, ws, ok, nbr, un);
             } else {
                 // every workgroup restricts the whole residual into its LDS
                 deep_down_last(A, mgl.halo, w);
-                ok = csync(gs, gen, ok);
+                ok = ok && grid_wait(gs, ws);
             }
             continue;
         }
         for (int k = 2; k <= pre; k++) {
             jacobi<kCO>(A, k, w, ex);
-            ok = vsync(gs, gen, ok, nbr, un);
+            ok = vsync(gs, ws, ok, nbr, un);
         }
         if (l - 1 > lb) {
             const GLevel C = glevel(mgl.lev + l - 1);
@@ -1123,14 +1100,14 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
                 fused_down(A, C, mgl.halo, P.omega / lam[l - 1], pre);
             } else {
                 residual<kCO>(A, sweep_buf(A, pre), ex);
-                ok = vsync(gs, gen, ok, nbr, un);
+                ok = vsync(gs, ws, ok, nbr, un);
                 restrict_to<kCO, kCO>(C, A, true, P.omega / lam[l - 1], own_rows(C.n));
             }
-            ok = vsync(gs, gen, ok, nbr, un);
+            ok = vsync(gs, ws, ok, nbr, un);
         } else {
             // every workgroup restricts the whole residual into its LDS
             residual<kCO>(A, sweep_buf(A, pre), ex);
-            ok = csync(gs, gen, ok);
+            ok = ok && grid_wait(gs, ws);
         }
     }
     MCL_PHASE(2);
@@ -1179,11 +1156,11 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
         if (deep_up_on(P, A)) {
             if (l - 1 == lb) {
                 const LdsLevel C = lds_level(mgl, lb, pre);
-                deep_up<false>(A, sweep_buf(C, kf), mgl.halo, w, finest, P, r, slot, lds);
+                deep_up<false>(A, sweep_buf(C, kf), mgl.halo, w, finest, P, r, rz);
             } else {
-                deep_up<kCO>(A, level_result(P, glevel(mgl.lev + l - 1)), mgl.halo, w, finest, P, r, slot, lds);
+                deep_up<kCO>(A, level_result(P, glevel(mgl.lev + l - 1)), mgl.halo, w, finest, P, r, rz);
             }
-            if (!finest) ok = vsync(gs, gen, ok, nbr, un);
+            if (!finest) ok = vsync(gs, ws, ok, nbr, un);
             continue;
         }
         const int kend = finest ? kf - 1 : kf;
@@ -1199,12 +1176,12 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
             if (fuse) fused_up<kCO>(A, xc, mgl.halo, w, pre);
             else prolong_add<kCO, kCO>(A, sweep_buf(A, pre), xc, ex);
         }
-        ok = vsync(gs, gen, ok, nbr, un);
+        ok = vsync(gs, ws, ok, nbr, un);
         for (int k = fuse ? pre + 2 : pre + 1; k <= kend; k++) {
             jacobi<kCO>(A, k, w, ex);
-            ok = vsync(gs, gen, ok, nbr, un);
+            ok = vsync(gs, ws, ok, nbr, un);
         }
-        if (finest) last_sweep_rz(P, mgl, r, slot, lds);
+        if (finest) last_sweep_rz(P, mgl, r, rz);
     }
     MCL_PHASE(4);
 }
@@ -1259,16 +1236,15 @@ __device__ __forceinline__ double ct_gather(const LevelDev &L, int i, double yi,
 // The caller writes b on this thread's rows (own_rows(neq)) in the phase
 // that calls the solve, so the start needs no barrier before it (with
 // hanging nodes the start reads b across rows: the caller waits on the grid
-// first).  With collect_ff the caller has published |F|^2 to slot 5 in that
-// phase and ff receives it.  x is stored with agent-scope stores and is
+// first).  facc: this thread's part of |F|^2 from that phase; with collect_ff
+// it is summed into ff.  x is stored with agent-scope stores and is
 // complete for agent-scope loads on return, which follows a barrier (with
 // hanging nodes, a fenced one after the expansion u = C u_f).
-// Reduction slots: 0,1 (start), 2 (r.z), 15 (d.q), 13,14 (r.r, r.z).
 // Returns the iteration count.
 __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *__restrict__ b,
-                                           double *__restrict__ x, const GridSync &gs, unsigned &gen, bool &ok,
-                                           dd (*lds)[MCL_BLOCK / MCL_WAVE], const MgLds &mgl, double ff_coef,
-                                           double &ff, bool collect_ff, int nbr, double rtol)
+                                           double *__restrict__ x, const GridSync &gs, WaitState &ws, bool &ok,
+                                           const MgLds &mgl, double ff_coef, double &ff, bool collect_ff, dd facc,
+                                           int nbr, double rtol)
 {
     const LevelDev &L = P.U.L;
     const bool use_mg = P.nmg > 1;
@@ -1279,14 +1255,15 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
     // rows of this thread: the same as on the V-cycle's finest level, so x, r
     // and q stay private to their thread; d and z are read by neighbours
     // (agent-scope accesses), and between the phases of an iteration the grid
-    // waits without cache maintenance (grid_sync_coherent)
+    // waits without cache maintenance (grid_reduce)
     const Ex ex = own_rows(n);
     double *__restrict__ r = P.rr, *__restrict__ q = P.U.cg_q;
     MCL_G double *dold = gp(P.U.cg_d), *dnew = gp(P.U.cg_s);
     MCL_G double *xg = gp(x);
     // r = b, then M r
+    double bn2 = 0.0, delta = 0.0;
     {
-        dd acc[2] = {dd_zero(), dd_zero()};
+        dd acc[3] = {dd_zero(), dd_zero(), facc};
         for (int i = ex.b; i < ex.e; i += ex.s) {
             double ri = b[i];
             vstd<kCO>(xg + i, 0.0);
@@ -1306,20 +1283,11 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
                 acc[1] = dd_add_prod(acc[1], ri, (double)zi);
             }
         }
-        reduce_publish<2>(P.U.rb, 0, acc, lds);
-    }
-    ok = csync(gs, gen, ok);
-    double bn2, delta;
-    {
-        double o[2];
-        reduce_collect<2>(P.U.rb, 0, gridDim.x, o, lds);
+        double o[3] = {0.0, 0.0, 0.0};
+        ok = ok && grid_sum<3>(gs, ws, acc, o);
         bn2 = o[0];
         delta = o[1];
-        if (collect_ff) {
-            double f[1];
-            reduce_collect<1>(P.U.rb, 5, gridDim.x, f, lds);
-            ff = f[0];
-        }
+        if (collect_ff) ff = o[2];
     }
     MCL_PHASE(1);
     const double stop2 = fmax(rtol * rtol * bn2, ff_coef * ff);
@@ -1331,10 +1299,10 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
     while (ok && it < P.max_inner) {
         // z = M r: the V-cycle's one call site, so the kernel holds one copy
         if (use_mg) {
-            vcycle_rest(P, mgl, gs, gen, ok, nbr, r, 2, lds);
-            ok = csync(gs, gen, ok);
-            double o[1];
-            reduce_collect<1>(P.U.rb, 2, gridDim.x, o, lds);
+            dd acc[1] = {dd_zero()};
+            vcycle_rest(P, mgl, gs, ws, ok, nbr, r, acc[0]);
+            double o[1] = {0.0};
+            ok = ok && grid_sum<1>(gs, ws, acc, o);
             rz = o[0];
             MCL_PHASE(5);
         }
@@ -1424,10 +1392,8 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
                 q[i] = s;
                 acc[0] = dd_add_prod(acc[0], di, s);
             }
-            reduce_publish<1>(P.U.rb, 15, acc, lds);
-            ok = csync(gs, gen, ok);
-            double o[1];
-            reduce_collect<1>(P.U.rb, 15, gridDim.x, o, lds);
+            double o[1] = {0.0};
+            ok = ok && grid_sum<1>(gs, ws, acc, o);
             dq = o[0];
             MCL_PHASE(0);
         }
@@ -1452,10 +1418,8 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
                     acc[1] = dd_add_prod(acc[1], ri, (double)zi);
                 }
             }
-            reduce_publish<2>(P.U.rb, 13, acc, lds);
-            ok = csync(gs, gen, ok);
-            double o[2];
-            reduce_collect<2>(P.U.rb, 13, gridDim.x, o, lds);
+            double o[2] = {0.0, 0.0};
+            ok = ok && grid_sum<2>(gs, ws, acc, o);
             rr = o[0];
             rz = o[1];
             MCL_PHASE(1);
@@ -1470,10 +1434,10 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
     // every exit follows a barrier that ends the phase of the last x update
     if (L.nh > 0) {
         // u = C u_f (hanging values from their parents across rows)
-        ok = ok && grid_sync(gs, gen);
+        ok = ok && grid_sync(gs, ws);
         for (int i = ex.b; i < ex.e; i += ex.s)
             if (L.hp_n[i] != 0) vstd<kCO>(xg + i, c_expand(L, i, [&](int j) { return vldd<kCO>(xg + j); }));
-        ok = ok && grid_sync(gs, gen);
+        ok = ok && grid_sync(gs, ws);
     }
     return it;
 }
@@ -1482,7 +1446,6 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
 
 __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
 {
-    __shared__ dd lds[MCL_RED_ROWS][MCL_BLOCK / MCL_WAVE];
     __shared__ float mg_vec[3 * MCL_MG_LDS_ROWS], mg_dinv[MCL_MG_LDS_ROWS], mg_val[MCL_MG_LDS_NNZ];
     __shared__ unsigned short mg_col[MCL_MG_LDS_NNZ];
     // level descriptors and Gershgorin bounds (read in every phase; LDS keeps
@@ -1507,8 +1470,8 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
     // this solve's augmented-Lagrangian weight (read before the first wait;
     // workgroup 0 rewrites it after the last)
     const double al_g = P.al_state ? *P.al_state : 0.0;
-    unsigned gen = __hip_atomic_load(U.gs.gen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-    bool ok = true;
+    WaitState ws;
+    bool ok = sync_begin(U.gs, ws);
     long long spmv = 0, inner = 0;
     // this thread's neighbour for the V-cycle's point-to-point waits
     int nbr = -1;
@@ -1552,6 +1515,7 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
     int cycle = 0, stage = 0;
     while (ok) {
         double rtol = P.inner_rtol, ffc = 0.0;
+        dd facc = dd_zero();
         if (stage != 1) {
             // momentum defect Ah = F - G p - K d; |F|^2 gives the solve an
             // absolute floor inner_rtol |F| (a warm start's small defect is
@@ -1559,16 +1523,14 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
             // iterations d and p were written by their owning threads with
             // plain stores and are now gathered across workgroups: a fenced
             // barrier first.
-            if (stage == 2) ok = ok && grid_sync(U.gs, gen);
-            dd acc[1] = {dd_zero()};
+            if (stage == 2) ok = ok && grid_sync(U.gs, ws);
             for (int i = rows.b; i < rows.e; i += rows.s) {
                 double u = ell_row(L.Kcol, L.Kval, L.Kncol[i], neq, i, U.d);
                 double f = L.F[i];
                 U.Ahv[i] = f - g_row(L, i, U.p) - u;
-                acc[0] = dd_add_prod(acc[0], f, f);
+                facc = dd_add_prod(facc, f, f);
             }
             spmv++;
-            if (stage == 0) reduce_publish<1>(U.rb, 5, acc, lds);
             ffc = P.inner_rtol * P.inner_rtol;
         } else {
             // Uzawa iteration `cycle`: the search direction s2 = z1 + delta
@@ -1591,13 +1553,13 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
             if (P.relax > 0.0) rtol = fmin(P.relax_max, fmax(P.inner_rtol, P.relax / fmax(dv, 1e-300)));
         }
         MCL_PHASE(6);
-        if (L.nh > 0) ok = ok && grid_sync(U.gs, gen);   // the solve's start reads b across rows
-        const int it = inner_mixed(P, U.Ahv, U.u1, U.gs, gen, ok, lds, mgl, ffc, ff, stage == 0, nbr, rtol);
+        if (L.nh > 0) ok = ok && grid_sync(U.gs, ws);   // the solve's start reads b across rows
+        const int it = inner_mixed(P, U.Ahv, U.u1, U.gs, ws, ok, mgl, ffc, ff, stage == 0, facc, nbr, rtol);
         inner += it;
         spmv += it;
         if (stage != 1) {
             for (int i = gtid; i < neq; i += gsize) U.d[i] += vldd<kCO>(u1 + i);
-            ok = ok && grid_sync(U.gs, gen);
+            ok = ok && grid_sync(U.gs, ws);
             if (stage == 2) break;
             if (P.probe) {
                 // initial Schur residual r1 = G^T K^-1 (F - G p) of this
@@ -1607,10 +1569,8 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
                     double r = gt_elem(L, e, U.d);
                     acc[0] = dd_add_prod(acc[0], r, r);
                 }
-                reduce_publish<1>(U.rb, 4, acc, lds);
-                ok = ok && grid_sync(U.gs, gen);
-                double o[1];
-                reduce_collect<1>(U.rb, 4, gridDim.x, o, lds);
+                double o[1] = {0.0};
+                ok = ok && grid_sum<1>(U.gs, ws, acc, o);
                 if (blockIdx.x == 0 && threadIdx.x == 0) {
                     U.stats->probe_r1 = o[0];
                     U.stats->cycles = 0;
@@ -1618,6 +1578,7 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
                     U.stats->spmv = spmv;
                     U.stats->aborted = ok ? 0 : 1;
                 }
+                sync_end(U.gs, ws);
                 return;
             }
             // Schur residual r1 = G^T d, z1 = M_S r1 and r1.z1 for the first
@@ -1631,16 +1592,13 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
                     vstd<kCO>(gp(z1) + e, z);
                     acc[0] = dd_add_prod(acc[0], r, z);
                 }
-                reduce_publish<1>(U.rb, 4, acc, lds);
-            }
-            ok = csync(U.gs, gen, ok);
-            {
-                double o[1];
-                reduce_collect<1>(U.rb, 4, gridDim.x, o, lds);
+                double o[1] = {0.0};
+                ok = ok && grid_sum<1>(U.gs, ws, acc, o);
                 r1z1 = o[0];
             }
             stage = 1;
         } else {
+            double alpha;
             {
                 dd acc[1] = {dd_zero()};
                 for (int e = gtid; e < nel; e += gsize) {
@@ -1648,13 +1606,8 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
                     U.Ahp[e] = a;
                     acc[0] = dd_add_prod(acc[0], vldd<kCO>(gp(s2) + e), a);
                 }
-                reduce_publish<1>(U.rb, 6, acc, lds);
-            }
-            ok = csync(U.gs, gen, ok);
-            double alpha;
-            {
-                double o[1];
-                reduce_collect<1>(U.rb, 6, gridDim.x, o, lds);
+                double o[1] = {0.0};
+                ok = ok && grid_sum<1>(U.gs, ws, acc, o);
                 alpha = r1z1 / o[0];
             }
             {
@@ -1680,12 +1633,8 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
                     acc[2] = dd_add_prod(acc[2], u, u);
                     acc[3] = dd_add_prod(acc[3], di, di);
                 }
-                reduce_publish<5>(U.rb, 8, acc, lds);
-            }
-            ok = csync(U.gs, gen, ok);
-            {
-                double o[5];
-                reduce_collect<5>(U.rb, 8, gridDim.x, o, lds);
+                double o[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+                ok = ok && grid_sum<5>(U.gs, ws, acc, o);
                 dp = alpha * sqrt(o[0] / (1.0e-32 + o[1]));
                 dv = alpha * sqrt(o[2] / (1.0e-32 + o[3]));
                 r0z0 = r1z1;
@@ -1707,7 +1656,7 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
     if (al_g > 0.0 && ok) {
         // the plain system's pressure p + gamma W G^T d (d was written by
         // its owners with plain stores: a fenced barrier first)
-        ok = grid_sync(U.gs, gen);
+        ok = grid_sync(U.gs, ws);
         if (ok)
             for (int e = gtid; e < nel; e += gsize) U.p[e] += al_g * P.al_w[e] * gt_elem(L, e, U.d);
     }
@@ -1726,6 +1675,7 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
         U.stats->aborted = ok ? 0 : 1;
         if (!(dv == dv) || !(dp == dp)) U.stats->nan_flag = 1;
     }
+    sync_end(U.gs, ws);
     MCL_PHASE(6);
 #if MCL_PHASE_TIMERS
     if (blockIdx.x == 0 && threadIdx.x == 0)
