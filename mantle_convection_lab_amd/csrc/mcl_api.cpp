@@ -258,7 +258,11 @@ extern "C" int mcl_create(int device, mcl_ctx **out)
     shape_tables(&st);
     if (mcl_upload_shape(&st) != hipSuccess) { delete c; return MCL_E_DEVICE; }
     int per_cu_u = 0, per_cu_h = 0;
-    hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_u, (const void *)k_uzawa_fp64, MCL_BLOCK, 0);
+    for (int sv = MCL_SOLVER_JC; sv <= MCL_SOLVER_MG; sv++) {
+        int per_cu_s = 0;
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_s, mcl_uzawa_fp64_kernel(sv), MCL_BLOCK, 0);
+        per_cu_u = sv == MCL_SOLVER_JC ? per_cu_s : std::min(per_cu_u, per_cu_s);
+    }
     hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_h, (const void *)k_heat_fp64, MCL_BLOCK, 0);
     int per_cu_m = 0;
     hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_m, (const void *)k_uzawa_mixed, MCL_BLOCK, 0);
@@ -1393,7 +1397,7 @@ extern "C" int mcl_velocity_pressure_KGF_matrix(mcl_ctx *c)
 // count); the mixed solve takes at most 128 rows per workgroup (its V-cycle
 // waits are mostly point-to-point, and more workgroups keep more loads in
 // flight: at 256x256 and above every CU has one workgroup).
-#define MCL_FP64_ROWS_PER_THREAD 2
+#define MCL_FP64_ROWS_PER_THREAD 1
 static unsigned coop_blocks(mcl_ctx *c, long long n, int rows_per_block, const char *knob)
 {
     const long long per = rows_per_block;
@@ -1512,6 +1516,7 @@ static UzawaParams uzawa_params(mcl_ctx *c, double accuracy, const SolveWork &W)
     P.mg_coarse_iteration = k.mg_coarse_iteration;
     P.xt = c->xt;
     P.xt2 = c->xt2;
+    P.cg_d2 = c->xt;   // conjugate gradients: no previous iterate to keep
     P.gsl = c->gs_tab;
     P.ngsl = c->nlev;
     // Gauss-Seidel sweeps and the multigrid V-cycle are sequential in the
@@ -2016,7 +2021,7 @@ static int solve_enqueue(mcl_ctx *c, const SolveWork &W, EnqMode mode, EventPair
     } else {
         void *args[] = {&P};
         if (ev) HIPCHK(c, hipEventRecord(ev->a, c->stream));
-        HIPCHK(c, launch_persistent(c, (const void *)k_uzawa_fp64, P.gs.nblocks, args, plain));
+        HIPCHK(c, launch_persistent(c, mcl_uzawa_fp64_kernel(k.solver), P.gs.nblocks, args, plain));
     }
     if (ev) HIPCHK(c, hipEventRecord(ev->b, c->stream));
     // nodal velocity and stress (Solver.c:8-9)
@@ -2211,6 +2216,7 @@ static int heat_enqueue(mcl_ctx *c, EnqMode mode, EventPair *ev)
     H.cg_s = w; w += nt;
     H.cg_d = w; w += nt;
     H.cg_q = w; w += nt;
+    H.cg_d2 = w; w += nt;
     H.model_time = c->model_time;
     H.accuracy = k.accuracy;
     H.theta = k.theta;

@@ -384,9 +384,11 @@ __device__ __forceinline__ bool grid_reduce(const GridSync &gs, WaitState &w, dd
 #pragma unroll
         for (int q = 0; q < NW; q++) word[q] = (NS || NM) && lane < WAVES ? part[q][lane] : 0.0;
         fold(8);
-        publish(blockIdx.x, 7);
-        int last;
-        if (nb <= MCL_WAVE) {
+        int last = 7;
+        if (nb > 1) publish(blockIdx.x, 7);
+        if (nb == 1) {
+            // nothing leaves the workgroup
+        } else if (nb <= MCL_WAVE) {
             collect(nb, 0, 1);
             fold(nb);
             last = nb <= 8 ? 7 : nb <= 16 ? 15 : 63;
@@ -434,13 +436,15 @@ __device__ __forceinline__ bool grid_wait(const GridSync &gs, WaitState &w)
 
 // Grid-wide wait for data written and read with plain accesses: an agent-scope
 // release before (thread 0 writes back the L2 after all waves' stores), an
-// acquire after (invalidates the caches).
+// acquire after (thread 0 invalidates the caches of its CU and XCD; every
+// thread doing so costs 18 us at 256 workgroups).
 __device__ __forceinline__ bool grid_sync(const GridSync &gs, WaitState &w)
 {
     wg_complete();
     if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     const bool ok = grid_wait(gs, w);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    __syncthreads();
     return ok;
 }
 

@@ -270,7 +270,8 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_assemble_K(const AsmLevel *__rest
 // global_p_prod, Array_work.c:287-341, at one rank).  Every workgroup computes
 // it itself: the products in parallel into LDS, the additions in order by one
 // thread, so all workgroups obtain the identical value without a barrier.
-// The vectors must be complete (called after a grid barrier).
+// The vectors must be complete (called after a grid wait) and written with
+// agent-scope stores.
 #define MCL_SEQ_CHUNK 2048
 __device__ double seq_dot(const double *__restrict__ x, const double *__restrict__ y, int n)
 {
@@ -280,7 +281,7 @@ __device__ double seq_dot(const double *__restrict__ x, const double *__restrict
     for (int base = 0; base < n; base += MCL_SEQ_CHUNK) {
         const int m = min(MCL_SEQ_CHUNK, n - base);
         __syncthreads();
-        for (int t = threadIdx.x; t < m; t += blockDim.x) buf[t] = x[base + t] * y[base + t];
+        for (int t = threadIdx.x; t < m; t += blockDim.x) buf[t] = ald(x + base + t) * ald(y + base + t);
         __syncthreads();
         if (threadIdx.x == 0) {
             // loads batched sixteen at a time, additions strictly in order
@@ -302,104 +303,139 @@ __device__ double seq_dot(const double *__restrict__ x, const double *__restrict
 
 // Conj_Grad (Solver.c:1589-1797) / Conj_Grad_heat (Update_temperature.c:
 // 1140-1354) inside a persistent kernel.  All workgroups execute the same
-// control flow: the scalars come from reduce_collect, identical everywhere.
+// control flow: the scalars come from the grid waits, identical everywhere.
 // kind 0: velocity (constraint on velocity dofs), 1: heat.
-// Returns the iteration count; *ok is cleared if a barrier aborted.
-__device__ int pcg_persistent(const LevelDev &L, const EllMat &A, const double *__restrict__ b,
-                              double *__restrict__ x, bool x_zero, double accu, int max_cycle, int precond,
-                              int kind, CgVecs v, const GridSync &gs, WaitState &ws, const RedBuf &rb,
-                              dd (*lds)[MCL_BLOCK / MCL_WAVE], double *ldsm, bool &ok, long long &spmv,
-                              bool exact)
+// Two grid waits an iteration:
+//   (1) d = s + beta d and q = A d in one pass (the product gathers s + beta d,
+//       the same rounding as the stored d), with d.q
+//   (2) x += alpha d, r -= alpha q (every 50th iteration r = b - A x, after a
+//       wait for x), s = r / diag, with r.s and max |alpha r|
+// s, d and x cross workgroups with agent-scope accesses, so the waits need no
+// cache maintenance and the matrix stays in the L2; r and q belong to the row's
+// thread.
+// ROWS: every thread owns at most one row (row_window): the row, r, q, d and x
+// stay in registers and the gathered vector comes through the window; what is
+// left of an iteration is the two waits and one round trip of loads.
+// Measured per inner iteration (three fenced barriers, the matrix re-read after
+// each, two rows a thread): 64x64 29 -> 7.7 us, 128x128 29 -> 8.2 us; of that
+// the windows and registers are 2.7 us against gathers by agent-scope loads.
+// The caller's phase may write b on this thread's rows (grid stride) right
+// before the call; a non-zero x must be complete.  x is complete on return.
+// Returns the iteration count; ok is cleared if a wait gave up.
+template <int W, bool ROWS>
+__device__ __forceinline__ int pcg_rows(const LevelDev &L, const EllMat &A, const RowReg<W> &row, const Window &win,
+                                        double diag, const double *__restrict__ b, double *x, bool x_zero, double accu,
+                                        int max_cycle, int precond, int kind, CgVecs v, const GridSync &gs,
+                                        WaitState &ws, bool &ok, long long &spmv, bool exact)
 {
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsize = gridDim.x * blockDim.x;
     const int n = A.n;
-    {
-        dd acc[1] = {dd_zero()};
-        for (int i = gtid; i < n; i += gsize) {
-            double ax = x_zero ? 0.0 : ell_row(A.col, A.val, A.ncol[i], n, i, x);
-            double r = b[i] - ax;
-            double dv = precond ? r / ell_diag(A, i) : r;
-            v.r[i] = r;
-            v.d[i] = dv;
-            acc[0] = dd_add_prod(acc[0], r, dv);
-        }
-        if (!x_zero) spmv++;
-        reduce_publish<1>(rb, 0, acc, lds);
-    }
-    ok = ok && grid_sync(gs, ws);
+    double rr = 0.0, rq = 0.0, rd = 0.0, rx = 0.0;
+    if (ROWS && !x_zero && gtid < n) rx = ald(x + gtid);
+    // row i times the vector value(j): the window's entries were filled before
+    auto times = [&](int i, auto value) {
+        if constexpr (ROWS) return row.dot(win.buf);
+        else return ell_row_ld(A.col, A.val, A.ncol[i], n, i, value);
+    };
+    auto xat = [&](int j) { return ald(x + j); };
+    // r of row i and s = M r, with r.s
+    auto residual = [&](int i, double r, dd &acc) {
+        const double s = precond ? r / (ROWS ? diag : ell_diag(A, i)) : r;
+        if (ROWS) rr = r;
+        if (!ROWS || exact) ast(v.r + i, r);
+        ast(v.s + i, s);
+        acc = dd_add_prod(acc, r, s);
+    };
     double delta_new;
     {
-        double o[1];
-        reduce_collect<1>(rb, 0, gridDim.x, o, lds);
-        delta_new = exact ? seq_dot(v.r, v.d, n) : o[0];
+        dd acc[1] = {dd_zero()};
+        if (ROWS && !x_zero) win.fill(xat);
+        for (int i = gtid; i < n; i += gsize) residual(i, b[i] - (x_zero ? 0.0 : times(i, xat)), acc[0]);
+        if (!x_zero) spmv++;
+        double o[1] = {0.0};
+        ok = ok && grid_sum<1>(gs, ws, acc, o);
+        delta_new = exact ? seq_dot(v.r, v.s, n) : o[0];
     }
     const double delta0 = delta_new;
+    double *dold = v.d, *dnew = v.d2, beta = 0.0;
     int cycle = 0;
     while (ok && cycle < max_cycle && delta_new > accu * delta0) {
-        // q = K d, d.q
-        {
-            dd acc[1] = {dd_zero()};
-            for (int i = gtid; i < n; i += gsize) {
-                double q = ell_row(A.col, A.val, A.ncol[i], n, i, v.d);
-                v.q[i] = q;
-                acc[0] = dd_add_prod(acc[0], v.d[i], q);
-            }
-            spmv++;
-            reduce_publish<1>(rb, 1, acc, lds);
-        }
-        ok = ok && grid_sync(gs, ws);
         double t1;
         {
-            double o[1];
-            reduce_collect<1>(rb, 1, gridDim.x, o, lds);
-            t1 = exact ? seq_dot(v.d, v.q, n) : o[0];
+            auto dat = [&](int j) { return cycle == 0 ? ald(v.s + j) : ald(v.s + j) + beta * ald(dold + j); };
+            dd acc[1] = {dd_zero()};
+            if (ROWS) win.fill(dat);
+            for (int i = gtid; i < n; i += gsize) {
+                const double d = ROWS ? win.buf[i - win.w0] : dat(i), q = times(i, dat);
+                ast(dnew + i, d);
+                if (ROWS) {
+                    rd = d;
+                    rq = q;
+                }
+                if (!ROWS || exact) ast(v.q + i, q);
+                acc[0] = dd_add_prod(acc[0], d, q);
+            }
+            spmv++;
+            double o[1] = {0.0};
+            ok = ok && grid_sum<1>(gs, ws, acc, o);
+            t1 = exact ? seq_dot(dnew, v.q, n) : o[0];
         }
         const double alpha = delta_new / t1;
-        for (int i = gtid; i < n; i += gsize) x[i] += alpha * v.d[i];
+        for (int i = gtid; i < n; i += gsize) {
+            rx = (ROWS ? rx : ald(x + i)) + alpha * (ROWS ? rd : ald(dnew + i));
+            ast(x + i, rx);
+        }
         if (L.nh > 0) {
-            ok = ok && grid_sync(gs, ws);
+            ok = ok && grid_wait(gs, ws);
             if (kind == 0) constrain_v(L, x, gtid, gsize);
             else constrain_T(L, x, gtid, gsize);
         }
         const bool recompute = (cycle % 50) == 0;
-        if (recompute) ok = ok && grid_sync(gs, ws);
-        double delta_old = delta_new;
-        {
-            dd acc[1] = {dd_zero()};
-            double mx = 0.0;
-            for (int i = gtid; i < n; i += gsize) {
-                double r;
-                if (recompute) r = b[i] - ell_row(A.col, A.val, A.ncol[i], n, i, x);
-                else r = v.r[i] - alpha * v.q[i];
-                v.r[i] = r;
-                double s = precond ? r / ell_diag(A, i) : r;
-                v.s[i] = s;
-                acc[0] = dd_add_prod(acc[0], r, s);
-                mx = fmax(mx, fabs(alpha * r));
-            }
-            if (recompute) spmv++;
-            reduce_publish<1>(rb, 2, acc, lds);
-            double bm = block_max(mx, ldsm);
-            if (threadIdx.x == 0) rb.pmax[0 * MCL_MAX_WG + blockIdx.x] = bm;
+        if (recompute || (ROWS && L.nh > 0)) {
+            ok = ok && grid_wait(gs, ws);
+            if (ROWS && gtid < n) rx = ald(x + gtid);   // a hanging value is written by another thread
+            if (ROWS && recompute) win.fill(xat);
         }
-        ok = ok && grid_sync(gs, ws);
+        const double delta_old = delta_new;
         double res;
         {
-            double o[1];
-            reduce_collect<1>(rb, 2, gridDim.x, o, lds);
+            dd acc[1] = {dd_zero()};
+            double mx[1] = {0.0}, o[2] = {0.0, 0.0};
+            for (int i = gtid; i < n; i += gsize) {
+                double r;
+                if (recompute) r = b[i] - times(i, xat);
+                else r = (ROWS ? rr : ald(v.r + i)) - alpha * (ROWS ? rq : ald(v.q + i));
+                residual(i, r, acc[0]);
+                mx[0] = fmax(mx[0], fabs(alpha * r));
+            }
+            if (recompute) spmv++;
+            ok = ok && grid_reduce<1, 1>(gs, ws, acc, mx, o);
             delta_new = exact ? seq_dot(v.r, v.s, n) : o[0];
-            double m = 0.0;
-            for (int bb = threadIdx.x; bb < (int)gridDim.x; bb += MCL_BLOCK) m = fmax(m, rb.pmax[bb]);
-            res = block_max(m, ldsm);
+            res = o[1];
         }
-        const double beta = delta_new / delta_old;
-        for (int i = gtid; i < n; i += gsize) v.d[i] = v.s[i] + beta * v.d[i];
+        beta = delta_new / delta_old;
+        double *t = dold;
+        dold = dnew;
+        dnew = t;
         cycle++;
-        bool brk = precond ? (res < accu) : (kind == 0 ? res < accu : (res < accu && cycle > 10));
-        ok = ok && grid_sync(gs, ws);
+        const bool brk = precond ? (res < accu) : (kind == 0 ? res < accu : (res < accu && cycle > 10));
         if (brk) break;
     }
+    if (exact) ok = ok && grid_wait(gs, ws);   // every workgroup is done with seq_dot's vectors
     return cycle;
+}
+
+template <int W>
+__device__ __forceinline__ int pcg_persistent(const LevelDev &L, const EllMat &A, const RowReg<W> &row,
+                                              const Window &win, double diag, const double *__restrict__ b, double *x,
+                                              bool x_zero, double accu, int max_cycle, int precond, int kind, CgVecs v,
+                                              const GridSync &gs, WaitState &ws, bool &ok, long long &spmv, bool exact)
+{
+    if (win.fits)
+        return pcg_rows<W, true>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws, ok,
+                                 spmv, exact);
+    return pcg_rows<W, false>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws, ok, spmv,
+                              exact);
 }
 
 // ------------------------------------------------ stationary inner solvers
@@ -409,49 +445,66 @@ __device__ int pcg_persistent(const LevelDev &L, const EllMat &A, const double *
 // max |x - x_old| < accu, no hanging-node constraint.
 
 // jacobi (Solver.c:1800-1864) over the whole grid: sweep k reads one buffer
-// and writes the other (x_old needs no copy); the sweep maxima alternate
-// between two reduction slots, so a workgroup writing a slot two sweeps later
-// cannot overtake a slower one still reading it.
-__device__ int jacobi_grid(const EllMat &A, const double *__restrict__ b, double *x, double *xt, double accu,
-                           int max_cycle, const GridSync &gs, WaitState &ws, const RedBuf &rb, double *ldsm, bool &ok,
-                           long long &spmv)
+// and writes the other (x_old needs no copy), both with agent-scope accesses;
+// the wait that ends a sweep carries its maximum.  With one row a thread
+// (row_window) the row stays in registers and x comes through the window: a
+// sweep at 32x32 takes 2.4 us (14.5 us with a fenced barrier, its maxima
+// collected in a second pass and every column's load waiting for the last).
+// The caller's x must be complete; it is complete on return.
+__device__ __forceinline__ int jacobi_grid(const EllMat &A, const RowReg<18> &row, const Window &win, double diag,
+                                           const double *__restrict__ b, double *x, double *xt, double accu,
+                                           int max_cycle, const GridSync &gs, WaitState &ws, bool &ok,
+                                           long long &spmv)
 {
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsize = gridDim.x * blockDim.x;
     const int n = A.n;
+    const bool mine = gtid < n;
+    int dslot = -1;
+    double bi = 0.0;
+    if (win.fits && mine) {
+        bi = b[gtid];
+#pragma unroll
+        for (int u = 0; u < 18; u++)
+            if (u < row.n && row.off[u] == 8u * (unsigned)(gtid - win.w0)) dslot = u;
+    }
     double *src = x, *dst = xt;
     int cycle = 0;
     while (ok && cycle < max_cycle) {
-        double mx = 0.0;
-        for (int i = gtid; i < n; i += gsize) {
-            double prod = 0.0, diag = 1.0;
-            const int nc = A.ncol[i];
-            for (int j = 0; j < nc; j++) {
-                const int c = A.col[j * n + i];
-                const double v = A.val[j * n + i];
-                if (c != i) prod += v * src[c];
-                else diag = v;
+        double mx[1] = {0.0}, o[1] = {0.0};
+        if (win.fits) {
+            win.fill([&](int j) { return ald(src + j); });
+            if (mine) {
+                const double xn = (bi - row.dot(win.buf, dslot)) / diag;
+                ast(dst + gtid, xn);
+                mx[0] = fabs(xn - win.buf[gtid - win.w0]);
             }
-            const double xn = (b[i] - prod) / diag;
-            dst[i] = xn;
-            mx = fmax(mx, fabs(xn - src[i]));
+        } else {
+            for (int i = gtid; i < n; i += gsize) {
+                double prod = 0.0, dg = 1.0;
+                const int nc = A.ncol[i];
+                for (int j = 0; j < nc; j++) {
+                    const int c = A.col[j * n + i];
+                    const double v = A.val[j * n + i];
+                    if (c != i) prod += v * ald(src + c);
+                    else dg = v;
+                }
+                const double xn = (b[i] - prod) / dg;
+                ast(dst + i, xn);
+                mx[0] = fmax(mx[0], fabs(xn - ald(src + i)));
+            }
         }
         spmv++;
-        const int slot = 4 + (cycle & 1);
-        double bm = block_max(mx, ldsm);
-        if (threadIdx.x == 0) rb.pmax[slot * MCL_MAX_WG + blockIdx.x] = bm;
-        ok = ok && grid_sync(gs, ws);
-        double m = 0.0;
-        for (int bb = threadIdx.x; bb < (int)gridDim.x; bb += MCL_BLOCK) m = fmax(m, rb.pmax[slot * MCL_MAX_WG + bb]);
-        const double diff = block_max(m, ldsm);
+        dd none[1] = {dd_zero()};
+        ok = ok && grid_reduce<0, 1>(gs, ws, none, mx, o);
         double *t = src;
         src = dst;
         dst = t;
         cycle++;
-        if (diff < accu) break;
+        if (o[0] < accu) break;
     }
     if (src != x) {
-        for (int i = gtid; i < n; i += gsize) x[i] = src[i];
-        ok = ok && grid_sync(gs, ws);
+        for (int i = gtid; i < n; i += gsize) ast(x + i, ald(src + i));
+        ok = ok && grid_wait(gs, ws);
     }
     return cycle;
 }
@@ -557,35 +610,45 @@ __device__ int mg_block(const GsLevelDev *lv, int nl, const double *b, double *x
     return cycle;
 }
 
-// The inner solve of citcom_solver (Solver.c:82-89) for the chosen solver.
-__device__ int inner_solve(const UzawaParams &P, const LevelDev &L, const EllMat &K, const double *b, double *x,
-                           bool x_zero, CgVecs cv, WaitState &ws, dd (*lds)[MCL_BLOCK / MCL_WAVE], double *ldsm,
-                           bool &ok, long long &spmv)
+// The inner solve of citcom_solver (Solver.c:82-89) for the chosen solver, on
+// a right-hand side that this thread's rows have just been written to and an x
+// that is complete or, with x_zero, just zeroed; x is complete on return.
+template <int SOLVER>
+__device__ __forceinline__ int inner_solve(const UzawaParams &P, const LevelDev &L, const EllMat &K,
+                                           const RowReg<18> &row, const Window &win, double diag, const double *b,
+                                           double *x, bool x_zero, CgVecs cv, WaitState &ws, double *ldsm, bool &ok,
+                                           long long &spmv)
 {
-    switch (P.solver) {
-    case MCL_INNER_JC:
-        return jacobi_grid(K, b, x, P.xt, P.accuracy, 1000, P.gs, ws, P.rb, ldsm, ok, spmv);
-    case MCL_INNER_GS: {
-        const int c = gs_block(P.gsl[P.ngsl - 1], b, x, P.xt, P.accuracy, 1000, ldsm, spmv);
+    if constexpr (SOLVER == MCL_INNER_CG) {
+        return pcg_persistent<18>(L, K, row, win, diag, b, x, x_zero, P.accuracy, P.max_cg_cycle, P.cg_precondition, 0,
+                                  cv, P.gs, ws, ok, spmv, P.exact_dots != 0);
+    } else if constexpr (SOLVER == MCL_INNER_JC) {
+        if (x_zero) ok = ok && grid_wait(P.gs, ws);
+        return jacobi_grid(K, row, win, diag, b, x, P.xt, P.accuracy, 1000, P.gs, ws, ok, spmv);
+    } else {
+        // one workgroup, plain accesses
+        ok = ok && grid_sync(P.gs, ws);
+        const int c = SOLVER == MCL_INNER_GS
+                          ? gs_block(P.gsl[P.ngsl - 1], b, x, P.xt, P.accuracy, 1000, ldsm, spmv)
+                          : mg_block(P.gsl, P.ngsl, b, x, P.xt2, P.xt, P.accuracy, P.mg_cycle, P.mg_finest_iteration,
+                                     P.mg_coarse_iteration, ldsm, spmv);
         ok = ok && grid_sync(P.gs, ws);
         return c;
-    }
-    case MCL_INNER_MG: {
-        const int c = mg_block(P.gsl, P.ngsl, b, x, P.xt2, P.xt, P.accuracy, P.mg_cycle, P.mg_finest_iteration,
-                               P.mg_coarse_iteration, ldsm, spmv);
-        ok = ok && grid_sync(P.gs, ws);
-        return c;
-    }
-    default:
-        return pcg_persistent(L, K, b, x, x_zero, P.accuracy, P.max_cg_cycle, P.cg_precondition, 0, cv, P.gs, ws,
-                              P.rb, lds, ldsm, ok, spmv, P.exact_dots != 0);
     }
 }
 
-// citcom_solver (Solver.c:14-249) as one persistent kernel.
+// citcom_solver (Solver.c:14-249) as one persistent kernel.  Vectors that other
+// workgroups read (u1, d and p at the start, z, s) are stored and loaded with
+// agent-scope accesses; the rest belong to the thread of the row or element
+// (grid stride).  An Uzawa iteration has three phases of its own: the search
+// direction s2 = z1 + delta s1 with G s2 (gathered as z1 + delta s1, the same
+// rounding), which the inner solve's start follows without a wait; G^T u1 with
+// s2.G^T u1; the updates with their norms and the next z and r.z.  (r0.z0 is
+// the previous iteration's r1.z1: the same vectors, the same sum.)
+// One kernel per inner solver (each then has the registers to itself).
+template <int SOLVER>
 __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
 {
-    __shared__ dd lds[MCL_RED_ROWS][MCL_BLOCK / MCL_WAVE];
     __shared__ double ldsm[MCL_BLOCK / MCL_WAVE];
     const LevelDev &L = P.L;
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsize = gridDim.x * blockDim.x;
@@ -594,8 +657,16 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
     WaitState ws;
     bool ok = sync_begin(P.gs, ws);
     long long spmv = 0, inner = 0;
-    EllMat K{L.Kcol, L.Kncol, L.Kval, L.Kdiag, nullptr, neq};
-    CgVecs cv{P.cg_r, P.cg_s, P.cg_d, P.cg_q};
+    EllMat K{L.Kcol, L.Kncol, L.Kval, L.Kdiag, nullptr, neq, L.WK};
+    CgVecs cv{P.cg_r, P.cg_s, P.cg_d, P.cg_q, P.cg_d2};
+    RowReg<18> row;
+    Window win{nullptr, 0, 0, false};
+    double diag = 1.0;
+    if constexpr (SOLVER == MCL_INNER_CG || SOLVER == MCL_INNER_JC) {
+        __shared__ double buf[MCL_WINDOW];
+        win = row_window(row, K.col, K.ncol, K.val, K.width, neq, buf);
+        if (gtid < neq) diag = K.diag[gtid];
+    }
     // Preconditioner data, Solver.c:54-64: BAB[e] = sum_i G_ie^2 / Kdiag_i
     for (int e = gtid; e < nel; e += gsize) {
         double s = 0.0;
@@ -608,105 +679,101 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
         }
         P.BAB[e] = s;
     }
-    // u1 = K d ; Ah = F - G p - u1   (:67-77)
-    for (int i = gtid; i < neq; i += gsize) {
-        double u = ell_row(L.Kcol, L.Kval, L.Kncol[i], neq, i, P.d);
-        double gp = g_row(L, i, P.p);
-        P.u1[i] = u;
-        P.Ahv[i] = L.F[i] - gp - u;
-    }
-    spmv++;
-    ok = ok && grid_sync(P.gs, ws);
-    inner += inner_solve(P, L, K, P.Ahv, P.u1, false, cv, ws, lds, ldsm, ok, spmv);
-    for (int i = gtid; i < neq; i += gsize) P.d[i] += P.u1[i];
-    ok = ok && grid_sync(P.gs, ws);
     double *r0 = P.r0, *r1 = P.r1, *r2 = P.r2, *z0 = P.z0, *z1 = P.z1, *s1 = P.s1, *s2 = P.s2;
-    for (int e = gtid; e < nel; e += gsize) r1[e] = gt_elem(L, e, P.d);
-    double dv = 1.0, dp = 1.0;
+    double dv = 1.0, dp = 1.0, r1z1 = 0.0, r0z0 = 0.0;
     int cycle = 0;
-    while (ok && (dv > P.citcom_accu || (dp > P.citcom_accu && P.check_v_only == 0)) &&
-           cycle < P.max_citcom_cycle) {
-        // z1 = BAB r1 (or r1 / BAB); r1.z1, r0.z0
-        {
-            dd acc[2] = {dd_zero(), dd_zero()};
+    bool first = true;   // the solve for the initial velocity's defect comes before the loop's
+    auto zvec = [&](int e, double r) { return P.schur ? r / P.BAB[e] : P.BAB[e] * r; };
+    while (true) {
+        // the inner solve's right-hand side, then its one call site
+        if (first) {
+            // u1 = K d ; Ah = F - G p - u1   (:67-77)
+            for (int i = gtid; i < neq; i += gsize) {
+                double u = ell_row(L.Kcol, L.Kval, L.Kncol[i], neq, i, P.d);
+                double gp = g_row(L, i, P.p);
+                ast(P.u1 + i, u);
+                P.Ahv[i] = L.F[i] - gp - u;
+            }
+            spmv++;
+            ok = ok && grid_wait(P.gs, ws);   // the solve starts from u1
+        } else {
+            if (!(ok && (dv > P.citcom_accu || (dp > P.citcom_accu && P.check_v_only == 0)) &&
+                  cycle < P.max_citcom_cycle))
+                break;
+            if (!(r1z1 == r1z1)) P.stats->nan_flag = 1;
+            const double delta = cycle > 0 ? r1z1 / r0z0 : 0.0;
+            auto s2at = [&](int e) { return cycle == 0 ? ald(z1 + e) : ald(z1 + e) + delta * ald(s1 + e); };
+            for (int e = gtid; e < nel; e += gsize) ast(s2 + e, s2at(e));
+            // Ah = G s2 ; u1 = 0 ; K u1 = Ah
+            for (int i = gtid; i < neq; i += gsize) {
+                P.Ahv[i] = g_row_ld(L, i, s2at);
+                ast(P.u1 + i, 0.0);
+            }
+        }
+        inner += inner_solve<SOLVER>(P, L, K, row, win, diag, P.Ahv, P.u1, !first, cv, ws, ldsm, ok, spmv);
+        if (first) {
+            first = false;
+            for (int i = gtid; i < neq; i += gsize) ast(P.d + i, ald(P.d + i) + ald(P.u1 + i));
+            ok = ok && grid_wait(P.gs, ws);
+            // r1 = G^T d, z1 = BAB r1 (or r1 / BAB); r1.z1
+            dd acc[1] = {dd_zero()};
             for (int e = gtid; e < nel; e += gsize) {
-                double z = P.schur ? r1[e] / P.BAB[e] : P.BAB[e] * r1[e];
-                z1[e] = z;
-                acc[0] = dd_add_prod(acc[0], r1[e], z);
-                if (cycle > 0) acc[1] = dd_add_prod(acc[1], r0[e], z0[e]);
+                const double r = gt_elem_ld(L, e, [&](int j) { return ald(P.d + j); }), z = zvec(e, r);
+                ast(r1 + e, r);
+                ast(z1 + e, z);
+                acc[0] = dd_add_prod(acc[0], r, z);
             }
-            reduce_publish<2>(P.rb, 4, acc, lds);
+            double o[1] = {0.0};
+            ok = ok && grid_sum<1>(P.gs, ws, acc, o);
+            r1z1 = P.exact_dots ? seq_dot(r1, z1, nel) : o[0];
+            continue;
         }
-        ok = ok && grid_sync(P.gs, ws);
-        double r1z1, delta = 0.0;
-        {
-            double o[2];
-            reduce_collect<2>(P.rb, 4, gridDim.x, o, lds);
-            if (P.exact_dots) {
-                o[0] = seq_dot(r1, z1, nel);
-                if (cycle > 0) o[1] = seq_dot(r0, z0, nel);
-            }
-            r1z1 = o[0];
-            if (cycle > 0) delta = r1z1 / o[1];
-        }
-        if (!(r1z1 == r1z1)) P.stats->nan_flag = 1;
-        for (int e = gtid; e < nel; e += gsize) s2[e] = cycle == 0 ? z1[e] : z1[e] + delta * s1[e];
-        ok = ok && grid_sync(P.gs, ws);
-        // Ah = G s2 ; u1 = 0 ; K u1 = Ah
-        for (int i = gtid; i < neq; i += gsize) {
-            P.Ahv[i] = g_row(L, i, s2);
-            P.u1[i] = 0.0;
-        }
-        ok = ok && grid_sync(P.gs, ws);
-        inner += inner_solve(P, L, K, P.Ahv, P.u1, true, cv, ws, lds, ldsm, ok, spmv);
         // Ah = G^T u1 ; alpha = r1.z1 / s2.Ah
+        double alpha;
         {
             dd acc[1] = {dd_zero()};
             for (int e = gtid; e < nel; e += gsize) {
-                double a = gt_elem(L, e, P.u1);
-                P.Ahp[e] = a;
-                acc[0] = dd_add_prod(acc[0], s2[e], a);
+                double a = gt_elem_ld(L, e, [&](int j) { return ald(P.u1 + j); });
+                ast(P.Ahp + e, a);
+                acc[0] = dd_add_prod(acc[0], ald(s2 + e), a);
             }
-            reduce_publish<1>(P.rb, 6, acc, lds);
-        }
-        ok = ok && grid_sync(P.gs, ws);
-        double alpha;
-        {
-            double o[1];
-            reduce_collect<1>(P.rb, 6, gridDim.x, o, lds);
+            double o[1] = {0.0};
+            ok = ok && grid_sum<1>(P.gs, ws, acc, o);
             if (P.exact_dots) o[0] = seq_dot(s2, P.Ahp, nel);
             alpha = r1z1 / o[0];
         }
         {
-            dd acc[4] = {dd_zero(), dd_zero(), dd_zero(), dd_zero()};
+            dd acc[5] = {dd_zero(), dd_zero(), dd_zero(), dd_zero(), dd_zero()};
             for (int e = gtid; e < nel; e += gsize) {
-                r2[e] = r1[e] - alpha * P.Ahp[e];
-                double pe = P.p[e] + alpha * s2[e];
-                P.p[e] = pe;
-                acc[0] = dd_add_prod(acc[0], s2[e], s2[e]);
+                const double r = ald(r1 + e) - alpha * ald(P.Ahp + e), se = ald(s2 + e), z = zvec(e, r);
+                const double pe = ald(P.p + e) + alpha * se;
+                ast(r2 + e, r);
+                ast(P.p + e, pe);
+                ast(z0 + e, z);   // z0's buffer becomes z1
+                acc[0] = dd_add_prod(acc[0], se, se);
                 acc[1] = dd_add_prod(acc[1], pe, pe);
+                acc[4] = dd_add_prod(acc[4], r, z);
             }
             for (int i = gtid; i < neq; i += gsize) {
-                double u = P.u1[i];
-                double di = P.d[i] - alpha * u;
-                P.d[i] = di;
+                const double u = ald(P.u1 + i), di = ald(P.d + i) - alpha * u;
+                ast(P.d + i, di);
                 acc[2] = dd_add_prod(acc[2], u, u);
                 acc[3] = dd_add_prod(acc[3], di, di);
             }
-            reduce_publish<4>(P.rb, 8, acc, lds);
-        }
-        ok = ok && grid_sync(P.gs, ws);
-        {
-            double o[4];
-            reduce_collect<4>(P.rb, 8, gridDim.x, o, lds);
+            double o[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+            ok = ok && grid_sum<5>(P.gs, ws, acc, o);
             if (P.exact_dots) {
                 o[0] = seq_dot(s2, s2, nel);
                 o[1] = seq_dot(P.p, P.p, nel);
                 o[2] = seq_dot(P.u1, P.u1, neq);
                 o[3] = seq_dot(P.d, P.d, neq);
+                o[4] = seq_dot(r2, z0, nel);
+                ok = ok && grid_wait(P.gs, ws);   // the next phases write s2's and u1's successors
             }
             dp = alpha * sqrt(o[0] / (1.0e-32 + o[1]));
             dv = alpha * sqrt(o[2] / (1.0e-32 + o[3]));
+            r0z0 = r1z1;
+            r1z1 = o[4];
         }
         cycle++;
         double *sh;
@@ -725,6 +792,16 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
         P.stats->t_end = wall_clock64();
     }
     sync_end(P.gs, ws);
+}
+
+const void *mcl_uzawa_fp64_kernel(int solver)
+{
+    switch (solver) {
+    case MCL_INNER_JC: return (const void *)k_uzawa_fp64<MCL_INNER_JC>;
+    case MCL_INNER_GS: return (const void *)k_uzawa_fp64<MCL_INNER_GS>;
+    case MCL_INNER_MG: return (const void *)k_uzawa_fp64<MCL_INNER_MG>;
+    default: return (const void *)k_uzawa_fp64<MCL_INNER_CG>;
+    }
 }
 
 // Zero n 32-bit words (a kernel rather than hipMemsetAsync, so that a caller
@@ -851,15 +928,25 @@ __device__ __forceinline__ void elem_center_u(const LevelDev &L, int e, const do
 
 // Heat row assembly (K_matrix_heat :293-423 with get_element_K_heat,
 // F_matrix_heat :425-508, C_matrix_heat :510-594): one thread per heat row,
-// element-ascending sums accumulated in place in the row's own slots.
-__device__ void heat_assemble_row(const LevelDev &L, const HeatParams &H, int P)
+// element-ascending sums accumulated in the thread's own LDS column for rows of
+// at most 9 slots (written to HBM once), else in place in the row's own slots;
+// the additions to each slot come in the same order either way.
+#define MCL_HEAT_LDS_SLOTS 9
+__device__ __forceinline__ void heat_assemble_row(const LevelDev &L, const HeatParams &H, const ShapeTables &S, int P,
+                                                  double *lk, double *lc)
 {
     const int n = L.heq_node[P];
     const int nadj = L.p2n_cnt[n];
     const int nT = L.neqT;
+    const bool inl = L.WT <= MCL_HEAT_LDS_SLOTS;
     for (int s = 0; s < L.WT; s++) {
-        H.hK[s * nT + P] = 0.0;
-        H.hC[s * nT + P] = 0.0;
+        if (inl) {
+            lk[s * MCL_BLOCK] = 0.0;
+            lc[s * MCL_BLOCK] = 0.0;
+        } else {
+            H.hK[s * nT + P] = 0.0;
+            H.hC[s * nT + P] = 0.0;
+        }
     }
     double F = 0.0;
     for (int k = 0; k < nadj; k++) {
@@ -873,26 +960,31 @@ __device__ void heat_assemble_row(const LevelDev &L, const HeatParams &H, int P)
             u1 += H.V[kn] * 0.25;
             u2 += H.V[L.nno + kn] * 0.25;
         }
-        double t0 = H.tau[e], t1 = H.tau[L.nel + e];
+        double t0 = ald(H.tau + e), t1 = ald(H.tau + L.nel + e);
         for (int b = 0; b < 4; b++) {
             double kv = 0.0, cv = 0.0;
             for (int g = 0; g < 4; g++) {
-                double ax = c_shape.dxi[a][g] * dzdeta - c_shape.deta[a][g] * 0.0;
-                double az = c_shape.deta[a][g] * dxdxi - c_shape.dxi[a][g] * 0.0;
-                double bx = c_shape.dxi[b][g] * dzdeta - c_shape.deta[b][g] * 0.0;
-                double bz = c_shape.deta[b][g] * dxdxi - c_shape.dxi[b][g] * 0.0;
+                double ax = S.dxi[a][g] * dzdeta - S.deta[a][g] * 0.0;
+                double az = S.deta[a][g] * dxdxi - S.dxi[a][g] * 0.0;
+                double bx = S.dxi[b][g] * dzdeta - S.deta[b][g] * 0.0;
+                double bz = S.deta[b][g] * dxdxi - S.dxi[b][g] * 0.0;
                 double nh = t0 * ax + t1 * az;
-                double tt1 = u1 * c_shape.N[a][g] * bx + u2 * c_shape.N[a][g] * bz;
+                double tt1 = u1 * S.N[a][g] * bx + u2 * S.N[a][g] * bz;
                 double tt2 = u1 * nh * bx + u2 * nh * bz;
                 double tt3 = ax * 1.0 * bx + ax * 0.0 * bz + az * 0.0 * bx + az * 1.0 * bz;
                 kv += tt1 + (tt2 + tt3) / jac;
-                cv += (c_shape.N[a][g] + nh) * c_shape.N[b][g];
+                cv += (S.N[a][g] + nh) * S.N[b][g];
             }
             cv *= jac;
             int slot = L.Tslot[(k * 4 + b) * nT + P];
             if (slot >= 0) {
-                H.hK[slot * nT + P] += kv;
-                H.hC[slot * nT + P] += cv;
+                if (inl) {
+                    lk[slot * MCL_BLOCK] += kv;
+                    lc[slot * MCL_BLOCK] += cv;
+                } else {
+                    H.hK[slot * nT + P] += kv;
+                    H.hC[slot * nT + P] += cv;
+                }
             }
             int nb = L.ienl[b * L.nel + e];
             if (L.T_bc[nb] == 'T') F -= kv * L.T_bc_val[nb];
@@ -903,7 +995,7 @@ __device__ void heat_assemble_row(const LevelDev &L, const HeatParams &H, int P)
         int lev = L.elev[e];
         double dxdxi = 0.5 * L.lvl_dx[lev], dzdeta = 0.5 * L.lvl_dz[lev];
         double jac = dxdxi * dzdeta - 0.0 * 0.0;
-        double t0 = H.tau[e], t1 = H.tau[L.nel + e];
+        double t0 = ald(H.tau + e), t1 = ald(H.tau + L.nel + e);
         int nat = 0;
         for (int c = 0; c < 4; c++)
             if (L.T_bc[L.ienl[c * L.nel + e]] == 'F') nat += c;
@@ -912,31 +1004,39 @@ __device__ void heat_assemble_row(const LevelDev &L, const HeatParams &H, int P)
         else if (nat == 0 || nat == 2) nat = 0;
         double f = 0.0;
         for (int g = 0; g < 4; g++) {
-            double ax = c_shape.dxi[a][g] * dzdeta - c_shape.deta[a][g] * 0.0;
-            double az = c_shape.deta[a][g] * dxdxi - c_shape.dxi[a][g] * 0.0;
+            double ax = S.dxi[a][g] * dzdeta - S.deta[a][g] * 0.0;
+            double az = S.deta[a][g] * dxdxi - S.dxi[a][g] * 0.0;
             double nh = t0 * ax + t1 * az;
-            f += (c_shape.N[a][g] + nh) * H.Q;
+            f += (S.N[a][g] + nh) * H.Q;
         }
         f *= jac;
         if (nat != 0) f -= 0.5 * L.lvl_dz[lev] * L.T_bc_val[L.ienl[a * L.nel + e]];
         F += f;
     }
     H.hF[P] = F;
+    if (inl)
+        for (int s = 0; s < L.WT; s++) {
+            H.hK[s * nT + P] = lk[s * MCL_BLOCK];
+            H.hC[s * nT + P] = lc[s * MCL_BLOCK];
+        }
 }
 
 // update_temperature (Update_temperature.c:3-133) as one persistent kernel.
 __global__ void __launch_bounds__(MCL_BLOCK) k_heat_fp64(HeatParams H)
 {
-    __shared__ dd lds[MCL_RED_ROWS][MCL_BLOCK / MCL_WAVE];
-    __shared__ double ldsm[MCL_BLOCK / MCL_WAVE];
+    __shared__ double lds[2 * MCL_HEAT_LDS_SLOTS * MCL_BLOCK];
+    __shared__ ShapeTables S;   // a thread's corner picks its entries: LDS serves 64 different ones at once
     const LevelDev &L = H.L;
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsize = gridDim.x * blockDim.x;
     const int n = L.neqT, nel = L.nel;
+    for (int t = threadIdx.x; t < (int)(sizeof S / sizeof(double)); t += blockDim.x)
+        ((double *)&S)[t] = ((const double *)&c_shape)[t];
     WaitState ws;
     bool ok = sync_begin(H.gs, ws);
     long long spmv = 0;
-    // tau per element and the advective dt bound
-    double dtmin = 1e10;
+    // tau per element and the advective dt bound: the smallest 0.5 / uu is 0.5
+    // over the largest uu (rounding is monotone)
+    double umax[1] = {0.0};
     for (int e = gtid; e < nel; e += gsize) {
         int lev = L.elev[e];
         double Lx = L.lvl_dx[lev], Lz = L.lvl_dz[lev];
@@ -950,64 +1050,66 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_heat_fp64(HeatParams H)
         }
         double us = (u[0] * u[0] + u[1] * u[1]);
         double kh = (xi[0] * u[0] * Ld[0] + xi[1] * u[1] * Ld[1]) * 0.5;
-        H.tau[e] = kh * u[0] / us;
-        H.tau[nel + e] = kh * u[1] / us;
+        ast(H.tau + e, kh * u[0] / us);
+        ast(H.tau + nel + e, kh * u[1] / us);
         // advection_dt with the sizes of the last element (H.Llast)
         double uu = fabs(u[0]) / H.Llast0 + fabs(u[1]) / H.Llast1;
-        double step = 0.5 / uu;
-        dtmin = step < dtmin ? step : dtmin;
+        umax[0] = fmax(umax[0], uu);
     }
-    {
-        double bm = block_min(dtmin, ldsm);
-        if (threadIdx.x == 0) H.rb.pmax[1 * MCL_MAX_WG + blockIdx.x] = bm;
-    }
-    ok = ok && grid_sync(H.gs, ws);
-    for (int P = gtid; P < n; P += gsize) heat_assemble_row(L, H, P);
     double dt;
     {
-        double m = 1e10;
-        for (int b = threadIdx.x; b < (int)gridDim.x; b += MCL_BLOCK) {
-            double v = H.rb.pmax[1 * MCL_MAX_WG + b];
-            m = v < m ? v : m;
-        }
-        dt = block_min(m, ldsm);
+        dd none[1] = {dd_zero()};
+        double o[1] = {0.0};
+        ok = ok && grid_reduce<0, 1>(H.gs, ws, none, umax, o);
+        const double step = 0.5 / o[0];
+        dt = step < 1e10 ? step : 1e10;
         dt = dt < H.diff_dt ? dt : H.diff_dt;
         dt = dt * 0.75;
     }
-    ok = ok && grid_sync(H.gs, ws);
-    EllMat Kh{L.Tcol, L.Tncol, H.hK, nullptr, L.Tdiag_slot, n};
-    EllMat Ch{L.Tcol, L.Tncol, H.hC, nullptr, L.Tdiag_slot, n};
-    EllMat Ah{L.Tcol, L.Tncol, H.hA, nullptr, L.Tdiag_slot, n};
-    CgVecs cv{H.cg_r, H.cg_s, H.cg_d, H.cg_q};
+    // rows, matrices and right-hand sides belong to their thread from here on;
+    // the waits are those of the vectors that the products gather
+    for (int P = gtid; P < n; P += gsize)
+        heat_assemble_row(L, H, S, P, lds + threadIdx.x, lds + MCL_HEAT_LDS_SLOTS * MCL_BLOCK + threadIdx.x);
+    EllMat Ch{L.Tcol, L.Tncol, H.hC, nullptr, L.Tdiag_slot, n, L.WT};
+    EllMat Ah{L.Tcol, L.Tncol, H.hA, nullptr, L.Tdiag_slot, n, L.WT};
+    CgVecs cv{H.cg_r, H.cg_s, H.cg_d, H.cg_q, H.cg_d2};
+    auto hd = [&](int j) { return ald(H.hd + j); };
+    // one of the two matrices at a time in registers; the LDS columns of the
+    // assembly become the window
+    static_assert(2 * MCL_HEAT_LDS_SLOTS * MCL_BLOCK >= MCL_WINDOW, "the window lies in the assembly's LDS");
+    RowReg<9> row;
+    auto cg = [&](const EllMat &A, double *x, bool x_zero, int max_cycle) __attribute__((always_inline)) {
+        __syncthreads();
+        const Window win = row_window(row, A.col, A.ncol, A.val, A.width, n, lds);
+        const double diag = gtid < n ? ell_diag(A, gtid) : 1.0;
+        return pcg_persistent<9>(L, A, row, win, diag, H.B, x, x_zero, 1e-3, max_cycle, H.cg_precondition, 1, cv, H.gs,
+                                 ws, ok, spmv, H.exact_dots != 0);
+    };
     int init_cycles = 0;
     if (H.first_call) {
         // initial_T_dot (:179-239)
-        for (int i = gtid; i < n; i += gsize) H.hd[i] = H.T[L.heq_node[i]];
-        ok = ok && grid_sync(H.gs, ws);
+        for (int i = gtid; i < n; i += gsize) ast(H.hd + i, H.T[L.heq_node[i]]);
+        ok = ok && grid_wait(H.gs, ws);
         for (int i = gtid; i < n; i += gsize) {
-            H.B[i] = H.hF[i] - ell_row(L.Tcol, H.hK, L.Tncol[i], n, i, H.hd);
-            H.hdd[i] = 0.0;
+            H.B[i] = H.hF[i] - ell_row_ld(L.Tcol, H.hK, L.Tncol[i], n, i, hd);
+            ast(H.hdd + i, 0.0);
         }
-        ok = ok && grid_sync(H.gs, ws);
-        init_cycles = pcg_persistent(L, Ch, H.B, H.hdd, true, 1e-3, 400, H.cg_precondition, 1, cv, H.gs, ws,
-                                     H.rb, lds, ldsm, ok, spmv, H.exact_dots != 0);
+        init_cycles = cg(Ch, H.hdd, true, 400);
     }
     const double td = H.theta * dt;
     for (int i = gtid; i < n; i += gsize) {
-        double ct = ell_row(L.Tcol, H.hC, L.Tncol[i], n, i, H.hd);
-        H.d0[i] = H.hd[i];
+        double ct = ell_row_ld(L.Tcol, H.hC, L.Tncol[i], n, i, hd);
+        H.d0[i] = hd(i);
         H.B[i] = H.hF[i] + ct / td;
         for (int s = 0; s < L.Tncol[i]; s++) H.hA[s * n + i] = H.hC[s * n + i] / td + H.hK[s * n + i];
     }
-    ok = ok && grid_sync(H.gs, ws);
-    int cycles = pcg_persistent(L, Ah, H.B, H.hd, false, 1e-3, 1000, H.cg_precondition, 1, cv, H.gs, ws, H.rb, lds,
-                                ldsm, ok, spmv, H.exact_dots != 0);
+    int cycles = cg(Ah, H.hd, false, 1000);
     for (int i = gtid; i < L.nno; i += gsize) {
         int k = L.heat_id[i];
-        H.T[i] = k >= 0 ? H.hd[k] : L.T_bc_val[i];
+        H.T[i] = k >= 0 ? hd(k) : L.T_bc_val[i];
     }
     for (int i = gtid; i < n; i += gsize)
-        H.hdd[i] = 1.0 / (H.theta * dt) * (H.hd[i] - H.d0[i]) - (1.0 - H.theta) / H.theta * H.hdd[i];
+        ast(H.hdd + i, 1.0 / (H.theta * dt) * (hd(i) - H.d0[i]) - (1.0 - H.theta) / H.theta * ald(H.hdd + i));
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         H.stats->cycles = cycles;
         H.stats->init_cycles = init_cycles;

@@ -106,7 +106,7 @@ struct UzawaParams {
     DevStats *stats;
     double *d, *p, *u1, *Ahv, *Ahp, *BAB;
     double *r0, *r1, *r2, *z0, *z1, *s1, *s2;
-    double *cg_r, *cg_s, *cg_d, *cg_q;
+    double *cg_r, *cg_s, *cg_d, *cg_q, *cg_d2;
     double accuracy, citcom_accu;
     int max_citcom_cycle, max_cg_cycle, cg_precondition, check_v_only, schur;
     int exact_dots;          // dot products in the reference's sequential order
@@ -125,7 +125,7 @@ struct HeatParams {
     DevStats *stats;
     const double *V;
     double *T, *tau, *hK, *hC, *hA, *hF, *hd, *hdd, *d0, *B;
-    double *cg_r, *cg_s, *cg_d, *cg_q;
+    double *cg_r, *cg_s, *cg_d, *cg_q, *cg_d2;
     double *model_time;
     double accuracy, theta, Q, Llast0, Llast1, diff_dt;
     int first_call, cg_precondition;
@@ -257,7 +257,8 @@ struct AsmLevel {
     int blk0;
 };
 __global__ void k_assemble_K(const AsmLevel *lv, int nlev);
-__global__ void k_uzawa_fp64(UzawaParams P);
+// k_uzawa_fp64 for an inner solver (MCL_INNER_*)
+const void *mcl_uzawa_fp64_kernel(int solver);
 __global__ void k_v_to_nodes(LevelDev L, const double *d, double *V);
 __global__ void k_stress_elem(LevelDev L, const double *vis, const double *V, double *es, double *area);
 __global__ void k_stress_node(LevelDev L, const double *es, const double *area, double *stress);

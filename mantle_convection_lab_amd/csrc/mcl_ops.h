@@ -5,10 +5,24 @@
 #pragma once
 #include "mcl_kernels.h"
 
+// Agent-scope accesses of vectors that other workgroups write or read between
+// two grid waits (GridSync).
+__device__ __forceinline__ double ald(const double *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void ast(double *p, double v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ------------------------------------------------------------- sparse products
 
-__device__ __forceinline__ double ell_row(const int *__restrict__ col, const double *__restrict__ val, int ncol,
-                                          int n, int row, const double *__restrict__ x)
+// (the vector's values read through load(j))
+template <typename LD>
+__device__ __forceinline__ double ell_row_ld(const int *__restrict__ col, const double *__restrict__ val, int ncol,
+                                             int n, int row, LD load)
 {
     // loads issued nine entries at a time (one memory round trip per chunk
     // instead of per entry); the sum keeps the ascending-column order
@@ -16,17 +30,116 @@ __device__ __forceinline__ double ell_row(const int *__restrict__ col, const dou
     int j = 0;
     for (; j + 9 <= ncol; j += 9) {
         int c[9];
-        double v[9];
+        double v[9], x[9];
 #pragma unroll
         for (int u = 0; u < 9; u++) {
             c[u] = col[(j + u) * n + row];
             v[u] = val[(j + u) * n + row];
         }
 #pragma unroll
-        for (int u = 0; u < 9; u++) s += v[u] * x[c[u]];
+        for (int u = 0; u < 9; u++) x[u] = load(c[u]);
+#pragma unroll
+        for (int u = 0; u < 9; u++) s += v[u] * x[u];
     }
-    for (; j < ncol; j++) s += val[j * n + row] * x[col[j * n + row]];
+    for (; j < ncol; j++) s += val[j * n + row] * load(col[j * n + row]);
     return s;
+}
+
+__device__ __forceinline__ double ell_row(const int *__restrict__ col, const double *__restrict__ val, int ncol,
+                                          int n, int row, const double *__restrict__ x)
+{
+    return ell_row_ld(col, val, ncol, n, row, [&](int j) { return x[j]; });
+}
+
+// Products of a persistent solve whose threads own at most one row each (row
+// = global thread number): the workgroup's rows are consecutive, so the vector
+// entries they read lie in a window of the vector (the rows of a few mesh
+// lines), which is read once, in order, into LDS; the row itself -- offsets
+// into the window and values -- stays in registers over the whole solve.
+// Gathering through agent-scope loads instead moves every entry up to 18 times
+// past the L2.
+#define MCL_WINDOW 6144   // doubles of LDS
+struct Window {
+    double *buf;    // LDS
+    int w0, n;      // vector entries [w0, w0 + n)
+    bool fits;
+    // the entries value(j) of the window into LDS, four loads in flight
+    template <typename F>
+    __device__ __forceinline__ void fill(F value) const
+    {
+        for (int j = threadIdx.x; j < n; j += 4 * MCL_BLOCK) {
+            double v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = j + k * MCL_BLOCK < n ? value(w0 + j + k * MCL_BLOCK) : 0.0;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (j + k * MCL_BLOCK < n) buf[j + k * MCL_BLOCK] = v[k];
+        }
+        __syncthreads();
+    }
+};
+
+template <int W>
+struct RowReg {
+    int n;             // entries
+    unsigned off[W];   // byte offsets in the window
+    double v[W];
+    // the row times the window's vector, in ell_row's order; skip: a slot
+    // left out (-1: none)
+    __device__ __forceinline__ double dot(const double *buf, int skip = -1) const
+    {
+        double x[W], s = 0.0;
+#pragma unroll
+        for (int u = 0; u < W; u++) x[u] = *(const double *)((const char *)buf + off[u]);
+        // opaque to the compiler, which would otherwise keep the comparisons
+        // of every slot with them in scalar registers over the whole solve
+        int m = n, k = skip;
+        asm volatile("" : "+v"(m), "+v"(k));
+#pragma unroll
+        for (int u = 0; u < W; u++)
+            if (u < m && u != k) s += v[u] * x[u];
+        return s;
+    }
+};
+
+// This thread's row of a matrix (row < rows: col, val slot-major, wk slots)
+// and the workgroup's window; fits = false: more slots than W, more rows than
+// threads, or a wider window than the LDS holds.
+template <int W>
+__device__ __forceinline__ Window row_window(RowReg<W> &r, const int *__restrict__ col, const int *__restrict__ ncol,
+                                             const double *__restrict__ val, int wk, int rows, double *buf)
+{
+    __shared__ int lo, hi;
+    const int row = blockIdx.x * blockDim.x + threadIdx.x;
+    Window w{buf, 0, 0, wk <= W && rows <= (int)(gridDim.x * blockDim.x)};
+    if (!w.fits) return w;
+    if (threadIdx.x == 0) {
+        lo = 0x7fffffff;
+        hi = -1;
+    }
+    __syncthreads();
+    r.n = row < rows ? ncol[row] : 0;
+    int c[W], l = 0x7fffffff, h = -1;
+#pragma unroll
+    for (int u = 0; u < W; u++) {
+        c[u] = u < r.n ? col[u * rows + row] : row;
+        r.v[u] = u < r.n ? val[u * rows + row] : 0.0;
+        if (u < r.n) {
+            l = min(l, c[u]);
+            h = max(h, c[u]);
+        }
+    }
+    if (r.n > 0) {
+        atomicMin(&lo, min(l, row));
+        atomicMax(&hi, max(h, row));
+    }
+    __syncthreads();
+    w.w0 = hi < 0 ? 0 : lo;
+    w.n = hi < 0 ? 0 : hi - lo + 1;
+    w.fits = w.n <= MCL_WINDOW;
+#pragma unroll
+    for (int u = 0; u < W; u++) r.off[u] = 8u * (unsigned)(u < r.n ? c[u] - w.w0 : 0);
+    return w;
 }
 
 // (G p)[P], G_prod_p (Solver.c:569-591): columns are the row's elements, ascending.
@@ -71,10 +184,11 @@ __device__ __forceinline__ double gt_elem(const LevelDev &L, int e, const double
 // ------------------------------------------------------------ persistent Uzawa
 
 struct CgVecs {
-    double *r, *s, *d, *q;
+    double *r, *s, *d, *q, *d2;   // d2: the other buffer of d
 };
 
-// Hanging-dof constraint, enforce_constrain_veq (Solver.c:1368-1437).
+// Hanging-dof constraint, enforce_constrain_veq (Solver.c:1368-1437); the
+// parents and the hanging values may belong to other workgroups.
 static __device__ __forceinline__ void constrain_v(const LevelDev &L, double *__restrict__ x, int gtid, int gsize)
 {
     if (L.nh == 0) return;
@@ -86,11 +200,11 @@ static __device__ __forceinline__ void constrain_v(const LevelDev &L, double *__
                 for (int c = 0; c < 2; c++) {
                     int kn = L.h_ci[c * L.nh + k];
                     int eqc = L.id[d * L.nno + kn];
-                    t += eqc != -1 ? x[eqc] : L.v_bc_val[d * L.nno + kn];
+                    t += eqc != -1 ? ald(x + eqc) : L.v_bc_val[d * L.nno + kn];
                 }
                 t *= 0.5;
                 int eq = L.id[d * L.nno + L.h_ni[k]];
-                if (eq >= 0) x[eq] = t;
+                if (eq >= 0) ast(x + eq, t);
             }
         }
         return;
@@ -101,11 +215,11 @@ static __device__ __forceinline__ void constrain_v(const LevelDev &L, double *__
             for (int c = 0; c < 2; c++) {
                 int kn = L.h_ci[c * L.nh + k];
                 int eqc = L.id[d * L.nno + kn];
-                t += eqc != -1 ? x[eqc] : L.v_bc_val[d * L.nno + kn];
+                t += eqc != -1 ? ald(x + eqc) : L.v_bc_val[d * L.nno + kn];
             }
             t *= 0.5;
             int eq = L.id[d * L.nno + L.h_ni[k]];
-            if (eq >= 0) x[eq] = t;
+            if (eq >= 0) ast(x + eq, t);
         }
     }
 }
@@ -120,11 +234,11 @@ static __device__ __forceinline__ void constrain_T(const LevelDev &L, double *__
         for (int c = 0; c < 2; c++) {
             int kn = L.h_ci[c * L.nh + k];
             int eqc = L.heat_id[kn];
-            t += eqc != -1 ? x[eqc] : L.T_bc_val[kn];
+            t += eqc != -1 ? ald(x + eqc) : L.T_bc_val[kn];
         }
         t *= 0.5;
         int eq = L.heat_id[L.h_ni[k]];
-        if (eq >= 0) x[eq] = t;
+        if (eq >= 0) ast(x + eq, t);
     }
 }
 
@@ -135,7 +249,7 @@ struct EllMat {
     const double *val;
     const double *diag;      // diagonal values, or NULL to use diag_slot
     const int *diag_slot;
-    int n;
+    int n, width;            // rows; slots per row
 };
 
 __device__ __forceinline__ double ell_diag(const EllMat &A, int i)
