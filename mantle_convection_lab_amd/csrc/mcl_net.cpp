@@ -35,22 +35,22 @@ struct ConvShape {
 };
 __global__ void k_conv3_fwd(ConvShape s, const uint16_t *in, const uint16_t *Wf, const float *bias, uint16_t *out,
                             int relu);
-__global__ void k_conv3_dgrad(ConvShape s, const uint16_t *dout, const uint16_t *relu_y, const uint16_t *Wd,
-                              uint16_t *din, int accum);
-__global__ void k_conv3_wgrad(ConvShape s, const uint16_t *dout, const uint16_t *relu_y, const uint16_t *in,
-                              float *dW, int pix_per_split);
-__global__ void k_conv3_mm(ConvShape s, int dgrad, const uint16_t *X, const uint16_t *mask, const uint16_t *Wt,
-                           const float *bias, uint16_t *Y, int flag);
-__global__ void k_conv3_mm_n32(ConvShape s, int dgrad, const uint16_t *X, const uint16_t *mask, const uint16_t *Wt,
-                               const float *bias, uint16_t *Y, int flag);
-__global__ void k_conv3_wgrad_mm(ConvShape s, const uint16_t *dout, const uint16_t *relu_y, const uint16_t *in,
-                                 float *dW, float *db, int tiles_per_split);
-__global__ void k_bias_grad(int M, int Cout, int cs, int coff, const uint16_t *dout, const uint16_t *relu_y,
-                            float *db);
+__global__ void k_conv3_dgrad(ConvShape s, const uint16_t *dout, const uint16_t *act, const uint16_t *Wd,
+                              uint16_t *din);
+__global__ void k_conv3_wgrad(ConvShape s, const uint16_t *dout, const uint16_t *in, float *dW, int pix_per_split);
+template <int MR, int NB, int WX, int WY, bool DG>
+__global__ void k_conv3_tile(ConvShape s, const uint16_t *X, const uint16_t *act, const uint16_t *Wt, const float *bias,
+                             uint16_t *Y, int relu);
+__global__ void k_conv3_mm(ConvShape s, int dgrad, const uint16_t *X, const uint16_t *act, const uint16_t *Wt,
+                           const float *bias, uint16_t *Y, int relu);
+template <int NBLK, int TH>
+__global__ void k_conv3_wgrad_tile(ConvShape s, const uint16_t *dout, const uint16_t *in, float *dW, float *db,
+                                   int tiles_per_split);
+__global__ void k_bias_grad(int M, int Cout, int cs, int coff, const uint16_t *dout, float *db);
 __global__ void k_pool_fwd(int B, int H, int W, int C, const uint16_t *in, int cs_in, int ci_off, uint16_t *out,
                            int cs_out, int co_off);
-__global__ void k_pool_bwd(int B, int H, int W, int C, const uint16_t *dout, int cs_out, int co_off, uint16_t *din,
-                           int cs_in, int ci_off, int accum);
+__global__ void k_pool_bwd(int B, int H, int W, int C, const uint16_t *dout, int cs_out, int co_off,
+                           const uint16_t *act, uint16_t *din, int cs_in, int ci_off);
 __global__ void k_up_fwd(int B, int H, int W, int C, const uint16_t *in, int cs_in, int ci_off, uint16_t *out,
                          int cs_out, int co_off);
 __global__ void k_up_bwd(int B, int H, int W, int C, const uint16_t *dout, int cs_out, int co_off, uint16_t *din,
@@ -149,86 +149,102 @@ static int make_conv(mcl_net *n, Conv &c, int Cin, int Cout, std::mt19937_64 &rn
 
 static unsigned gblocks(size_t n) { return (unsigned)std::min<size_t>((n + 255) / 256, 8192); }
 
-// The LDS-staged kernels (k_conv3_mm: 64 pixels x 64 channels a workgroup;
-// k_conv3_mm_n32: 128 x 32, for N <= 32 output channels) apply when MT
-// consecutive pixels form a rectangle of one image (TW = min(W, MT) divides
-// both W and MT, TH = MT / TW divides H) and the summed channels and the
-// staged buffer's channel stride and offset are multiples of 8 (16-byte
-// loads).  Returns MT, or 0 for the unstaged kernels; MCL_CONV_DIRECT=1
-// keeps the unstaged kernels (for comparisons).
-static int conv_staged(const ConvShape &s, int N, int Kc, int xst, int xof)
+// MCL_CONV_DIRECT=1 keeps the unstaged kernels everywhere (for comparisons).
+static bool conv_direct()
 {
     const char *e = getenv("MCL_CONV_DIRECT");
-    if (e && atoi(e)) return 0;
-    if (Kc % 8 || xst % 8 || xof % 8) return 0;
-    const int MT = N <= 32 ? 128 : 64;
-    const int TW = s.W < MT ? s.W : MT;
-    if (TW <= 0 || s.W % TW || MT % TW || s.H % (MT / TW)) return 0;
-    return MT;
+    return e && atoi(e);
 }
 
-// one launch of the staged kernel of tile MT (64 or 128) over M pixels, N channels
-static void conv_mm(mcl_net *n, const ConvShape &s, int MT, int M, int N, int dgrad, const uint16_t *X,
-                    const uint16_t *mask, const uint16_t *Wt, const float *bias, uint16_t *Y, int flag)
+// One 3x3 product of `dg` = false: the forward pass, true: the data gradient.
+// Tiles of whole 16-pixel runs (k_conv3_tile) need a width that is a multiple
+// of 16 and 16-byte aligned pixels of the summed buffer; the tile is the
+// largest that leaves at least a workgroup a CU (the large ones stage less and
+// read less LDS per MFMA; a layer with few pixels is bound by the latency of
+// its chunks, which only more workgroups hide).  A forward pass of 15 images of
+// 32 x 256 takes 362 us with that line at one workgroup a CU, 371 at two, 384
+// at four; the 14 products of one 256 x 256 image take 119 us (280 us as 64
+// pixels x 64 channels a workgroup throughout).  Narrower layers whose 64
+// consecutive pixels form a rectangle of one image take k_conv3_mm, the rest
+// the unstaged kernels.
+template <bool DG>
+static void conv_product(mcl_net *n, const ConvShape &s, const uint16_t *X, const uint16_t *act, const uint16_t *Wt,
+                         const float *bias, uint16_t *Y, int relu)
 {
-    if (MT == 128)
-        hipLaunchKernelGGL(k_conv3_mm_n32, dim3(M / 128, (N + 31) / 32), dim3(256), 0, n->stream, s, dgrad, X, mask,
-                           Wt, bias, Y, flag);
+    const int Kc = DG ? s.Cout : s.Cin, N = DG ? s.Cin : s.Cout;
+    const int xst = DG ? s.cs_out : s.cs_in, xof = DG ? s.co_off : s.ci_off;
+    const int M = s.B * s.H * s.W;
+    const bool staged = !conv_direct() && Kc % 8 == 0 && xst % 8 == 0 && xof % 8 == 0;
+    if (staged && s.W % 16 == 0 && s.H % 4 == 0 && N % 32 == 0) {
+        auto fits = [&](int px, int tw, int th, int nt, int least) {
+            return s.W % tw == 0 && s.H % th == 0 && N % nt == 0 && (long long)(M / px) * (N / nt) >= least;
+        };
+#define CONV_TILE(MR, NB, WX, WY)                                                                                   \
+    hipLaunchKernelGGL((k_conv3_tile<MR, NB, WX, WY, DG>), dim3((M / (16 * WX * MR * WY)) * (N / (16 * NB))),         \
+                       dim3(64 * WX * WY), 0, n->stream, s, X, act, Wt, bias, Y, relu)
+        if (fits(256, 32, 8, 64, 256)) CONV_TILE(4, 4, 2, 2);
+        else if (fits(256, 32, 8, 32, 256)) CONV_TILE(4, 2, 2, 2);
+        else if (fits(128, 32, 4, 32, 256)) CONV_TILE(2, 2, 2, 2);
+        else if (fits(64, 32, 2, 32, 1)) CONV_TILE(1, 2, 2, 2);
+        else CONV_TILE(1, 2, 1, 4);
+#undef CONV_TILE
+        return;
+    }
+    const int TW = s.W < 64 ? s.W : 64;
+    if (staged && s.W % TW == 0 && 64 % TW == 0 && s.H % (64 / TW) == 0) {
+        hipLaunchKernelGGL(k_conv3_mm, dim3(M / 64, (N + 63) / 64), dim3(256), 0, n->stream, s, DG ? 1 : 0, X, act, Wt,
+                           bias, Y, relu);
+        return;
+    }
+    if constexpr (DG)
+        hipLaunchKernelGGL(k_conv3_dgrad, dim3((M + 63) / 64, (N + 63) / 64), dim3(256), 0, n->stream, s, X, act, Wt, Y);
     else
-        hipLaunchKernelGGL(k_conv3_mm, dim3(M / 64, (N + 63) / 64), dim3(256), 0, n->stream, s, dgrad, X, mask, Wt,
-                           bias, Y, flag);
+        hipLaunchKernelGGL(k_conv3_fwd, dim3((M + 63) / 64, (N + 63) / 64), dim3(256), 0, n->stream, s, X, Wt, bias, Y,
+                           relu);
 }
 
 static void conv_fwd(mcl_net *n, Conv &c, const Act &in, int ci_off, Act &out, int co_off, bool relu)
 {
     ConvShape s{n->B, in.H, in.W, c.Cin, c.Cout, in.C, ci_off, out.C, co_off};
-    int M = n->B * in.H * in.W;
-    const int MT = conv_staged(s, c.Cout, c.Cin, in.C, ci_off);
-    if (MT)
-        conv_mm(n, s, MT, M, c.Cout, 0, (const uint16_t *)in.y, nullptr, (const uint16_t *)c.Wf, (const float *)c.b,
-                out.y, relu ? 1 : 0);
-    else
-        hipLaunchKernelGGL(k_conv3_fwd, dim3((M + 63) / 64, (c.Cout + 63) / 64), dim3(256), 0, n->stream, s,
-                           (const uint16_t *)in.y, (const uint16_t *)c.Wf, (const float *)c.b, out.y, relu ? 1 : 0);
+    conv_product<false>(n, s, in.y, nullptr, c.Wf, c.b, out.y, relu ? 1 : 0);
 }
 
-// Backward of a ReLU convolution: weight and bias gradients, and the data
-// gradient into in.g (skipped when din is false).
-static void conv_bwd(mcl_net *n, Conv &c, const Act &in, int ci_off, Act &out, int co_off, bool din, bool accum)
+// Backward of a ReLU convolution whose output gradient out.g is already zero
+// where the ReLU was: weight and bias gradients, and the data gradient into
+// in.g (skipped when din is false), zeroed where the input is not positive if
+// the input is a ReLU's output (in_relu).
+static void conv_bwd(mcl_net *n, Conv &c, const Act &in, int ci_off, Act &out, int co_off, bool din, bool in_relu)
 {
     ConvShape s{n->B, in.H, in.W, c.Cin, c.Cout, in.C, ci_off, out.C, co_off};
-    int M = n->B * in.H * in.W;
-    const uint16_t *mask = out.y;
-    const int TW = in.W < 64 ? in.W : 64;
-    if (conv_staged(s, 64, c.Cin, in.C, ci_off) == 64 && TW % 8 == 0 && out.C % 8 == 0 && co_off % 8 == 0) {
-        // staged weight gradient (and bias gradient): workgroups of 64 x 32 x
-        // 9 taps, about 512 in all, each summing at least 8 tiles of 64 pixels
-        const int tiles = M / 64, nbn = (c.Cout + 63) / 64, nbc = (c.Cin + 31) / 32;
-        int splits = std::max(1, std::min(tiles / 8, 512 / (nbn * nbc)));
+    const int M = n->B * in.H * in.W;
+    const uint16_t *g = out.g, *x = in.y;
+    if (!conv_direct() && in.W % 32 == 0 && in.H % 4 == 0 && c.Cin % 8 == 0 && in.C % 8 == 0 && ci_off % 8 == 0 &&
+        c.Cout % 32 == 0 && out.C % 8 == 0 && co_off % 8 == 0) {
+        // tiles of 32 x 8 pixels (32 x 4 on lower images), about 512
+        // workgroups, each summing at least two tiles where there are that many
+        const int th = in.H % 8 == 0 ? 8 : 4, tiles = M / (32 * th), nblk = c.Cout % 64 == 0 ? 64 : 32;
+        const int nbn = c.Cout / nblk, nbc = (c.Cin + 31) / 32;
+        int splits = std::max(1, std::min((tiles + 1) / 2, 512 / (nbn * nbc)));
         const int tps = (tiles + splits - 1) / splits;
         splits = (tiles + tps - 1) / tps;
-        hipLaunchKernelGGL(k_conv3_wgrad_mm, dim3(nbn, nbc, splits), dim3(256), 0, n->stream, s,
-                           (const uint16_t *)out.g, mask, (const uint16_t *)in.y, c.dw, c.db, tps);
+        const dim3 grid(nbn, nbc, splits);
+#define WGRAD_TILE(NBLK, TH) \
+    hipLaunchKernelGGL((k_conv3_wgrad_tile<NBLK, TH>), grid, dim3(256), 0, n->stream, s, g, x, c.dw, c.db, tps)
+        if (nblk == 64 && th == 8) WGRAD_TILE(64, 8);
+        else if (nblk == 64) WGRAD_TILE(64, 4);
+        else if (th == 8) WGRAD_TILE(32, 8);
+        else WGRAD_TILE(32, 4);
+#undef WGRAD_TILE
     } else {
         int splits = std::max(1, std::min(256, M / 4096));
         int pps = ((M + splits - 1) / splits + 15) / 16 * 16;
         splits = (M + pps - 1) / pps;
         dim3 gw((c.Cout + 63) / 64, (9 * c.Cin + 63) / 64, splits);
-        hipLaunchKernelGGL(k_conv3_wgrad, gw, dim3(256), 0, n->stream, s, (const uint16_t *)out.g, mask,
-                           (const uint16_t *)in.y, c.dw, pps);
+        hipLaunchKernelGGL(k_conv3_wgrad, gw, dim3(256), 0, n->stream, s, g, x, c.dw, pps);
         hipLaunchKernelGGL(k_bias_grad, dim3(std::min(1024, (M + 63) / 64)), dim3(256), 0, n->stream, M, c.Cout,
-                           out.C, co_off, (const uint16_t *)out.g, mask, c.db);
+                           out.C, co_off, g, c.db);
     }
-    if (din) {
-        dim3 gd((M + 63) / 64, (c.Cin + 63) / 64);
-        const int MT = conv_staged(s, c.Cin, c.Cout, out.C, co_off);
-        if (MT)
-            conv_mm(n, s, MT, M, c.Cin, 1, (const uint16_t *)out.g, mask, (const uint16_t *)c.Wd, nullptr, in.g,
-                    accum ? 1 : 0);
-        else
-            hipLaunchKernelGGL(k_conv3_dgrad, gd, dim3(256), 0, n->stream, s, (const uint16_t *)out.g, mask,
-                               (const uint16_t *)c.Wd, in.g, accum ? 1 : 0);
-    }
+    if (din) conv_product<true>(n, s, g, in_relu ? x : nullptr, c.Wd, nullptr, in.g, 0);
 }
 
 static void refresh_bf16(mcl_net *n, Conv &c)
@@ -342,27 +358,27 @@ static void forward(mcl_net *n)
     hipLaunchKernelGGL(k_pack_input, dim3(gblocks(M)), dim3(256), 0, n->stream, M, (const float *)n->xin, n->x0.y);
     conv_fwd(n, n->enc1a, n->x0, 0, n->e1a, 0, true);
     conv_fwd(n, n->enc1b, n->e1a, 0, n->cat1, 64, true);
-    hipLaunchKernelGGL(k_pool_fwd, dim3(gblocks(M / 4 * 32)), dim3(256), 0, n->stream, B, n->H, n->W, 32,
+    hipLaunchKernelGGL(k_pool_fwd, dim3(gblocks(M / 4 * 4)), dim3(256), 0, n->stream, B, n->H, n->W, 32,
                        (const uint16_t *)n->cat1.y, 96, 64, n->p1.y, 32, 0);
     conv_fwd(n, n->enc2a, n->p1, 0, n->e2a, 0, true);
     conv_fwd(n, n->enc2b, n->e2a, 0, n->cat2, 128, true);
-    hipLaunchKernelGGL(k_pool_fwd, dim3(gblocks(M / 16 * 64)), dim3(256), 0, n->stream, B, n->H / 2, n->W / 2, 64,
+    hipLaunchKernelGGL(k_pool_fwd, dim3(gblocks(M / 16 * 8)), dim3(256), 0, n->stream, B, n->H / 2, n->W / 2, 64,
                        (const uint16_t *)n->cat2.y, 192, 128, n->p2.y, 64, 0);
     conv_fwd(n, n->enc3a, n->p2, 0, n->e3a, 0, true);
     conv_fwd(n, n->enc3b, n->e3a, 0, n->cat3, 256, true);
-    hipLaunchKernelGGL(k_pool_fwd, dim3(gblocks(M / 64 * 128)), dim3(256), 0, n->stream, B, n->H / 4, n->W / 4, 128,
+    hipLaunchKernelGGL(k_pool_fwd, dim3(gblocks(M / 64 * 16)), dim3(256), 0, n->stream, B, n->H / 4, n->W / 4, 128,
                        (const uint16_t *)n->cat3.y, 384, 256, n->p3.y, 128, 0);
     conv_fwd(n, n->bota, n->p3, 0, n->b1, 0, true);
     conv_fwd(n, n->botb, n->b1, 0, n->b2, 0, true);
-    hipLaunchKernelGGL(k_up_fwd, dim3(gblocks(M / 16 * 256)), dim3(256), 0, n->stream, B, n->H / 8, n->W / 8, 256,
+    hipLaunchKernelGGL(k_up_fwd, dim3(gblocks(M / 16 * 32)), dim3(256), 0, n->stream, B, n->H / 8, n->W / 8, 256,
                        (const uint16_t *)n->b2.y, 256, 0, n->cat3.y, 384, 0);
     conv_fwd(n, n->dec3a, n->cat3, 0, n->d3a, 0, true);
     conv_fwd(n, n->dec3b, n->d3a, 0, n->d3b, 0, true);
-    hipLaunchKernelGGL(k_up_fwd, dim3(gblocks(M / 4 * 128)), dim3(256), 0, n->stream, B, n->H / 4, n->W / 4, 128,
+    hipLaunchKernelGGL(k_up_fwd, dim3(gblocks(M / 4 * 16)), dim3(256), 0, n->stream, B, n->H / 4, n->W / 4, 128,
                        (const uint16_t *)n->d3b.y, 128, 0, n->cat2.y, 192, 0);
     conv_fwd(n, n->dec2a, n->cat2, 0, n->d2a, 0, true);
     conv_fwd(n, n->dec2b, n->d2a, 0, n->d2b, 0, true);
-    hipLaunchKernelGGL(k_up_fwd, dim3(gblocks(M * 64)), dim3(256), 0, n->stream, B, n->H / 2, n->W / 2, 64,
+    hipLaunchKernelGGL(k_up_fwd, dim3(gblocks(M * 8)), dim3(256), 0, n->stream, B, n->H / 2, n->W / 2, 64,
                        (const uint16_t *)n->d2b.y, 64, 0, n->cat1.y, 96, 0);
     conv_fwd(n, n->dec1a, n->cat1, 0, n->d1a, 0, true);
     conv_fwd(n, n->dec1b, n->d1a, 0, n->d1b, 0, true);
@@ -390,31 +406,31 @@ static void backward(mcl_net *n)
     hipLaunchKernelGGL(k_head_bwd, dim3(std::min(1024, (M + 255) / 256)), dim3(256), 0, n->stream, M,
                        (const uint16_t *)n->d1b.y, 32, (const float *)n->wh, (const float *)n->y,
                        (const float *)n->tgt, scale, n->d1b.g, n->dwh, n->dbh, n->loss);
-    conv_bwd(n, n->dec1b, n->d1a, 0, n->d1b, 0, true, false);
-    conv_bwd(n, n->dec1a, n->cat1, 0, n->d1a, 0, true, false);
-    hipLaunchKernelGGL(k_up_bwd, dim3(gblocks((size_t)M / 4 * 64)), dim3(256), 0, n->stream, B, n->H / 2, n->W / 2, 64,
+    conv_bwd(n, n->dec1b, n->d1a, 0, n->d1b, 0, true, true);
+    conv_bwd(n, n->dec1a, n->cat1, 0, n->d1a, 0, true, true);
+    hipLaunchKernelGGL(k_up_bwd, dim3(gblocks((size_t)M / 4 * 8)), dim3(256), 0, n->stream, B, n->H / 2, n->W / 2, 64,
                        (const uint16_t *)n->cat1.g, 96, 0, n->d2b.g, 64, 0);
-    conv_bwd(n, n->dec2b, n->d2a, 0, n->d2b, 0, true, false);
-    conv_bwd(n, n->dec2a, n->cat2, 0, n->d2a, 0, true, false);
-    hipLaunchKernelGGL(k_up_bwd, dim3(gblocks((size_t)M / 16 * 128)), dim3(256), 0, n->stream, B, n->H / 4, n->W / 4,
+    conv_bwd(n, n->dec2b, n->d2a, 0, n->d2b, 0, true, true);
+    conv_bwd(n, n->dec2a, n->cat2, 0, n->d2a, 0, true, true);
+    hipLaunchKernelGGL(k_up_bwd, dim3(gblocks((size_t)M / 16 * 16)), dim3(256), 0, n->stream, B, n->H / 4, n->W / 4,
                        128, (const uint16_t *)n->cat2.g, 192, 0, n->d3b.g, 128, 0);
-    conv_bwd(n, n->dec3b, n->d3a, 0, n->d3b, 0, true, false);
-    conv_bwd(n, n->dec3a, n->cat3, 0, n->d3a, 0, true, false);
-    hipLaunchKernelGGL(k_up_bwd, dim3(gblocks((size_t)M / 64 * 256)), dim3(256), 0, n->stream, B, n->H / 8, n->W / 8,
+    conv_bwd(n, n->dec3b, n->d3a, 0, n->d3b, 0, true, true);
+    conv_bwd(n, n->dec3a, n->cat3, 0, n->d3a, 0, true, true);
+    hipLaunchKernelGGL(k_up_bwd, dim3(gblocks((size_t)M / 64 * 32)), dim3(256), 0, n->stream, B, n->H / 8, n->W / 8,
                        256, (const uint16_t *)n->cat3.g, 384, 0, n->b2.g, 256, 0);
-    conv_bwd(n, n->botb, n->b1, 0, n->b2, 0, true, false);
+    conv_bwd(n, n->botb, n->b1, 0, n->b2, 0, true, true);
     conv_bwd(n, n->bota, n->p3, 0, n->b1, 0, true, false);
-    hipLaunchKernelGGL(k_pool_bwd, dim3(gblocks((size_t)M / 16 * 128)), dim3(256), 0, n->stream, B, n->H / 4, n->W / 4,
-                       128, (const uint16_t *)n->p3.g, 128, 0, n->cat3.g, 384, 256, 1);
-    conv_bwd(n, n->enc3b, n->e3a, 0, n->cat3, 256, true, false);
+    hipLaunchKernelGGL(k_pool_bwd, dim3(gblocks((size_t)M / 16 * 16)), dim3(256), 0, n->stream, B, n->H / 4, n->W / 4,
+                       128, (const uint16_t *)n->p3.g, 128, 0, (const uint16_t *)n->cat3.y, n->cat3.g, 384, 256);
+    conv_bwd(n, n->enc3b, n->e3a, 0, n->cat3, 256, true, true);
     conv_bwd(n, n->enc3a, n->p2, 0, n->e3a, 0, true, false);
-    hipLaunchKernelGGL(k_pool_bwd, dim3(gblocks((size_t)M / 4 * 64)), dim3(256), 0, n->stream, B, n->H / 2, n->W / 2,
-                       64, (const uint16_t *)n->p2.g, 64, 0, n->cat2.g, 192, 128, 1);
-    conv_bwd(n, n->enc2b, n->e2a, 0, n->cat2, 128, true, false);
+    hipLaunchKernelGGL(k_pool_bwd, dim3(gblocks((size_t)M / 4 * 8)), dim3(256), 0, n->stream, B, n->H / 2, n->W / 2,
+                       64, (const uint16_t *)n->p2.g, 64, 0, (const uint16_t *)n->cat2.y, n->cat2.g, 192, 128);
+    conv_bwd(n, n->enc2b, n->e2a, 0, n->cat2, 128, true, true);
     conv_bwd(n, n->enc2a, n->p1, 0, n->e2a, 0, true, false);
-    hipLaunchKernelGGL(k_pool_bwd, dim3(gblocks((size_t)M * 32)), dim3(256), 0, n->stream, B, n->H, n->W, 32,
-                       (const uint16_t *)n->p1.g, 32, 0, n->cat1.g, 96, 64, 1);
-    conv_bwd(n, n->enc1b, n->e1a, 0, n->cat1, 64, true, false);
+    hipLaunchKernelGGL(k_pool_bwd, dim3(gblocks((size_t)M * 4)), dim3(256), 0, n->stream, B, n->H, n->W, 32,
+                       (const uint16_t *)n->p1.g, 32, 0, (const uint16_t *)n->cat1.y, n->cat1.g, 96, 64);
+    conv_bwd(n, n->enc1b, n->e1a, 0, n->cat1, 64, true, true);
     conv_bwd(n, n->enc1a, n->x0, 0, n->e1a, 0, false, false);
 }
 
