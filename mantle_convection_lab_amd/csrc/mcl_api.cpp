@@ -581,7 +581,27 @@ static int build_level(mcl_ctx *c, const mcl_mesh_view &v, Level &Lv)
     rc |= dev_upload(c, o, &D.elev, elev);
     rc |= dev_upload(c, o, &D.lm, lm);
     rc |= dev_upload(c, o, &D.gt_row, gt_row);
-    rc |= dev_upload(c, o, &D.gt_p, gt_p);
+    {
+        // the entries of G by element row and by velocity row (gtab of the
+        // element's quadtree level)
+        std::vector<double> gt_val(8 * (size_t)nel, 0.0), g_val(4 * (size_t)std::max(neq, 1), 0.0);
+        std::vector<int> g_el(4 * (size_t)std::max(neq, 1), -1);
+        for (int e = 0; e < nel; e++)
+            for (int t = 0; t < 8; t++)
+                if (gt_row[t * (size_t)nel + e] >= 0)
+                    gt_val[t * (size_t)nel + e] = gtab[elev[e] * 8 + gt_p[t * (size_t)nel + e]];
+        for (int P = 0; P < neq; P++) {
+            const int nd = veq_node[P];
+            for (int k = 0; k < cnt[nd]; k++) {
+                const int e = p2n_el[k * (size_t)nno + nd], a = p2n_a[k * (size_t)nno + nd];
+                g_el[k * (size_t)neq + P] = e;
+                g_val[k * (size_t)neq + P] = gtab[elev[e] * 8 + 2 * a + veq_dof[P]];
+            }
+        }
+        rc |= dev_upload(c, o, &D.gt_val, gt_val);
+        rc |= dev_upload(c, o, &D.g_el, g_el);
+        rc |= dev_upload(c, o, &D.g_val, g_val);
+    }
     rc |= dev_upload(c, o, &D.node, nodev);
     rc |= dev_upload(c, o, &D.p2n_cnt, cnt);
     rc |= dev_upload(c, o, &D.p2n_el, p2n_el);

@@ -667,18 +667,7 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
         win = row_window(row, K.col, K.ncol, K.val, K.width, neq, buf);
         if (gtid < neq) diag = K.diag[gtid];
     }
-    // Preconditioner data, Solver.c:54-64: BAB[e] = sum_i G_ie^2 / Kdiag_i
-    for (int e = gtid; e < nel; e += gsize) {
-        double s = 0.0;
-        int lev = L.elev[e];
-        for (int t = 0; t < 8; t++) {
-            int r = L.gt_row[t * nel + e];
-            if (r < 0) break;
-            double g = L.gtab[lev * 8 + L.gt_p[t * nel + e]];
-            s += g * g / L.Kdiag[r];
-        }
-        P.BAB[e] = s;
-    }
+    for (int e = gtid; e < nel; e += gsize) P.BAB[e] = bab_elem(L, e);
     double *r0 = P.r0, *r1 = P.r1, *r2 = P.r2, *z0 = P.z0, *z1 = P.z1, *s1 = P.s1, *s2 = P.s2;
     double dv = 1.0, dp = 1.0, r1z1 = 0.0, r0z0 = 0.0;
     int cycle = 0;

@@ -19,7 +19,9 @@ struct LevelDev {
     const int *elev;                 // [nel] element quadtree level
     const int *lm;                   // [8][nel] velocity eq of (dof d, corner a) at (d*4+a)
     const int *gt_row;               // [8][nel] free velocity rows of the element, ascending, -1 padded
-    const signed char *gt_p;         // [8][nel] element dof index 2a+d of gt_row
+    const double *gt_val;            // [8][nel] G of (gt_row, element)
+    const int *g_el;                 // [4][neq] elements of the row's node, ascending, -1 padded
+    const double *g_val;             // [4][neq] G of (row, g_el)
     // nodes
     const int *node;                 // [nno] global node id
     const int *p2n_cnt;              // [nno] number of elements at the node

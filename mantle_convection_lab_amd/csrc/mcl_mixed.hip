@@ -83,14 +83,7 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_al_weights(const AlLevel *__restr
     const LevelDev &L = A.L;
     const int e = ((int)blockIdx.x - A.eblk0) * MCL_BLOCK + (int)threadIdx.x;
     if (e >= L.nel) return;
-    double s = 0.0;
-    const int lev = L.elev[e];
-    for (int t = 0; t < 8; t++) {
-        const int r = L.gt_row[t * L.nel + e];
-        if (r < 0) break;
-        const double g = L.gtab[lev * 8 + L.gt_p[t * L.nel + e]];
-        s += g * g / L.Kdiag[r];
-    }
+    const double s = bab_elem(L, e);
     A.w[e] = s > 0.0 ? 1.0 / s : 0.0;
 }
 
@@ -421,7 +414,20 @@ __device__ __forceinline__ float ell32c(int WK, int n, CP col, VP val, int i, XP
 #pragma unroll
         for (int u = 0; u < 9; u++) s += v[u] * g[u];
     }
-    for (; k < WK; k++) s += val[k * n + i] * vld<CO>(x + col[k * n + i]);
+    if (k < WK) {
+        int c[8];
+        float v[8], g[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            c[u] = k + u < WK ? (int)col[(k + u) * n + i] : -1;
+            v[u] = k + u < WK ? val[(k + u) * n + i] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) g[u] = c[u] >= 0 ? vld<CO>(x + c[u]) : 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (k + u < WK) s += v[u] * g[u];
+    }
     return s;
 }
 
@@ -618,7 +624,20 @@ __device__ __forceinline__ float ell32_map(const GLevel &F, MP map, int nloc, in
 #pragma unroll
         for (int u = 0; u < 9; u++) s += v[u] * g[u];
     }
-    for (; k < F.WK; k++) s += F.val[k * F.n + row] * x[map[k * nloc + t]];
+    if (k < F.WK) {
+        int c[8];
+        float v[8], g[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            c[u] = k + u < F.WK ? (int)map[(k + u) * nloc + t] : -1;
+            v[u] = k + u < F.WK ? F.val[(k + u) * F.n + row] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) g[u] = c[u] >= 0 ? x[c[u]] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (k + u < F.WK) s += v[u] * g[u];
+    }
     return s;
 }
 
@@ -1199,18 +1218,18 @@ __device__ __forceinline__ double c_expand(const LevelDev &L, int j, F v)
 {
     const int np = L.hp_n[j];
     if (np == 0) return v(j);
-    double s = 0.0;
-    for (int k = 0; k < np; k++) s += L.hp_w[k * L.neq + j] * v(L.hp_i[k * L.neq + j]);
-    return s;
-}
-
-// row i of K (C v)
-template <typename F>
-__device__ __forceinline__ double k_row_c(const LevelDev &L, int i, F v)
-{
-    const int nc = L.Kncol[i], n = L.neq;
-    double s = 0.0;
-    for (int k = 0; k < nc; k++) s += L.Kval[k * n + i] * c_expand(L, L.Kcol[k * n + i], v);
+    int p[4];
+    double w[4], x[4], s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        p[k] = k < np ? L.hp_i[k * L.neq + j] : -1;
+        w[k] = k < np ? L.hp_w[k * L.neq + j] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = p[k] >= 0 ? v(p[k]) : 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if (p[k] >= 0) s += w[k] * x[k];
     return s;
 }
 
@@ -1312,21 +1331,34 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
         {
             dd acc[1] = {dd_zero()};
             if (L.nh > 0) {
-                // q = C^T K C d', d' = z + beta d (zero on hanging equations)
+                // q = C^T K C d', d' = z + beta d (zero on hanging equations),
+                // in three phases: v = C d', y = K v, q = C^T y.  (In one, every
+                // row expanded every column and every parent repeated its
+                // children's rows, one dependent load after another: 48 us an
+                // iteration at 11 662 equations, 14 us so.)
                 auto dv = [&](int j) {
                     double v = (double)vld<kCO>(zf + j);
                     if (!first) v += beta * vldd<kCO>(dold + j);
                     return v;
                 };
+                double *cv = P.U.cg_r, *ky = P.U.xt2;
                 for (int i = ex.b; i < ex.e; i += ex.s) {
-                    double qi = 0.0, di = 0.0;
-                    if (L.hp_n[i] == 0) {
-                        di = dv(i);
-                        qi = ct_gather(L, i, k_row_c(L, i, dv), [&](int h) { return k_row_c(L, h, dv); });
-                    }
+                    const bool hang = L.hp_n[i] != 0;
+                    const double di = hang ? 0.0 : dv(i);
+                    ast(cv + i, hang ? c_expand(L, i, dv) : di);
                     vstd<kCO>(dnew + i, di);
+                }
+                ok = ok && grid_wait(gs, ws);
+                for (int i = ex.b; i < ex.e; i += ex.s)
+                    ast(ky + i, ell_row_ld(L.Kcol, L.Kval, L.Kncol[i], n, i, [&](int j) { return ald(cv + j); }));
+                ok = ok && grid_wait(gs, ws);
+                for (int i = ex.b; i < ex.e; i += ex.s) {
+                    double qi = 0.0;
+                    if (L.hp_n[i] == 0) {
+                        qi = ct_gather(L, i, ald(ky + i), [&](int h) { return ald(ky + h); });
+                        acc[0] = dd_add_prod(acc[0], vldd<kCO>(dnew + i), qi);
+                    }
                     q[i] = qi;
-                    acc[0] = dd_add_prod(acc[0], di, qi);
                 }
             } else
             for (int i = ex.b; i < ex.e; i += ex.s) {
@@ -1485,17 +1517,7 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
         mcl_ph[MCL_PHASES] = (long long)wall_clock64();
     }
 #endif
-    for (int e = gtid; e < nel; e += gsize) {
-        double s = 0.0;
-        int lev = L.elev[e];
-        for (int t = 0; t < 8; t++) {
-            int r = L.gt_row[t * nel + e];
-            if (r < 0) break;
-            double g = L.gtab[lev * 8 + L.gt_p[t * nel + e]];
-            s += g * g / L.Kdiag[r];
-        }
-        U.BAB[e] = s;
-    }
+    for (int e = gtid; e < nel; e += gsize) U.BAB[e] = bab_elem(L, e);
     // One inner solve call site for all three kinds of inner solve (the
     // kernel then holds one copy of the inner solve and its V-cycle):
     //   stage 0: the first solve, for the momentum defect of the initial guess;
@@ -1542,8 +1564,25 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
                 vstd<kCO>(gp(s2) + e, cycle == 0 ? z : z + delta * vldd<kCO>(gp(s1) + e));
             }
             for (int i = rows.b; i < rows.e; i += rows.s) {
-                double a = g_row_ld(L, i, [&](int e) { return vldd<kCO>(gp(z1) + e); });
-                if (cycle > 0) a += delta * g_row_ld(L, i, [&](int e) { return vldd<kCO>(gp(s1) + e); });
+                int e[4];
+                double v[4], z[4], sv[4], a = 0.0, b = 0.0;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    e[k] = L.g_el[k * neq + i];
+                    v[k] = L.g_val[k * neq + i];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    z[k] = e[k] >= 0 ? vldd<kCO>(gp(z1) + e[k]) : 0.0;
+                    sv[k] = e[k] >= 0 && cycle > 0 ? vldd<kCO>(gp(s1) + e[k]) : 0.0;
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (e[k] >= 0) {
+                        a += v[k] * z[k];
+                        b += v[k] * sv[k];
+                    }
+                if (cycle > 0) a += delta * b;
                 U.Ahv[i] = a;
             }
             // relaxed inner accuracy (P.relax > 0): the update this solve

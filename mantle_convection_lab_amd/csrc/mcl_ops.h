@@ -41,7 +41,22 @@ __device__ __forceinline__ double ell_row_ld(const int *__restrict__ col, const 
 #pragma unroll
         for (int u = 0; u < 9; u++) s += v[u] * x[u];
     }
-    for (; j < ncol; j++) s += val[j * n + row] * load(col[j * n + row]);
+    if (j < ncol) {
+        // the rest (a boundary row's, or of a longer row) in one round trip too
+        int c[8];
+        double v[8], x[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const bool in = j + u < ncol;
+            c[u] = in ? col[(j + u) * n + row] : -1;
+            v[u] = in ? val[(j + u) * n + row] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) x[u] = c[u] >= 0 ? load(c[u]) : 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (c[u] >= 0) s += v[u] * x[u];
+    }
     return s;
 }
 
@@ -142,17 +157,29 @@ __device__ __forceinline__ Window row_window(RowReg<W> &r, const int *__restrict
     return w;
 }
 
-// (G p)[P], G_prod_p (Solver.c:569-591): columns are the row's elements, ascending.
-// (G p) for velocity row P with the element values read through load(e)
+// G and G^T are applied from tables of a row's elements (an element's rows) and
+// the entries: the index and the entry come in one round trip, the vector in a
+// second.  (Through node, adjacency, element level and gradient table it took
+// five: an Uzawa iteration's own phases at 32x32 17 us, 14 so; 27 and 22 at
+// 256x256.)
+
+// (G p)[P], G_prod_p (Solver.c:569-591): the row's elements ascending, their
+// values read through load(e)
 template <typename LD>
 __device__ __forceinline__ double g_row_ld(const LevelDev &L, int P, LD load)
 {
-    int n = L.veq_node[P], ip = L.veq_dof[P];
-    double s = 0.0;
-    for (int k = 0; k < L.p2n_cnt[n]; k++) {
-        int e = L.p2n_el[k * L.nno + n], a = L.p2n_a[k * L.nno + n];
-        s += L.gtab[L.elev[e] * 8 + 2 * a + ip] * load(e);
+    int e[4];
+    double v[4], x[4], s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        e[k] = L.g_el[k * L.neq + P];
+        v[k] = L.g_val[k * L.neq + P];
     }
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = e[k] >= 0 ? load(e[k]) : 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if (e[k] >= 0) s += v[k] * x[k];
     return s;
 }
 
@@ -166,19 +193,37 @@ __device__ __forceinline__ double g_row(const LevelDev &L, int P, const double *
 template <typename LD>
 __device__ __forceinline__ double gt_elem_ld(const LevelDev &L, int e, LD load)
 {
-    double s = 0.0;
-    int lev = L.elev[e];
+    int r[8];
+    double v[8], x[8], s = 0.0;
+#pragma unroll
     for (int t = 0; t < 8; t++) {
-        int r = L.gt_row[t * L.nel + e];
-        if (r < 0) break;
-        s += L.gtab[lev * 8 + L.gt_p[t * L.nel + e]] * load(r);
+        r[t] = L.gt_row[t * L.nel + e];
+        v[t] = L.gt_val[t * L.nel + e];
     }
+#pragma unroll
+    for (int t = 0; t < 8; t++) x[t] = r[t] >= 0 ? load(r[t]) : 0.0;
+#pragma unroll
+    for (int t = 0; t < 8; t++)
+        if (r[t] >= 0) s += v[t] * x[t];
     return s;
 }
 
 __device__ __forceinline__ double gt_elem(const LevelDev &L, int e, const double *__restrict__ x)
 {
     return gt_elem_ld(L, e, [&](int r) { return x[r]; });
+}
+
+// Preconditioner data, Solver.c:54-64: BAB_e = sum_i G_ie^2 / Kdiag_i
+__device__ __forceinline__ double bab_elem(const LevelDev &L, int e)
+{
+    double s = 0.0;
+    for (int t = 0; t < 8; t++) {
+        const int r = L.gt_row[t * L.nel + e];
+        if (r < 0) break;
+        const double g = L.gt_val[t * L.nel + e];
+        s += g * g / L.Kdiag[r];
+    }
+    return s;
 }
 
 // ------------------------------------------------------------ persistent Uzawa
