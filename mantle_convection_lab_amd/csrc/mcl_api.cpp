@@ -737,7 +737,7 @@ static int build_multigrid(mcl_ctx *c)
         std::vector<void *> &o = Lv.owned;
         int n = std::max(Lv.neq, 1);
         int rc = 0;
-        rc |= dev_alloc(c, o, &Lv.val32, (size_t)std::max(Lv.WK, 1) * n);
+        rc |= dev_alloc(c, o, &Lv.val32, 2 * (size_t)((std::max(Lv.WK, 1) + 1) / 2) * n);
         rc |= dev_alloc(c, o, &Lv.dinv32, n);
         rc |= dev_alloc(c, o, &Lv.mx, n);
         rc |= dev_alloc(c, o, &Lv.mb, n);
@@ -749,12 +749,18 @@ static int build_multigrid(mcl_ctx *c)
         M.WK = Lv.WK;
         M.block = 0;
         M.lds_off = 0;
-        M.col = Lv.dev.Kcol;
-        M.ncol = Lv.dev.Kncol;
+        {
+            const int w2 = (Lv.WK + 1) / 2;
+            std::vector<int> col2(2 * (size_t)std::max(w2, 1) * n, 0);
+            for (int s = 0; s < 2 * w2; s++)
+                for (int i = 0; i < Lv.neq; i++)
+                    col2[2 * ((size_t)(s >> 1) * Lv.neq + i) + (s & 1)] =
+                        s < Lv.WK ? Lv.Kcol_h[(size_t)s * Lv.neq + i] : i;
+            if (dev_upload(c, o, &M.col, col2)) return MCL_E_DEVICE;
+            M.WK2 = w2;
+        }
         M.val = Lv.val32;
         M.dinv = Lv.dinv32;
-        M.val64 = Lv.dev.Kval;
-        M.diag64 = Lv.dev.Kdiag;
         M.x = Lv.mx;
         M.b = Lv.mb;
         M.r = Lv.mr;
@@ -779,12 +785,15 @@ static int build_multigrid(mcl_ctx *c)
         int off = 0, nnz = 0;
         for (int k = 0; k < nlev - 1; k++) {
             Level &Lv = c->levels[k];
-            const int n = Lv.neq, m = Lv.WK * n;
+            const int n = Lv.neq, w2 = mg[k].WK2, m = 2 * w2 * n;
             if (k > 0 && n > block_rows_threshold()) break;
             if (off / 3 + n > MCL_MG_LDS_ROWS || nnz + m > MCL_MG_LDS_NNZ || n > 65535) break;
-            std::vector<unsigned short> col16(std::max(m, 1), 0);
-            for (int e = 0; e < m; e++) col16[e] = (unsigned short)Lv.Kcol_h[e];
-            const unsigned short *cp;
+            std::vector<unsigned> col16((size_t)std::max(w2 * n, 1), 0);
+            for (int s = 0; s < 2 * w2; s++)
+                for (int i = 0; i < n; i++)
+                    col16[(size_t)(s >> 1) * n + i] |=
+                        (unsigned)(s < Lv.WK ? Lv.Kcol_h[(size_t)s * n + i] : i) << (16 * (s & 1));
+            const unsigned *cp;
             if (dev_upload(c, Lv.owned, &cp, col16)) return MCL_E_DEVICE;
             mg[k].col16 = cp;
             mg[k].block = 1;
@@ -1632,7 +1641,7 @@ static int build_halos(mcl_ctx *c, int nb, Add &add)
         MgLevelDev &M = mg[l];
         Level &A = c->levels[l];
         Level &C = c->levels[l - 1];
-        const int n = A.neq, WK = A.WK, nc = C.neq, rw = C.rw;
+        const int n = A.neq, WK = A.WK, W2 = (WK + 1) / 2, nc = C.neq, rw = C.rw;
         if (n == 0) continue;
         const int R = (n + nb - 1) / nb, Rc = (nc + nb - 1) / nb;
         const bool coarse_grid = l - 1 > lb;
@@ -1645,9 +1654,14 @@ static int build_halos(mcl_ctx *c, int nb, Add &add)
             }
         };
         std::vector<int> h1_ptr(nb + 1, 0), h1_row, h2_ptr(nb + 1, 0), h2_row;
-        std::vector<unsigned short> kl((size_t)WK * n, 0), hm;
+        // pairs of slots packed into a word (16 bits an index: the lists hold at
+        // most MCL_HALO_LDS rows); slot WK of an odd length is the row itself
+        std::vector<unsigned> kl((size_t)W2 * n, 0), hm;
+        auto put = [](std::vector<unsigned> &v, size_t at, int s, int q) {
+            v[at] |= (unsigned)std::min(std::max(q, 0), 65535) << (16 * (s & 1));
+        };
         std::vector<int> f_ptr(nb + 1, 0), f_row, th_ptr(nb + 1, 0), th_row, uh_ptr(nb + 1, 0), uh_row;
-        std::vector<unsigned short> mt, mf;
+        std::vector<unsigned> mt, mf;
         std::vector<short> rl((size_t)std::max(rw, 1) * std::max(nc, 1), -1);
         bool up1 = true, up2 = fuse_level >= 2, dn1 = coarse_grid && (int)C.rcol_h.size() == rw * nc && nc > 0;
         bool dn2 = dn1 && fuse_level >= 2;
@@ -1680,18 +1694,20 @@ static int build_halos(mcl_ctx *c, int nb, Add &add)
                 const int p2 = pos(H2, j);
                 return p2 >= 0 ? R + (int)H1.size() + p2 : -1;
             };
-            for (int s = 0; s < WK; s++)
+            for (int s = 0; s < 2 * W2; s++)
                 for (int i = b0; i < e0; i++) {
-                    const int q = locV(kcol(i, s));
+                    const int q = locV(s < WK ? kcol(i, s) : i);
                     if (q < 0 || q >= nW) up1 = up2 = false;
-                    kl[(size_t)s * n + i] = (unsigned short)std::max(q, 0);
+                    put(kl, (size_t)(s >> 1) * n + i, s, q);
                 }
-            // hm: H1 rows -> V, slot-major within the workgroup's block
-            for (int s = 0; s < WK; s++)
-                for (int j : H1) {
-                    const int q = locV(kcol(j, s));
+            // hm: H1 rows -> V, pair-major within the workgroup's block
+            const size_t hm0 = hm.size();
+            hm.resize(hm0 + (size_t)W2 * H1.size(), 0);
+            for (int s = 0; s < 2 * W2; s++)
+                for (size_t t = 0; t < H1.size(); t++) {
+                    const int q = locV(s < WK ? kcol(H1[t], s) : H1[t]);
                     if (q < 0 || q >= nV) up2 = false;
-                    hm.push_back((unsigned short)std::max(q, 0));
+                    put(hm, hm0 + (size_t)(s >> 1) * H1.size() + t, s, q);
                 }
             h1_row.insert(h1_row.end(), H1.begin(), H1.end());
             h1_ptr[g + 1] = (int)h1_row.size();
@@ -1752,26 +1768,24 @@ static int build_halos(mcl_ctx *c, int nb, Add &add)
                 const int pu = pos(Uh, j);
                 return pu >= 0 ? R + (int)Th.size() + pu : -1;
             };
-            // mt: T rows (O padded to R, then Th) -> U, slot-major in the block
-            for (int s = 0; s < WK; s++) {
-                for (int t = 0; t < R; t++) {
-                    const int i = b0 + t;
-                    const int q = i < e0 ? locU(kcol(i, s)) : 0;
+            // mt: T rows (O padded to R, then Th) -> U, pair-major in the block
+            const size_t mt0 = mt.size();
+            mt.resize(mt0 + (size_t)W2 * nT, 0);
+            for (int s = 0; s < 2 * W2; s++)
+                for (long long t = 0; t < nT; t++) {
+                    const int i = t < R ? b0 + (int)t : Th[t - R];
+                    const int q = t < R && i >= e0 ? 0 : locU(s < WK ? kcol(i, s) : i);
                     if (q < 0 || q >= nU) dn2 = false;
-                    mt.push_back((unsigned short)std::max(q, 0));
+                    put(mt, mt0 + (size_t)(s >> 1) * nT + t, s, q);
                 }
-                for (int j : Th) {
-                    const int q = locU(kcol(j, s));
-                    if (q < 0 || q >= nU) dn2 = false;
-                    mt.push_back((unsigned short)std::max(q, 0));
-                }
-            }
             // mf: F rows -> T (K columns of F lie in T by construction)
-            for (int s = 0; s < WK; s++)
-                for (int u : F) {
-                    const int q = locU(kcol(u, s));
+            const size_t mf0 = mf.size();
+            mf.resize(mf0 + (size_t)W2 * F.size(), 0);
+            for (int s = 0; s < 2 * W2; s++)
+                for (size_t t = 0; t < F.size(); t++) {
+                    const int q = locU(s < WK ? kcol(F[t], s) : F[t]);
                     if (q < 0 || q >= nT) dn2 = false;
-                    mf.push_back((unsigned short)std::max(q, 0));
+                    put(mf, mf0 + (size_t)(s >> 1) * F.size() + t, s, q);
                 }
             f_row.insert(f_row.end(), F.begin(), F.end());
             f_ptr[g + 1] = (int)f_row.size();

@@ -154,13 +154,17 @@ struct MgLevelDev {
     int block;               // coarse level run per workgroup from LDS
     int lds_off;             // offset of its vectors in the LDS block (floats)
     int moff;                // offset of its matrix in the LDS matrix block (entries)
-    const unsigned short *col16;  // [WK][n] col as 16-bit indices (LDS levels)
-    const int *col;          // [WK][n] (the level's FP64 ELL pattern)
-    const int *ncol;         // [n]
-    float *val;              // [WK][n] FP32 copy of the level's K
+    // The FP32 matrix and every column map hold two slots of a row together
+    // (WK2 = (WK + 1) / 2 pairs, [pair][row]; an odd row length is padded with
+    // the row itself and 0): half the loads of one slot each, and their address
+    // registers (28 spilled registers before, 10 so; a solve at 32x32 3.81 ms
+    // before, 3.72).  Maps into lists of at most 65 535 rows pack a pair into
+    // one word.
+    int WK2;
+    const unsigned *col16;   // [WK2][n] (LDS levels)
+    const int *col;          // [WK2][n][2]
+    float *val;              // [WK2][n][2]
     float *dinv;             // [n] 1 / diag(K)
-    const double *val64;     // [WK][n] the FP64 K of the level
-    const double *diag64;    // [n]
     // prolongation from level-1: fine row u <- mean of pn[u] coarse rows pcol[k][u] (-1 = fixed)
     const int *pn;           // [n]
     const int *pcol;         // [4][n]
@@ -183,18 +187,25 @@ struct MgLevelDev {
     //      the residual on O).
     int fuse_up, fuse_down, deep_up, deep_down;
     const int *hu_ptr, *hu_row;        // [nb + 1], H1
-    const unsigned short *kl;          // [WK][n] K columns of O as local indices (into W, V)
+    const unsigned *kl;                // [WK2][n] K columns of O as local indices (into W, V)
     const int *h2_ptr, *h2_row;        // [nb + 1], H2
-    const unsigned short *hm;          // H1 rows' K columns -> V, block hu_ptr[g] WK, slot-major
+    const unsigned *hm;                // H1 rows' K columns -> V, block hu_ptr[g] WK2, pair-major
     const int *hd_ptr, *hd_row;        // [nb + 1], F
     const short *rl;                   // [rw][n] (coarse level) restriction columns as indices into F
     const int *th_ptr, *th_row;        // [nb + 1], Th
     const int *uh_ptr, *uh_row;        // [nb + 1], Uh
-    const unsigned short *mt;          // T rows' K columns -> U, block (g R + th_ptr[g]) WK, slot-major
-    const unsigned short *mf;          // F rows' K columns -> T, block hd_ptr[g] WK, slot-major
+    const unsigned *mt;                // T rows' K columns -> U, block (g R + th_ptr[g]) WK2, pair-major
+    const unsigned *mf;                // F rows' K columns -> T, block hd_ptr[g] WK2, pair-major
 };
 
-// floats of the LDS buffer of the fused V-cycle phases (per workgroup)
+// Rows of a workgroup's halo lists kept in LDS (16-bit row numbers).
+#ifndef MCL_LDS_LIST
+#define MCL_LDS_LIST 4608
+#endif
+// floats of the LDS buffer of the fused V-cycle phases (per workgroup).  The
+// phases repeat their halo's row products, so more is not better: with 6144 the
+// two-sweep form reaches the finest level of 256x256 and the one-sweep forms
+// that of 512x512 (32.3 and 71.6 ms a solve; 30.4 and 67.5 so).
 #ifndef MCL_HALO_LDS
 #define MCL_HALO_LDS 4096
 #endif
@@ -274,7 +285,7 @@ __global__ void k_uzawa_probe(MixedParams P);
 struct PrepLevel {
     int n, W;
     const double *val, *diag;
-    float *val32, *dinv;
+    float *val32, *dinv;         // val32: [(W + 1) / 2][n][2]
     unsigned *bound;
     int blk0;
 };

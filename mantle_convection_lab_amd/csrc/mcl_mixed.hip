@@ -13,6 +13,8 @@
 #include "mcl_kernels.h"
 #include "mcl_ops.h"
 
+typedef float f2v __attribute__((ext_vector_type(2)));
+
 // Optional phase timers (build with -DMCL_PHASE_TIMERS=1): thread 0 of
 // workgroup 0 charges the 100 MHz wall clock since its previous stamp to a
 // phase; grid barriers keep every workgroup in step, so workgroup 0's split
@@ -51,10 +53,11 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_prepare_fp32(const PrepLevel *__r
     float m = 0.f;
     if (i < A.n) {
         double s = 0.0;
-        for (int k = 0; k < A.W; k++) {
-            const double v = A.val[k * A.n + i];
-            A.val32[k * A.n + i] = (float)v;
-            s += fabs(v);
+        for (int k = 0; k < A.W; k += 2) {
+            const double v0 = A.val[k * A.n + i], v1 = k + 1 < A.W ? A.val[(k + 1) * A.n + i] : 0.0;
+            ((f2v *)A.val32)[(k >> 1) * A.n + i] = f2v{(float)v0, (float)v1};
+            s += fabs(v0);
+            s += fabs(v1);
         }
         const double d = A.diag[i];
         A.dinv[i] = (float)(1.0 / d);
@@ -273,42 +276,52 @@ __device__ __forceinline__ void vstd(Ptr p, double v)
     else *p = v;
 }
 
+// Two slots of a row: their values, and their columns as a pair of integers or
+// packed into one word.
+typedef int i2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ i2v col_pair(i2v c) { return c; }
+__device__ __forceinline__ i2v col_pair(unsigned c) { return i2v{(int)(c & 0xffffu), (int)(c >> 16)}; }
+
+// This workgroup's halo lists of a grid level: where they start and their
+// lengths in the level's arrays, and where their rows lie in MgLds::rows (-1:
+// not there).  Read from memory in every phase, the offsets, the rows and then
+// the rows' data are three dependent round trips; from here one (a solve at
+// 192x64 27.5 ms, 29.1 without; 256x256 30.4, 31.8; hanging nodes at 32x16
+// 55.5, 58.4).
+struct LevelLists {
+    int t0, nth, u0, nuh, f0, nf, h10, nh1, h20, nh2;
+    int pt, pf, ph;   // rows of [Th | Uh], F and [H1 | H2]
+};
+
 // A grid level as the level operations see it.
 struct GLevel {
-    int n, WK, rw;
-    const MCL_G int *col;
-    const MCL_G float *val, *dinv;
+    int n, WK2, rw;
+    const MCL_G i2v *col;
+    const MCL_G f2v *val;
+    const MCL_G float *dinv;
     const MCL_G int *pn, *pcol, *rcol;
     const MCL_G float *rval;
     MCL_G float *x, *b, *r, *t;
     int fuse_up, fuse_down, deep_up, deep_down;
     const MCL_G int *hu_ptr, *hu_row, *hd_ptr, *hd_row, *h2_ptr, *h2_row, *th_ptr, *th_row, *uh_ptr, *uh_row;
-    const MCL_G unsigned short *kl, *hm, *mt, *mf;
+    const MCL_G unsigned *kl, *hm, *mt, *mf;
     const MCL_G short *rl;
+    LevelLists ls;
+    const MCL_L unsigned short *rows;
 };
 
 // A coarse level as seen by one workgroup: vectors x, t, b (3 n floats at
 // lds_off), 1/diag(K) (n floats at lds_off / 3) and the FP32 K with 16-bit
-// columns (WK n entries at moff) in LDS, copied from HBM once per launch; the
+// columns (2 WK2 n entries at moff) in LDS, copied from HBM once per launch; the
 // transfer maps stay in HBM.
 struct LdsLevel {
-    int n, WK, rw;
-    const MCL_L unsigned short *col;
-    const MCL_L float *val, *dinv;
+    int n, WK2, rw;
+    const MCL_L unsigned *col;
+    const MCL_L f2v *val;
+    const MCL_L float *dinv;
     const MCL_G int *pn, *pcol, *rcol;
     const MCL_G float *rval;
     MCL_L float *x, *b, *r, *t;
-};
-
-// the workgroup's LDS blocks: level descriptors, Gershgorin bounds (both read
-// in every phase, so kept out of the grid barriers' cache invalidations), and
-// the coarse levels' vectors and matrices
-struct MgLds {
-    const MCL_L MgLevelDev *lev;
-    const MCL_L float *lam;
-    MCL_L float *vec, *dinv, *val;
-    MCL_L unsigned short *col;
-    MCL_L float *halo;       // [MCL_HALO_LDS] buffer of the fused phases
 };
 
 template <typename LV>
@@ -317,14 +330,29 @@ __device__ __forceinline__ auto sweep_buf(const LV &A, int k)
     return (k & 1) ? A.x : A.t;
 }
 
-__device__ __forceinline__ GLevel glevel(const MCL_L MgLevelDev *G)
+// the workgroup's LDS blocks: level descriptors, Gershgorin bounds (both read
+// in every phase, so kept out of the grid barriers' cache invalidations), and
+// the coarse levels' vectors and matrices
+struct MgLds {
+    const MCL_L MgLevelDev *lev;
+    const MCL_L float *lam;
+    MCL_L float *vec, *dinv;
+    MCL_L f2v *val;
+    MCL_L unsigned *col;
+    MCL_L float *halo;       // [MCL_HALO_LDS] buffer of the fused phases
+    LevelLists *lists;       // LDS
+    MCL_L unsigned short *rows;   // [MCL_LDS_LIST]
+};
+
+__device__ __forceinline__ GLevel glevel(const MgLds &S, int l)
 {
+    const MCL_L MgLevelDev *G = S.lev + l;
     GLevel A;
     A.n = G->n;
-    A.WK = G->WK;
+    A.WK2 = G->WK2;
     A.rw = G->rw;
-    A.col = gp(G->col);
-    A.val = gp(G->val);
+    A.col = (const MCL_G i2v *)G->col;
+    A.val = (const MCL_G f2v *)G->val;
     A.dinv = gp(G->dinv);
     A.pn = gp(G->pn);
     A.pcol = gp(G->pcol);
@@ -353,6 +381,8 @@ __device__ __forceinline__ GLevel glevel(const MCL_L MgLevelDev *G)
     A.mt = gp(G->mt);
     A.mf = gp(G->mf);
     A.rl = gp(G->rl);
+    A.ls = S.lists[l];
+    A.rows = S.rows;
     return A;
 }
 
@@ -362,10 +392,10 @@ __device__ __forceinline__ LdsLevel lds_level(const MgLds &S, int l, int pre)
     const MCL_L MgLevelDev *G = S.lev + l;
     LdsLevel A;
     A.n = G->n;
-    A.WK = G->WK;
+    A.WK2 = G->WK2;
     A.rw = G->rw;
-    A.col = S.col + G->moff;
-    A.val = S.val + G->moff;
+    A.col = S.col + G->moff / 2;
+    A.val = S.val + G->moff / 2;
     A.dinv = S.dinv + G->lds_off / 3;
     A.pn = gp(G->pn);
     A.pcol = gp(G->pcol);
@@ -378,55 +408,74 @@ __device__ __forceinline__ LdsLevel lds_level(const MgLds &S, int l, int pre)
     return A;
 }
 
-// Row i of an FP32 ELL matrix (WK slots, slot-major over n rows, columns col)
-// times x.  Rows of width 18 (the bilinear-quad velocity stencil) issue all
-// their loads at once, other widths nine entries per round trip; the sum keeps
-// the slot order.
+// A row of an FP32 matrix (WK2 pairs of slots, values val[pair * vs + vi],
+// columns col[pair * cs + ci]) times x.  Rows of 9 pairs (the bilinear-quad
+// velocity stencil) issue all their loads at once, others six pairs per round
+// trip; the sum keeps the slot order.
 template <bool CO, typename CP, typename VP, typename XP>
-__device__ __forceinline__ float ell32c(int WK, int n, CP col, VP val, int i, XP x)
+__device__ __forceinline__ float ellp(int WK2, CP col, int cs, int ci, VP val, int vs, int vi, XP x)
 {
     float s = 0.f;
-    if (WK == 18) {
-        int c[18];
-        float v[18], g[18];
+    if (WK2 == 9) {
+        i2v c[9];
+        f2v v[9], g[9];
 #pragma unroll
-        for (int u = 0; u < 18; u++) {
-            c[u] = col[u * n + i];
-            v[u] = val[u * n + i];
+        for (int u = 0; u < 9; u++) {
+            c[u] = col_pair(col[u * cs + ci]);
+            v[u] = val[u * vs + vi];
         }
 #pragma unroll
-        for (int u = 0; u < 18; u++) g[u] = vld<CO>(x + c[u]);
+        for (int u = 0; u < 9; u++) {
+            g[u].x = vld<CO>(x + c[u].x);
+            g[u].y = vld<CO>(x + c[u].y);
+        }
 #pragma unroll
-        for (int u = 0; u < 18; u++) s += v[u] * g[u];
+        for (int u = 0; u < 9; u++) {
+            s += v[u].x * g[u].x;
+            s += v[u].y * g[u].y;
+        }
         return s;
     }
     int k = 0;
-    for (; k + 9 <= WK; k += 9) {
-        int c[9];
-        float v[9], g[9];
+    for (; k + 6 <= WK2; k += 6) {
+        i2v c[6];
+        f2v v[6], g[6];
 #pragma unroll
-        for (int u = 0; u < 9; u++) {
-            c[u] = col[(k + u) * n + i];
-            v[u] = val[(k + u) * n + i];
+        for (int u = 0; u < 6; u++) {
+            c[u] = col_pair(col[(k + u) * cs + ci]);
+            v[u] = val[(k + u) * vs + vi];
         }
 #pragma unroll
-        for (int u = 0; u < 9; u++) g[u] = vld<CO>(x + c[u]);
+        for (int u = 0; u < 6; u++) {
+            g[u].x = vld<CO>(x + c[u].x);
+            g[u].y = vld<CO>(x + c[u].y);
+        }
 #pragma unroll
-        for (int u = 0; u < 9; u++) s += v[u] * g[u];
+        for (int u = 0; u < 6; u++) {
+            s += v[u].x * g[u].x;
+            s += v[u].y * g[u].y;
+        }
     }
-    if (k < WK) {
-        int c[8];
-        float v[8], g[8];
+    if (k < WK2) {
+        i2v c[5];
+        f2v v[5], g[5];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            c[u] = k + u < WK ? (int)col[(k + u) * n + i] : -1;
-            v[u] = k + u < WK ? val[(k + u) * n + i] : 0.f;
+        for (int u = 0; u < 5; u++) {
+            const bool in = k + u < WK2;
+            c[u] = in ? col_pair(col[(k + u) * cs + ci]) : i2v{-1, -1};
+            v[u] = in ? val[(k + u) * vs + vi] : f2v{0.f, 0.f};
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) g[u] = c[u] >= 0 ? vld<CO>(x + c[u]) : 0.f;
+        for (int u = 0; u < 5; u++) {
+            g[u].x = c[u].x >= 0 ? vld<CO>(x + c[u].x) : 0.f;
+            g[u].y = c[u].x >= 0 ? vld<CO>(x + c[u].y) : 0.f;
+        }
 #pragma unroll
-        for (int u = 0; u < 8; u++)
-            if (k + u < WK) s += v[u] * g[u];
+        for (int u = 0; u < 5; u++)
+            if (c[u].x >= 0) {
+                s += v[u].x * g[u].x;
+                s += v[u].y * g[u].y;
+            }
     }
     return s;
 }
@@ -434,7 +483,77 @@ __device__ __forceinline__ float ell32c(int WK, int n, CP col, VP val, int i, XP
 template <bool CO, typename LV, typename XP>
 __device__ __forceinline__ float ell32(const LV &A, int i, XP x)
 {
-    return ell32c<CO>(A.WK, A.n, A.col, A.val, i, x);
+    return ellp<CO>(A.WK2, A.col, A.n, i, A.val, A.n, i, x);
+}
+
+// A workgroup's rows O = [b0, b0 + no) of a grid level (R = own_rows' block).
+struct Own {
+    int R, b0, no;
+};
+
+__device__ __forceinline__ Own own_block(int n)
+{
+    const int R = (n + (int)gridDim.x - 1) / (int)gridDim.x, b0 = (int)blockIdx.x * R;
+    return Own{R, b0, max(0, min(R, n - b0))};
+}
+
+// a row of U = [O | Th | Uh], of F
+__device__ __forceinline__ int urow(const GLevel &F, const Own &o, int t)
+{
+    const LevelLists &l = F.ls;
+    if (t < o.R) return o.b0 + t;
+    if (l.pt >= 0) return F.rows[l.pt + t - o.R];
+    return t < o.R + l.nth ? F.th_row[l.t0 + t - o.R] : F.uh_row[l.u0 + t - o.R - l.nth];
+}
+
+__device__ __forceinline__ int frow(const GLevel &F, int t)
+{
+    return F.ls.pf >= 0 ? F.rows[F.ls.pf + t] : F.hd_row[F.ls.f0 + t];
+}
+
+// a row of V = [O | H1 | H2]
+__device__ __forceinline__ int vrow(const GLevel &F, const Own &o, int t)
+{
+    const LevelLists &l = F.ls;
+    if (t < o.R) return o.b0 + t;
+    if (l.ph >= 0) return F.rows[l.ph + t - o.R];
+    return t < o.R + l.nh1 ? F.hu_row[l.h10 + t - o.R] : F.h2_row[l.h20 + t - o.R - l.nh1];
+}
+
+// The lists of every grid level into LDS: their places, and their rows as far
+// as the space goes, from the coarsest level on (the phases there are the
+// shortest).
+__device__ __forceinline__ void lds_load_lists(const MixedParams &P, const MgLds &S)
+{
+    const int g = blockIdx.x;
+    int used = 0;
+    for (int l = 0; l < P.nmg; l++) {
+        const MCL_L MgLevelDev *G = S.lev + l;
+        LevelLists a = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, -1, -1, -1};
+        const bool deep = P.pre == 2;
+        auto place = [&](const int *ptr, int &first, int &n) {
+            if (!ptr) return;
+            first = gp(ptr)[g];
+            n = gp(ptr)[g + 1] - first;
+        };
+        place(G->th_ptr, a.t0, a.nth);
+        place(G->uh_ptr, a.u0, a.nuh);
+        place(G->hd_ptr, a.f0, a.nf);
+        place(G->hu_ptr, a.h10, a.nh1);
+        place(G->h2_ptr, a.h20, a.nh2);
+        auto keep = [&](int &at, const int *r1, int f1, int n1, const int *r2, int f2, int n2) {
+            if (!r1 || G->n > 65536 || used + n1 + n2 > MCL_LDS_LIST) return;
+            at = used;
+            used += n1 + n2;
+            for (int t = threadIdx.x; t < n1 + n2; t += blockDim.x)
+                S.rows[at + t] = (unsigned short)(t < n1 ? gp(r1)[f1 + t] : gp(r2)[f2 + t - n1]);
+        };
+        if (deep && G->deep_down) keep(a.pt, G->th_row, a.t0, a.nth, G->uh_row, a.u0, a.nuh);
+        keep(a.ph, G->hu_row, a.h10, a.nh1, G->h2_row, a.h20, a.nh2);
+        keep(a.pf, G->hd_row, a.f0, a.nf, nullptr, 0, 0);
+        if (threadIdx.x == 0) S.lists[l] = a;
+    }
+    __syncthreads();
 }
 
 // sweep k >= 2: x_k = x_{k-1} + w D^-1 (b - K x_{k-1})
@@ -540,10 +659,10 @@ __device__ __forceinline__ void restrict_from_lds(const GLevel &C, LB rF, float 
 template <typename LB>
 __device__ __forceinline__ void fused_down(const GLevel &F, const GLevel &C, LB buf, float wc, int pre)
 {
-    const int h0 = F.hd_ptr[blockIdx.x], nh = F.hd_ptr[blockIdx.x + 1] - h0;
+    const int nh = F.ls.nf;
     const auto x = sweep_buf(F, pre);
     for (int t = threadIdx.x; t < nh; t += blockDim.x) {
-        const int u = F.hd_row[h0 + t];
+        const int u = frow(F, t);
         buf[t] = vld<kCO>(F.b + u) - ell32<kCO>(F, u, x);
     }
     __syncthreads();
@@ -558,13 +677,11 @@ __device__ __forceinline__ void fused_down(const GLevel &F, const GLevel &C, LB 
 template <bool CC, typename XC, typename LB>
 __device__ __forceinline__ void fused_up(const GLevel &F, XC xc, LB buf, float w, int pre)
 {
-    const int R = (F.n + (int)gridDim.x - 1) / (int)gridDim.x, b0 = (int)blockIdx.x * R;
-    const int no = max(0, min(R, F.n - b0));
-    const int h0 = F.hu_ptr[blockIdx.x], nh = F.hu_ptr[blockIdx.x + 1] - h0;
+    const Own o = own_block(F.n);
     const auto xin = sweep_buf(F, pre);
-    for (int t = threadIdx.x; t < R + nh; t += blockDim.x) {
-        if (t >= no && t < R) continue;
-        const int u = t < R ? b0 + t : F.hu_row[h0 + t - R];
+    for (int t = threadIdx.x; t < o.R + F.ls.nh1; t += blockDim.x) {
+        if (t >= o.no && t < o.R) continue;
+        const int u = vrow(F, o, t);
         const int m = F.pn[u];
         int lc[4];
         float g[4];
@@ -584,72 +701,18 @@ __device__ __forceinline__ void fused_up(const GLevel &F, XC xc, LB buf, float w
     }
     __syncthreads();
     const auto out = sweep_buf(F, pre + 1);
-    for (int i = b0 + (int)threadIdx.x; i < b0 + no; i += blockDim.x)
+    for (int i = o.b0 + (int)threadIdx.x; i < o.b0 + o.no; i += blockDim.x)
         vst<kCO>(out + i,
-                 buf[i - b0] + w * F.dinv[i] * (vld<kCO>(F.b + i) - ell32c<false>(F.WK, F.n, F.kl, F.val, i, buf)));
+                 buf[i - o.b0] + w * F.dinv[i] * (vld<kCO>(F.b + i) - ellp<false>(F.WK2, F.kl, F.n, i, F.val, F.n, i, buf)));
 }
 
 // Row `row` of F's FP32 K times a vector held in LDS: the columns come from a
-// local map (slot k of local row t at map[k nloc + t]), the values from the
+// local map (pair p of local row t at map[p nloc + t]), the values from the
 // matrix; the sum in slot order, as ell32.
 template <typename MP, typename XP>
 __device__ __forceinline__ float ell32_map(const GLevel &F, MP map, int nloc, int t, int row, XP x)
 {
-    float s = 0.f;
-    if (F.WK == 18) {
-        int c[18];
-        float v[18], g[18];
-#pragma unroll
-        for (int u = 0; u < 18; u++) {
-            c[u] = map[u * nloc + t];
-            v[u] = F.val[u * F.n + row];
-        }
-#pragma unroll
-        for (int u = 0; u < 18; u++) g[u] = x[c[u]];
-#pragma unroll
-        for (int u = 0; u < 18; u++) s += v[u] * g[u];
-        return s;
-    }
-    int k = 0;
-    for (; k + 9 <= F.WK; k += 9) {
-        int c[9];
-        float v[9], g[9];
-#pragma unroll
-        for (int u = 0; u < 9; u++) {
-            c[u] = map[(k + u) * nloc + t];
-            v[u] = F.val[(k + u) * F.n + row];
-        }
-#pragma unroll
-        for (int u = 0; u < 9; u++) g[u] = x[c[u]];
-#pragma unroll
-        for (int u = 0; u < 9; u++) s += v[u] * g[u];
-    }
-    if (k < F.WK) {
-        int c[8];
-        float v[8], g[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            c[u] = k + u < F.WK ? (int)map[(k + u) * nloc + t] : -1;
-            v[u] = k + u < F.WK ? F.val[(k + u) * F.n + row] : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) g[u] = c[u] >= 0 ? x[c[u]] : 0.f;
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-            if (k + u < F.WK) s += v[u] * g[u];
-    }
-    return s;
-}
-
-// A workgroup's rows O = [b0, b0 + no) of a grid level (R = own_rows' block).
-struct Own {
-    int R, b0, no;
-};
-
-__device__ __forceinline__ Own own_block(int n)
-{
-    const int R = (n + (int)gridDim.x - 1) / (int)gridDim.x, b0 = (int)blockIdx.x * R;
-    return Own{R, b0, max(0, min(R, n - b0))};
+    return ellp<false>(F.WK2, map, nloc, t, F.val, F.n, row, x);
 }
 
 // ------------------------------------ one-row-per-thread two-sweep phases
@@ -657,21 +720,21 @@ __device__ __forceinline__ Own own_block(int n)
 // threads, so a thread holds at most one row of each.  These forms issue all
 // loads of a phase that do not wait on another workgroup at its start -- the
 // K rows' local columns and values, 1/diag, right-hand sides, transfer maps --
-// right after the row indices, so the phase costs three dependent memory
-// round trips instead of two per list; a K row needed by two sweeps is loaded
-// once.  Same operations in the same order as the general forms below.
+// at once (the row indices come from LDS); a K row needed by two sweeps is
+// loaded once.  Same operations in the same order as the general forms below.
 
-// a K row of width 18 in registers: its columns as local indices and values
+// a K row of 9 pairs in registers: its columns as local indices, packed, and
+// its values
 struct KRow18 {
-    int c[18];
-    float v[18];
+    unsigned c[9];
+    f2v v[9];
 };
 
-__device__ __forceinline__ void krow_load(KRow18 &k, const MCL_G unsigned short *map, int ms, int mi,
-                                          const GLevel &F, int row)
+__device__ __forceinline__ void krow_load(KRow18 &k, const MCL_G unsigned *map, int ms, int mi, const GLevel &F,
+                                          int row)
 {
 #pragma unroll
-    for (int u = 0; u < 18; u++) {
+    for (int u = 0; u < 9; u++) {
         k.c[u] = map[u * ms + mi];
         k.v[u] = F.val[u * F.n + row];
     }
@@ -682,7 +745,11 @@ __device__ __forceinline__ float krow_dot(const KRow18 &k, XP x)
 {
     float s = 0.f;
 #pragma unroll
-    for (int u = 0; u < 18; u++) s += k.v[u] * x[k.c[u]];
+    for (int u = 0; u < 9; u++) {
+        const i2v c = col_pair(k.c[u]);
+        s += k.v[u].x * x[c.x];
+        s += k.v[u].y * x[c.y];
+    }
     return s;
 }
 
@@ -691,24 +758,21 @@ template <typename LB>
 __device__ __forceinline__ bool deep_down1(const GLevel &F, const GLevel &C, LB buf, float wf, float wc)
 {
     const Own o = own_block(F.n), oc = own_block(C.n);
-    const int g = blockIdx.x;
-    const int t0 = F.th_ptr[g], nth = F.th_ptr[g + 1] - t0;
-    const int u0 = F.uh_ptr[g], nuh = F.uh_ptr[g + 1] - u0;
-    const int f0 = F.hd_ptr[g], nf = F.hd_ptr[g + 1] - f0;
-    const int nT = o.R + nth, nU = nT + nuh;
-    if (F.WK != 18 || C.rw > 9 || nU > MCL_BLOCK || nf > MCL_BLOCK || oc.R > MCL_BLOCK) return false;
+    const int g = blockIdx.x, t0 = F.ls.t0, f0 = F.ls.f0, nf = F.ls.nf;
+    const int nT = o.R + F.ls.nth, nU = nT + F.ls.nuh;
+    if (F.WK2 != 9 || C.rw > 9 || nU > MCL_BLOCK || nf > MCL_BLOCK || oc.R > MCL_BLOCK) return false;
     const int t = threadIdx.x;
     const auto xU = buf;
     const auto xT = buf + nU;
     const auto rF = xT + nT;
     // this thread's row of U (T is its prefix) and of F
     const bool inU = t < nU && (t >= o.R || t < o.no), inT = inU && t < nT, inF = t < nf;
-    const int ru = inU ? (t < o.R ? o.b0 + t : t < nT ? F.th_row[t0 + t - o.R] : F.uh_row[u0 + t - nT]) : 0;
-    const int rf = inF ? F.hd_row[f0 + t] : 0;
+    const int ru = inU ? urow(F, o, t) : 0;
+    const int rf = inF ? frow(F, t) : 0;
     // every load that does not wait on another workgroup
     KRow18 kt, kf;
-    if (inT) krow_load(kt, F.mt + (size_t)((long long)g * o.R + t0) * F.WK, nT, t, F, ru);
-    if (inF) krow_load(kf, F.mf + (size_t)f0 * F.WK, nf, t, F, rf);
+    if (inT) krow_load(kt, F.mt + (size_t)((long long)g * o.R + t0) * F.WK2, nT, t, F, ru);
+    if (inF) krow_load(kf, F.mf + (size_t)f0 * F.WK2, nf, t, F, rf);
     const float dT = inT ? F.dinv[ru] : 0.f;
     const float bT = inT ? vld<kCO>(F.b + ru) : 0.f;
     const float bF = inF ? vld<kCO>(F.b + rf) : 0.f;
@@ -754,32 +818,28 @@ __device__ __forceinline__ void deep_down(const GLevel &F, const GLevel &C, LB b
 {
     if (deep_down1(F, C, buf, wf, wc)) return;
     const Own o = own_block(F.n);
-    const int g = blockIdx.x;
-    const int t0 = F.th_ptr[g], nth = F.th_ptr[g + 1] - t0;
-    const int u0 = F.uh_ptr[g], nuh = F.uh_ptr[g + 1] - u0;
-    const int f0 = F.hd_ptr[g], nf = F.hd_ptr[g + 1] - f0;
-    const int nT = o.R + nth, nU = nT + nuh;
+    const int g = blockIdx.x, t0 = F.ls.t0, f0 = F.ls.f0, nf = F.ls.nf;
+    const int nT = o.R + F.ls.nth, nU = nT + F.ls.nuh;
     const auto xU = buf;
     const auto xT = buf + nU;
     const auto rF = xT + nT;
-    auto urow = [&](int t) { return t < o.R ? o.b0 + t : t < nT ? F.th_row[t0 + t - o.R] : F.uh_row[u0 + t - nT]; };
     const auto x1 = sweep_buf(F, 1);
     for (int t = threadIdx.x; t < nU; t += blockDim.x)
-        if (t >= o.R || t < o.no) xU[t] = vld<kCO>(x1 + urow(t));
+        if (t >= o.R || t < o.no) xU[t] = vld<kCO>(x1 + urow(F, o, t));
     __syncthreads();
     const auto x2 = sweep_buf(F, 2);
-    const MCL_G unsigned short *mt = F.mt + (size_t)((long long)g * o.R + t0) * F.WK;
+    const MCL_G unsigned *mt = F.mt + (size_t)((long long)g * o.R + t0) * F.WK2;
     for (int t = threadIdx.x; t < nT; t += blockDim.x) {
         if (t < o.R && t >= o.no) continue;
-        const int row = urow(t);
+        const int row = urow(F, o, t);
         const float v = xU[t] + wf * F.dinv[row] * (vld<kCO>(F.b + row) - ell32_map(F, mt, nT, t, row, xU));
         xT[t] = v;
         if (t < o.R) vst<kCO>(x2 + row, v);
     }
     __syncthreads();
-    const MCL_G unsigned short *mf = F.mf + (size_t)f0 * F.WK;
+    const MCL_G unsigned *mf = F.mf + (size_t)f0 * F.WK2;
     for (int t = threadIdx.x; t < nf; t += blockDim.x) {
-        const int row = F.hd_row[f0 + t];
+        const int row = frow(F, t);
         rF[t] = vld<kCO>(F.b + row) - ell32_map(F, mf, nf, t, row, xT);
     }
     __syncthreads();
@@ -790,33 +850,21 @@ __device__ __forceinline__ void deep_down(const GLevel &F, const GLevel &C, LB b
 // (the map: kl for O rows, hm for H1 rows)
 struct Halo2 {
     Own o;
-    int h10, nh1, h20, nh2, nW, nV;
+    int h10, nh1, nW, nV;
 };
 
 __device__ __forceinline__ Halo2 halo2(const GLevel &F)
 {
-    Halo2 h;
-    h.o = own_block(F.n);
-    const int g = blockIdx.x;
-    h.h10 = F.hu_ptr[g];
-    h.nh1 = F.hu_ptr[g + 1] - h.h10;
-    h.h20 = F.h2_ptr[g];
-    h.nh2 = F.h2_ptr[g + 1] - h.h20;
-    h.nW = h.o.R + h.nh1;
-    h.nV = h.nW + h.nh2;
-    return h;
-}
-
-__device__ __forceinline__ int vrow(const GLevel &F, const Halo2 &h, int t)
-{
-    return t < h.o.R ? h.o.b0 + t : t < h.nW ? F.hu_row[h.h10 + t - h.o.R] : F.h2_row[h.h20 + t - h.nW];
+    const Own o = own_block(F.n);
+    const LevelLists &l = F.ls;
+    return Halo2{o, l.h10, l.nh1, o.R + l.nh1, o.R + l.nh1 + l.nh2};
 }
 
 template <typename XP>
 __device__ __forceinline__ float kw_row(const GLevel &F, const Halo2 &h, int t, int row, XP xV)
 {
-    if (t < h.o.R) return ell32c<false>(F.WK, F.n, F.kl, F.val, row, xV);
-    return ell32_map(F, F.hm + (size_t)h.h10 * F.WK, h.nh1, t - h.o.R, row, xV);
+    if (t < h.o.R) return ellp<false>(F.WK2, F.kl, F.n, row, F.val, F.n, row, xV);
+    return ell32_map(F, F.hm + (size_t)h.h10 * F.WK2, h.nh1, t - h.o.R, row, xV);
 }
 
 // The thread's row of V (-1: none), and its K row when it is a row of W:
@@ -825,12 +873,12 @@ __device__ __forceinline__ float kw_row(const GLevel &F, const Halo2 &h, int t, 
 __device__ __forceinline__ int v_row1(const GLevel &F, const Halo2 &h, int t, KRow18 &kw, float &dW, float &bW)
 {
     const bool inV = t < h.nV && (t >= h.o.R || t < h.o.no);
-    const int rv = inV ? vrow(F, h, t) : -1;
+    const int rv = inV ? vrow(F, h.o, t) : -1;
     dW = 0.f;
     bW = 0.f;
     if (inV && t < h.nW) {
         if (t < h.o.R) krow_load(kw, F.kl, F.n, rv, F, rv);
-        else krow_load(kw, F.hm + (size_t)h.h10 * F.WK, h.nh1, t - h.o.R, F, rv);
+        else krow_load(kw, F.hm + (size_t)h.h10 * F.WK2, h.nh1, t - h.o.R, F, rv);
         dW = F.dinv[rv];
         bW = vld<kCO>(F.b + rv);
     }
@@ -841,7 +889,7 @@ __device__ __forceinline__ int v_row1(const GLevel &F, const Halo2 &h, int t, KR
 template <typename LB>
 __device__ __forceinline__ bool deep_down_last1(const GLevel &F, const Halo2 &h, LB buf, float wf)
 {
-    if (F.WK != 18 || h.nV > MCL_BLOCK) return false;
+    if (F.WK2 != 9 || h.nV > MCL_BLOCK) return false;
     const int t = threadIdx.x;
     const auto xV = buf;
     const auto xW = buf + h.nV;
@@ -874,19 +922,19 @@ __device__ __forceinline__ void deep_down_last(const GLevel &F, LB buf, float wf
     const auto xW = buf + h.nV;
     const auto x1 = sweep_buf(F, 1);
     for (int t = threadIdx.x; t < h.nV; t += blockDim.x)
-        if (t >= h.o.R || t < h.o.no) xV[t] = vld<kCO>(x1 + vrow(F, h, t));
+        if (t >= h.o.R || t < h.o.no) xV[t] = vld<kCO>(x1 + vrow(F, h.o, t));
     __syncthreads();
     const auto x2 = sweep_buf(F, 2);
     for (int t = threadIdx.x; t < h.nW; t += blockDim.x) {
         if (t < h.o.R && t >= h.o.no) continue;
-        const int row = vrow(F, h, t);
+        const int row = vrow(F, h.o, t);
         const float v = xV[t] + wf * F.dinv[row] * (vld<kCO>(F.b + row) - kw_row(F, h, t, row, xV));
         xW[t] = v;
         if (t < h.o.R) vst<kCO>(x2 + row, v);
     }
     __syncthreads();
     for (int i = h.o.b0 + (int)threadIdx.x; i < h.o.b0 + h.o.no; i += blockDim.x)
-        vst<kCO>(F.r + i, vld<kCO>(F.b + i) - ell32c<false>(F.WK, F.n, F.kl, F.val, i, xW));
+        vst<kCO>(F.r + i, vld<kCO>(F.b + i) - ellp<false>(F.WK2, F.kl, F.n, i, F.val, F.n, i, xW));
 }
 
 // Two-sweep up-leg phase of grid level F (pre = 2): x' = x_2 + P x_c on V
@@ -901,7 +949,7 @@ template <bool CC, typename XC, typename LB>
 __device__ __forceinline__ bool deep_up1(const GLevel &F, const Halo2 &h, XC xc, LB buf, float w, bool finest,
                                          const MixedParams &P, const double *__restrict__ r, dd &rz)
 {
-    if (F.WK != 18 || h.nV > MCL_BLOCK) return false;
+    if (F.WK2 != 9 || h.nV > MCL_BLOCK) return false;
     const int t = threadIdx.x;
     const auto xV = buf;
     const auto xW = buf + h.nV;
@@ -954,7 +1002,7 @@ __device__ __forceinline__ void deep_up(const GLevel &F, XC xc, LB buf, float w,
     const auto x2 = sweep_buf(F, 2);
     for (int t = threadIdx.x; t < h.nV; t += blockDim.x) {
         if (t < h.o.R && t >= h.o.no) continue;
-        const int u = vrow(F, h, t);
+        const int u = vrow(F, h.o, t);
         const int m = F.pn[u];
         int lc[4];
         float gv[4];
@@ -975,13 +1023,13 @@ __device__ __forceinline__ void deep_up(const GLevel &F, XC xc, LB buf, float w,
     __syncthreads();
     for (int t = threadIdx.x; t < h.nW; t += blockDim.x) {
         if (t < h.o.R && t >= h.o.no) continue;
-        const int row = vrow(F, h, t);
+        const int row = vrow(F, h.o, t);
         xW[t] = xV[t] + w * F.dinv[row] * (vld<kCO>(F.b + row) - kw_row(F, h, t, row, xV));
     }
     __syncthreads();
     const LevelDev &L = P.U.L;
     for (int i = h.o.b0 + (int)threadIdx.x; i < h.o.b0 + h.o.no; i += blockDim.x) {
-        float z = xW[i - h.o.b0] + w * F.dinv[i] * (vld<kCO>(F.b + i) - ell32c<false>(F.WK, F.n, F.kl, F.val, i, xW));
+        float z = xW[i - h.o.b0] + w * F.dinv[i] * (vld<kCO>(F.b + i) - ellp<false>(F.WK2, F.kl, F.n, i, F.val, F.n, i, xW));
         if (finest) {
             if (L.nh > 0 && L.hp_n[i] != 0) z = 0.f;  // z lives in the constrained space
             rz = dd_add_prod(rz, r[i], (double)z);
@@ -1013,9 +1061,10 @@ __device__ __forceinline__ void lds_load_levels(const MixedParams &P, const MgLd
     for (int l = 0; l + 1 < P.nmg; l++) {
         const MCL_L MgLevelDev *G = S.lev + l;
         if (!G->block) continue;
-        const int m = G->WK * G->n, moff = G->moff, doff = G->lds_off / 3, n = G->n;
-        const MCL_G float *val = gp(G->val), *dinv = gp(G->dinv);
-        const MCL_G unsigned short *col = gp(G->col16);
+        const int m = G->WK2 * G->n, moff = G->moff / 2, doff = G->lds_off / 3, n = G->n;
+        const MCL_G f2v *val = (const MCL_G f2v *)G->val;
+        const MCL_G float *dinv = gp(G->dinv);
+        const MCL_G unsigned *col = gp(G->col16);
         for (int e = threadIdx.x; e < m; e += blockDim.x) {
             S.val[moff + e] = val[e];
             S.col[moff + e] = col[e];
@@ -1044,7 +1093,7 @@ __device__ __forceinline__ void coarse_solve(const MixedParams &P, const LdsLeve
 __device__ __forceinline__ void last_sweep_rz(const MixedParams &P, const MgLds &mgl, const double *__restrict__ r,
                                               dd &rz)
 {
-    const GLevel A = glevel(mgl.lev + P.nmg - 1);
+    const GLevel A = glevel(mgl, P.nmg - 1);
     const float w = P.omega / mgl.lam[P.nmg - 1];
     const int kf = 2 * P.pre;
     const auto in = sweep_buf(A, kf - 1);
@@ -1095,12 +1144,12 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
     for (int l = 0; l < top; l++)
         if (mgl.lev[l].block) lb = l;
     for (int l = top; l > lb; l--) {
-        const GLevel A = glevel(mgl.lev + l);
+        const GLevel A = glevel(mgl, l);
         const Ex ex = own_rows(A.n);
         const float w = P.omega / lam[l];
         if (deep_down_on(P, A)) {
             if (l - 1 > lb) {
-                deep_down(A, glevel(mgl.lev + l - 1), mgl.halo, w, P.omega / lam[l - 1]);
+                deep_down(A, glevel(mgl, l - 1), mgl.halo, w, P.omega / lam[l - 1]);
                 ok = vsync(gs, ws, ok, nbr, un);
             } else {
                 // every workgroup restricts the whole residual into its LDS
@@ -1114,7 +1163,7 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
             ok = vsync(gs, ws, ok, nbr, un);
         }
         if (l - 1 > lb) {
-            const GLevel C = glevel(mgl.lev + l - 1);
+            const GLevel C = glevel(mgl, l - 1);
             if (A.fuse_down) {
                 fused_down(A, C, mgl.halo, P.omega / lam[l - 1], pre);
             } else {
@@ -1132,7 +1181,7 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
     MCL_PHASE(2);
     {
         const LdsLevel B = lds_level(mgl, lb, pre);
-        restrict_to<kCO, false>(B, glevel(mgl.lev + lb + 1), lb > 0, P.omega / lam[lb], wg_rows(B.n));
+        restrict_to<kCO, false>(B, glevel(mgl, lb + 1), lb > 0, P.omega / lam[lb], wg_rows(B.n));
         __syncthreads();
         MCL_PHASE(7);
         for (int l = lb; l > 0; l--) {
@@ -1168,7 +1217,7 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
     }
     MCL_PHASE(3);
     for (int l = lb + 1; l <= top; l++) {
-        const GLevel A = glevel(mgl.lev + l);
+        const GLevel A = glevel(mgl, l);
         const Ex ex = own_rows(A.n);
         const float w = P.omega / lam[l];
         const bool finest = l == top;
@@ -1177,7 +1226,7 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
                 const LdsLevel C = lds_level(mgl, lb, pre);
                 deep_up<false>(A, sweep_buf(C, kf), mgl.halo, w, finest, P, r, rz);
             } else {
-                deep_up<kCO>(A, level_result(P, glevel(mgl.lev + l - 1)), mgl.halo, w, finest, P, r, rz);
+                deep_up<kCO>(A, level_result(P, glevel(mgl, l - 1)), mgl.halo, w, finest, P, r, rz);
             }
             if (!finest) ok = vsync(gs, ws, ok, nbr, un);
             continue;
@@ -1191,7 +1240,7 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
             if (fuse) fused_up<false>(A, sweep_buf(C, kf), mgl.halo, w, pre);
             else prolong_add<kCO, false>(A, sweep_buf(A, pre), sweep_buf(C, kf), ex);
         } else {
-            const auto xc = level_result(P, glevel(mgl.lev + l - 1));
+            const auto xc = level_result(P, glevel(mgl, l - 1));
             if (fuse) fused_up<kCO>(A, xc, mgl.halo, w, pre);
             else prolong_add<kCO, kCO>(A, sweep_buf(A, pre), xc, ex);
         }
@@ -1267,7 +1316,7 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
 {
     const LevelDev &L = P.U.L;
     const bool use_mg = P.nmg > 1;
-    const GLevel A = glevel(mgl.lev + P.nmg - 1);
+    const GLevel A = glevel(mgl, P.nmg - 1);
     const float wtop = use_mg ? P.omega / mgl.lam[P.nmg - 1] : 0.f;
     const MCL_G float *zf = use_mg ? level_result(P, A) : A.x;
     const int n = L.neq;
@@ -1478,13 +1527,16 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
 
 __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
 {
-    __shared__ float mg_vec[3 * MCL_MG_LDS_ROWS], mg_dinv[MCL_MG_LDS_ROWS], mg_val[MCL_MG_LDS_NNZ];
-    __shared__ unsigned short mg_col[MCL_MG_LDS_NNZ];
+    __shared__ float mg_vec[3 * MCL_MG_LDS_ROWS], mg_dinv[MCL_MG_LDS_ROWS];
+    __shared__ f2v mg_val[MCL_MG_LDS_NNZ / 2];
+    __shared__ unsigned mg_col[MCL_MG_LDS_NNZ / 2];
     // level descriptors and Gershgorin bounds (read in every phase; LDS keeps
     // them out of the grid barriers' cache invalidations)
     __shared__ MgLevelDev mg_lev[MCL_MG_MAX_LEVELS];
     __shared__ float mg_lam[MCL_MG_MAX_LEVELS];
     __shared__ float mg_halo[MCL_HALO_LDS];
+    __shared__ LevelLists mg_lists[MCL_MG_MAX_LEVELS];
+    __shared__ unsigned short mg_rows[MCL_LDS_LIST];
     {
         const int nw = P.nmg * (int)(sizeof(MgLevelDev) / sizeof(int));
         for (int e = threadIdx.x; e < nw; e += blockDim.x) ((int *)mg_lev)[e] = ((const int *)P.mg)[e];
@@ -1492,9 +1544,12 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
         __syncthreads();
     }
     const MgLds mgl{(const MCL_L MgLevelDev *)mg_lev, (const MCL_L float *)mg_lam, (MCL_L float *)mg_vec,
-                    (MCL_L float *)mg_dinv, (MCL_L float *)mg_val, (MCL_L unsigned short *)mg_col,
-                    (MCL_L float *)mg_halo};
-    if (P.nmg > 1) lds_load_levels(P, mgl);
+                    (MCL_L float *)mg_dinv, (MCL_L f2v *)mg_val, (MCL_L unsigned *)mg_col,
+                    (MCL_L float *)mg_halo, mg_lists, (MCL_L unsigned short *)mg_rows};
+    if (P.nmg > 1) {
+        lds_load_levels(P, mgl);
+        lds_load_lists(P, mgl);
+    }
     const UzawaParams &U = P.U;
     const LevelDev &L = U.L;
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsize = gridDim.x * blockDim.x;
