@@ -748,7 +748,7 @@ static int build_multigrid(mcl_ctx *c)
         M.n = Lv.neq;
         M.WK = Lv.WK;
         M.block = 0;
-        M.lds_off = 0;
+        M.p_off = M.r_off = M.i_off = -1;
         {
             const int w2 = (Lv.WK + 1) / 2;
             std::vector<int> col2(2 * (size_t)std::max(w2, 1) * n, 0);
@@ -781,13 +781,19 @@ static int build_multigrid(mcl_ctx *c)
     // the levels above it while each has at most block_rows_threshold() rows,
     // their rows sum to at most MCL_MG_LDS_ROWS, their ELL entries to at most
     // MCL_MG_LDS_NNZ, and the level is not the finest
+    int pool = 0;   // words of the LDS pool in use
+    auto take = [&](int words) {
+        const int at = pool;
+        pool += (words + 1) / 2 * 2;
+        return at;
+    };
     {
-        int off = 0, nnz = 0;
+        int rows = 0, nnz = 0;
         for (int k = 0; k < nlev - 1; k++) {
             Level &Lv = c->levels[k];
             const int n = Lv.neq, w2 = mg[k].WK2, m = 2 * w2 * n;
             if (k > 0 && n > block_rows_threshold()) break;
-            if (off / 3 + n > MCL_MG_LDS_ROWS || nnz + m > MCL_MG_LDS_NNZ || n > 65535) break;
+            if (rows + n > MCL_MG_LDS_ROWS || nnz + m > MCL_MG_LDS_NNZ || n > 65535) break;
             std::vector<unsigned> col16((size_t)std::max(w2 * n, 1), 0);
             for (int s = 0; s < 2 * w2; s++)
                 for (int i = 0; i < n; i++)
@@ -797,9 +803,11 @@ static int build_multigrid(mcl_ctx *c)
             if (dev_upload(c, Lv.owned, &cp, col16)) return MCL_E_DEVICE;
             mg[k].col16 = cp;
             mg[k].block = 1;
-            mg[k].lds_off = off;
-            mg[k].moff = nnz;
-            off += 3 * n;
+            mg[k].v_off = take(3 * n);
+            mg[k].d_off = take(n);
+            mg[k].a_off = take(m);
+            mg[k].c_off = take(m / 2);
+            rows += n;
             nnz += m;
             c->mg_lb = k;
         }
@@ -852,6 +860,36 @@ static int build_multigrid(mcl_ctx *c)
             mg[k - 1].rw = rw;
             mg[k - 1].rcol = C.rcol;
             mg[k - 1].rval = C.rval;
+        }
+        // the LDS levels' transfer maps and the coarsest inverse into what is left
+        // of the LDS pool, from the smallest on
+        auto room = [&](int words) { return pool + (words + 1) / 2 * 2 <= MCL_MG_POOL; };
+        if (mg[0].block && c->levels[0].neq <= 64 && room(2 * mg[0].n * mg[0].n))
+            mg[0].i_off = take(2 * mg[0].n * mg[0].n);
+        for (int k = 0; k <= c->mg_lb && k < nlev - 1; k++) {
+            const Level &C = c->levels[k], &F = c->levels[k + 1];
+            if (!mg[k].block) continue;
+            const int n = C.neq;
+            if (k > 0 && room(2 * n) && n < 0xfff) {
+                std::vector<unsigned> w(2 * (size_t)n);
+                for (int u = 0; u < n; u++) {
+                    const int m = C.interp_n[u];
+                    w[2 * u] = (unsigned)m << 24;
+                    for (int a = 0; a < 4; a++) {
+                        const int l = m > a ? C.interp_eq[a * (size_t)n + u] : -1;
+                        w[2 * u + (a >> 1)] |= (l >= 0 ? (unsigned)l : 0xfffu) << (12 * (a & 1));
+                    }
+                }
+                if (dev_upload(c, c->levels[k].owned, &mg[k].pro, w)) return MCL_E_DEVICE;
+                mg[k].p_off = take(2 * n);
+            }
+            if (F.neq <= 65536 && room(C.rw * n)) {
+                std::vector<unsigned> w((size_t)C.rw * n);
+                for (size_t e = 0; e < w.size(); e++)
+                    w[e] = C.rcol_h[e] >= 0 ? (unsigned)C.rcol_h[e] | (unsigned)F.interp_n[C.rcol_h[e]] << 16 : 0u;
+                if (dev_upload(c, c->levels[k].owned, &mg[k].res, w)) return MCL_E_DEVICE;
+                mg[k].r_off = take(C.rw * n);
+            }
         }
         if (c->levels[0].neq > 64) maps = false;  // the coarse solve holds a dense inverse of at most 64 rows
     }

@@ -149,11 +149,21 @@ struct HeatParams {
 #define MCL_MG_LDS_NNZ 16384
 #endif
 
+// 32-bit words of the LDS pool of the coarse levels: vectors, matrices, and
+// 8 KB more for the transfer maps and the coarsest inverse; smaller levels leave
+// room for all of them (a solve at 32x32 3.64 ms, 3.70 with the maps in memory;
+// 256x256 29.8, 30.4; hanging nodes at 32x16 54.1, 55.7).
+#define MCL_MG_POOL (4 * MCL_MG_LDS_ROWS + MCL_MG_LDS_NNZ * 3 / 2 + 2048)
+
 struct MgLevelDev {
     int n, WK;
     int block;               // coarse level run per workgroup from LDS
-    int lds_off;             // offset of its vectors in the LDS block (floats)
-    int moff;                // offset of its matrix in the LDS matrix block (entries)
+    // places in the LDS pool (32-bit words) of an LDS level: its vectors x, t, b,
+    // 1/diag, matrix values and columns; its transfer maps and (level 0) the
+    // coarsest inverse, -1: read from memory
+    int v_off, d_off, a_off, c_off, p_off, r_off, i_off;
+    const unsigned *pro;     // [n][2] prolongation packed: c0 | c1 << 12 | m << 24, c2 | c3 << 12, 0xfff: none
+    const unsigned *res;     // [rw][n] restriction packed: fine row | m << 16, weight 1 / m, 0: none
     // The FP32 matrix and every column map hold two slots of a row together
     // (WK2 = (WK + 1) / 2 pairs, [pair][row]; an odd row length is padded with
     // the row itself and 0): half the loads of one slot each, and their address

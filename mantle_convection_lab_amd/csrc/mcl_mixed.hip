@@ -238,6 +238,13 @@ __device__ __forceinline__ MCL_G T *gp(T *p)
     return (MCL_G T *)p;
 }
 
+// p + i with a 32-bit byte offset: a uniform p stays in scalar registers
+template <typename T>
+__device__ __forceinline__ const MCL_G T *at(const MCL_G T *p, int i)
+{
+    return (const MCL_G T *)((const MCL_G char *)p + (unsigned)i * (unsigned)sizeof(T));
+}
+
 // Vector accesses of the V-cycle.  CO = true for vectors of the grid levels
 // between neighbour waits: agent-scope atomic loads and stores (coherent
 // across the XCDs' L2 caches, see GridSync); CO = false for LDS vectors and
@@ -310,10 +317,10 @@ struct GLevel {
     const MCL_L unsigned short *rows;
 };
 
-// A coarse level as seen by one workgroup: vectors x, t, b (3 n floats at
-// lds_off), 1/diag(K) (n floats at lds_off / 3) and the FP32 K with 16-bit
-// columns (2 WK2 n entries at moff) in LDS, copied from HBM once per launch; the
-// transfer maps stay in HBM.
+// A coarse level as seen by one workgroup: vectors x, t, b, 1/diag(K) and the
+// FP32 K with 16-bit columns in LDS, copied from HBM once per launch; the
+// transfer maps too if they fit (pro, res: null otherwise, then from memory:
+// a round trip for each of the levels' six transfers).
 struct LdsLevel {
     int n, WK2, rw;
     const MCL_L unsigned *col;
@@ -321,6 +328,7 @@ struct LdsLevel {
     const MCL_L float *dinv;
     const MCL_G int *pn, *pcol, *rcol;
     const MCL_G float *rval;
+    const MCL_L unsigned *pro, *res;
     MCL_L float *x, *b, *r, *t;
 };
 
@@ -336,9 +344,7 @@ __device__ __forceinline__ auto sweep_buf(const LV &A, int k)
 struct MgLds {
     const MCL_L MgLevelDev *lev;
     const MCL_L float *lam;
-    MCL_L float *vec, *dinv;
-    MCL_L f2v *val;
-    MCL_L unsigned *col;
+    MCL_L float *pool;       // [MCL_MG_POOL]
     MCL_L float *halo;       // [MCL_HALO_LDS] buffer of the fused phases
     LevelLists *lists;       // LDS
     MCL_L unsigned short *rows;   // [MCL_LDS_LIST]
@@ -394,14 +400,16 @@ __device__ __forceinline__ LdsLevel lds_level(const MgLds &S, int l, int pre)
     A.n = G->n;
     A.WK2 = G->WK2;
     A.rw = G->rw;
-    A.col = S.col + G->moff / 2;
-    A.val = S.val + G->moff / 2;
-    A.dinv = S.dinv + G->lds_off / 3;
+    A.col = (const MCL_L unsigned *)(S.pool + G->c_off);
+    A.val = (const MCL_L f2v *)(S.pool + G->a_off);
+    A.dinv = S.pool + G->d_off;
+    A.pro = G->p_off >= 0 ? (const MCL_L unsigned *)(S.pool + G->p_off) : nullptr;
+    A.res = G->r_off >= 0 ? (const MCL_L unsigned *)(S.pool + G->r_off) : nullptr;
     A.pn = gp(G->pn);
     A.pcol = gp(G->pcol);
     A.rcol = gp(G->rcol);
     A.rval = gp(G->rval);
-    A.x = S.vec + G->lds_off;
+    A.x = S.pool + G->v_off;
     A.t = A.x + A.n;
     A.b = A.t + A.n;
     A.r = sweep_buf(A, pre - 1);
@@ -573,6 +581,62 @@ __device__ __forceinline__ void residual(const LV &A, XP x, Ex ex)
     for (int i = ex.b; i < ex.e; i += ex.s) vst<CO>(A.r + i, vld<CO>(A.b + i) - ell32<CO>(A, i, x));
 }
 
+// Nine entries of a coarse row's restriction from slot k0: fine rows (-1: none)
+// and weights.
+__device__ __forceinline__ void restriction9(const GLevel &C, int c, int k0, int (&u)[9], float (&v)[9])
+{
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const bool in = k0 + k < C.rw;
+        u[k] = in ? *at(C.rcol + (k0 + k) * C.n, c) : -1;
+        v[k] = in ? *at(C.rval + (k0 + k) * C.n, c) : 0.f;
+    }
+}
+
+__device__ __forceinline__ void restriction9(const LdsLevel &C, int c, int k0, int (&u)[9], float (&v)[9])
+{
+    if (C.res) {
+#pragma unroll
+        for (int k = 0; k < 9; k++) {
+            const unsigned w = k0 + k < C.rw ? C.res[(k0 + k) * C.n + c] : 0u, m = w >> 16;
+            u[k] = m ? (int)(w & 0xffffu) : -1;
+            v[k] = m < 3 ? (m < 2 ? 1.f : 0.5f) : (m < 4 ? 1.f / 3.f : 0.25f);
+        }
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const bool in = k0 + k < C.rw;
+        u[k] = in ? *at(C.rcol + (k0 + k) * C.n, c) : -1;
+        v[k] = in ? *at(C.rval + (k0 + k) * C.n, c) : 0.f;
+    }
+}
+
+// A row's prolongation: the mean of m coarse rows l (-1 past m and for fixed
+// ones)
+__device__ __forceinline__ int prolongation4(const GLevel &F, int u, int (&l)[4])
+{
+#pragma unroll
+    for (int k = 0; k < 4; k++) l[k] = *at(F.pcol + k * F.n, u);
+    return F.pn[u];
+}
+
+__device__ __forceinline__ int prolongation4(const LdsLevel &F, int u, int (&l)[4])
+{
+    if (F.pro) {
+        const unsigned w[2] = {F.pro[2 * u], F.pro[2 * u + 1]};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const unsigned c = w[k >> 1] >> (12 * (k & 1)) & 0xfffu;
+            l[k] = c == 0xfffu ? -1 : (int)c;
+        }
+        return (int)(w[0] >> 24);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) l[k] = *at(F.pcol + k * F.n, u);
+    return F.pn[u];
+}
+
 // Coarse right-hand side b_c = sum_k R_ck r_u (R = P^T, arrays on the coarse
 // level), fused with the coarse level's first sweep x_c = w_c D^-1 b_c unless
 // the coarse level is solved directly.  CF: access mode of the fine level's
@@ -586,12 +650,7 @@ __device__ __forceinline__ void restrict_to(const LC &C, const LF &F, bool sweep
         for (int k0 = 0; k0 < C.rw; k0 += 9) {
             int u[9];
             float v[9], g[9];
-#pragma unroll
-            for (int k = 0; k < 9; k++) {
-                const bool in = k0 + k < C.rw;
-                u[k] = in ? C.rcol[(k0 + k) * C.n + c] : -1;
-                v[k] = in ? C.rval[(k0 + k) * C.n + c] : 0.f;
-            }
+            restriction9(C, c, k0, u, v);
 #pragma unroll
             for (int k = 0; k < 9; k++) g[k] = u[k] >= 0 ? vld<CF>(F.r + u[k]) : 0.f;
 #pragma unroll
@@ -609,11 +668,9 @@ template <bool CF, bool CC, typename LF, typename XF, typename XC>
 __device__ __forceinline__ void prolong_add(const LF &F, XF xf, XC xc, Ex ex)
 {
     for (int u = ex.b; u < ex.e; u += ex.s) {
-        const int m = F.pn[u];
         int l[4];
         float g[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) l[k] = F.pcol[k * F.n + u];
+        const int m = prolongation4(F, u, l);
 #pragma unroll
         for (int k = 0; k < 4; k++) g[k] = (k < m && l[k] >= 0) ? vld<CC>(xc + l[k]) : 0.f;
         if (m == 0) continue;
@@ -1055,34 +1112,44 @@ __device__ __forceinline__ bool vsync(const GridSync &gs, WaitState &ws, bool ok
 #endif
 }
 
-// Copy of the LDS levels' matrices into the workgroup's LDS block.
+// Copy of the LDS levels' matrices, transfer maps and the coarsest inverse into
+// the workgroup's LDS pool.
 __device__ __forceinline__ void lds_load_levels(const MixedParams &P, const MgLds &S)
 {
+    auto copy = [&](int off, const void *from, int words) {
+        const MCL_G unsigned *p = (const MCL_G unsigned *)from;
+        MCL_L unsigned *q = (MCL_L unsigned *)(S.pool + off);
+        for (int e = threadIdx.x; e < words; e += blockDim.x) q[e] = p[e];
+    };
     for (int l = 0; l + 1 < P.nmg; l++) {
         const MCL_L MgLevelDev *G = S.lev + l;
         if (!G->block) continue;
-        const int m = G->WK2 * G->n, moff = G->moff / 2, doff = G->lds_off / 3, n = G->n;
-        const MCL_G f2v *val = (const MCL_G f2v *)G->val;
-        const MCL_G float *dinv = gp(G->dinv);
-        const MCL_G unsigned *col = gp(G->col16);
-        for (int e = threadIdx.x; e < m; e += blockDim.x) {
-            S.val[moff + e] = val[e];
-            S.col[moff + e] = col[e];
-        }
-        for (int i = threadIdx.x; i < n; i += blockDim.x) S.dinv[doff + i] = dinv[i];
+        const int n = G->n, m = G->WK2 * n;
+        copy(G->a_off, G->val, 2 * m);
+        copy(G->c_off, G->col16, m);
+        copy(G->d_off, G->dinv, n);
+        if (G->p_off >= 0) copy(G->p_off, G->pro, 2 * n);
+        if (G->r_off >= 0) copy(G->r_off, G->res, G->rw * n);
+        if (G->i_off >= 0) copy(G->i_off, P.cinv, 2 * n * n);
     }
     __syncthreads();
 }
 
 // Coarsest level: x = K0^-1 b by the dense FP64 inverse, four lanes per row
 // (MCL_BLOCK >= 4 n threads; n <= 64).
-__device__ __forceinline__ void coarse_solve(const MixedParams &P, const LdsLevel &C)
+__device__ __forceinline__ void coarse_solve(const MixedParams &P, const MgLds &S)
 {
-    const int i = threadIdx.x >> 2, q = threadIdx.x & 3;
+    const LdsLevel C = lds_level(S, 0, P.pre);
+    const int i = threadIdx.x >> 2, q = threadIdx.x & 3, i_off = S.lev[0].i_off;
+    const MCL_L double *li = (const MCL_L double *)(S.pool + max(i_off, 0));
     const MCL_G double *cinv = gp(P.cinv);
     double s = 0.0;
-    if (i < C.n)
-        for (int j = q; j < C.n; j += 4) s += cinv[i * C.n + j] * (double)C.b[j];
+    if (i < C.n) {
+        if (i_off >= 0)
+            for (int j = q; j < C.n; j += 4) s += li[i * C.n + j] * (double)C.b[j];
+        else
+            for (int j = q; j < C.n; j += 4) s += cinv[i * C.n + j] * (double)C.b[j];
+    }
     s += __shfl_xor(s, 1, MCL_WAVE);
     s += __shfl_xor(s, 2, MCL_WAVE);
     if (q == 0 && i < C.n) sweep_buf(C, 2 * P.pre)[i] = (float)s;
@@ -1199,7 +1266,7 @@ __device__ __forceinline__ void vcycle_rest(const MixedParams &P, const MgLds &m
             __syncthreads();
         }
         MCL_PHASE(8);
-        coarse_solve(P, lds_level(mgl, 0, pre));
+        coarse_solve(P, mgl);
         __syncthreads();
         MCL_PHASE(9);
         for (int l = 1; l <= lb; l++) {
@@ -1527,9 +1594,7 @@ __device__ __forceinline__ int inner_mixed(const MixedParams &P, const double *_
 
 __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
 {
-    __shared__ float mg_vec[3 * MCL_MG_LDS_ROWS], mg_dinv[MCL_MG_LDS_ROWS];
-    __shared__ f2v mg_val[MCL_MG_LDS_NNZ / 2];
-    __shared__ unsigned mg_col[MCL_MG_LDS_NNZ / 2];
+    __shared__ __attribute__((aligned(16))) float mg_pool[MCL_MG_POOL];
     // level descriptors and Gershgorin bounds (read in every phase; LDS keeps
     // them out of the grid barriers' cache invalidations)
     __shared__ MgLevelDev mg_lev[MCL_MG_MAX_LEVELS];
@@ -1543,8 +1608,7 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
         for (int e = threadIdx.x; e < P.nmg; e += blockDim.x) mg_lam[e] = P.lam[e];
         __syncthreads();
     }
-    const MgLds mgl{(const MCL_L MgLevelDev *)mg_lev, (const MCL_L float *)mg_lam, (MCL_L float *)mg_vec,
-                    (MCL_L float *)mg_dinv, (MCL_L f2v *)mg_val, (MCL_L unsigned *)mg_col,
+    const MgLds mgl{(const MCL_L MgLevelDev *)mg_lev, (const MCL_L float *)mg_lam, (MCL_L float *)mg_pool,
                     (MCL_L float *)mg_halo, mg_lists, (MCL_L unsigned short *)mg_rows};
     if (P.nmg > 1) {
         lds_load_levels(P, mgl);
