@@ -43,8 +43,6 @@ struct Level {
     // device fields
     double *T = nullptr, *vis = nullptr, *buoy = nullptr, *V = nullptr, *d = nullptr, *p = nullptr;
     double *stress = nullptr, *es = nullptr, *area = nullptr, *avg = nullptr;
-    double *bterms = nullptr;  // [4][entries] terms of the buoyancy row averages
-    int bnent = 0;
     // multigrid (mixed precision): prolongation maps of this level (fine side)
     std::vector<int> interp_n, interp_eq;
     int *c2f = nullptr;                       // coarse node -> finest local node
@@ -76,6 +74,8 @@ struct mcl_ctx {
     int nlev = 0;
     const AsmLevel *asm_tab = nullptr;  // [nlev] all-levels assembly table (device)
     int asm_blocks = 0;                 // workgroups of its launch
+    const FieldLevel *field_tab = nullptr;  // [nlev] all-levels nodal field table (device)
+    int field_blocks = 0, inject_blocks = 0;   // workgroups over all levels, over the coarser ones
     const PrepLevel *prep_tab = nullptr;  // [prep_n] FP32 preparation table of the mixed solve (device)
     int prep_n = 0, prep_blocks = 0;
     double al_gamma = 0.0;               // > 0: the mixed solve runs on K_al (al_tab: [prep_n] levels)
@@ -695,8 +695,6 @@ static int build_level(mcl_ctx *c, const mcl_mesh_view &v, Level &Lv)
     rc |= dev_upload(c, o, &cp, bent); Lv.brow_e = (int *)cp;
     rc |= dev_upload(c, o, &sp, bx); Lv.brow_xi = (signed char *)sp;
     rc |= dev_upload(c, o, &sp, bz); Lv.brow_eta = (signed char *)sp;
-    Lv.bnent = (int)bent.size();
-    rc |= dev_alloc(c, o, &Lv.bterms, 4 * std::max<size_t>(bent.size(), 1));
     rc |= dev_alloc(c, o, &Lv.T, nno);
     rc |= dev_alloc(c, o, &Lv.vis, nno);
     rc |= dev_alloc(c, o, &Lv.buoy, nno);
@@ -1076,13 +1074,29 @@ extern "C" int mcl_mesh_upload(mcl_ctx *c, const mcl_mesh_view *levels, int nlev
             tab[l].vis = Lv.vis;
             tab[l].buoy = Lv.buoy;
             tab[l].blk0 = blk;
-            blk += (Lv.neq + MCL_BLOCK - 1) / MCL_BLOCK;
+            blk += (Lv.neq + MCL_ASM_BLOCK - 1) / MCL_ASM_BLOCK;
         }
         const AsmLevel *tp = nullptr;
         int rc = dev_upload(c, c->levels[nlev - 1].owned, &tp, tab);
         if (rc) return rc;
         c->asm_tab = tp;
         c->asm_blocks = blk;
+    }
+    {
+        // and the nodal field table
+        std::vector<FieldLevel> tab(nlev);
+        int blk = 0;
+        for (int l = 0; l < nlev; l++) {
+            Level &Lv = c->levels[l];
+            tab[l] = FieldLevel{Lv.nno, blk, Lv.c2f, Lv.dev.X, Lv.T, Lv.vis};
+            if (l == nlev - 1) c->inject_blocks = blk;
+            blk += (Lv.nno + MCL_BLOCK - 1) / MCL_BLOCK;
+        }
+        const FieldLevel *tp = nullptr;
+        int rc = dev_upload(c, c->levels[nlev - 1].owned, &tp, tab);
+        if (rc) return rc;
+        c->field_tab = tp;
+        c->field_blocks = blk;
     }
     {
         // warm-start history of the mixed solve (MCL_EXTRAPOLATE=n:
@@ -1392,9 +1406,9 @@ extern "C" int mcl_viscosity(mcl_ctx *c)
     int rc = ready(c);
     if (rc) return rc;
     HIPCHK(c, hipSetDevice(c->device));
-    for (auto &L : c->levels) {
-        hipLaunchKernelGGL(k_viscosity, dim3(grid_for(c, L.nno)), dim3(MCL_BLOCK), 0, c->stream, L.nno, L.T,
-                           L.dev.X, c->ctl.A, c->ctl.refT, c->ctl.lm_jump, L.vis);
+    if (c->field_blocks > 0) {
+        hipLaunchKernelGGL(k_viscosity, dim3(c->field_blocks), dim3(MCL_BLOCK), 0, c->stream, c->field_tab, c->nlev,
+                           c->ctl.A, c->ctl.refT, c->ctl.lm_jump);
         HIPCHK(c, hipGetLastError());
     }
     return 0;
@@ -1402,11 +1416,9 @@ extern "C" int mcl_viscosity(mcl_ctx *c)
 
 static int inject_temperature(mcl_ctx *c)
 {
-    Level &F = c->levels.back();
-    for (int k = 0; k + 1 < c->nlev; k++) {
-        Level &Lv = c->levels[k];
-        hipLaunchKernelGGL(k_inject, dim3(grid_for(c, Lv.nno)), dim3(MCL_BLOCK), 0, c->stream, Lv.nno,
-                           (const int *)Lv.c2f, (const double *)F.T, Lv.T);
+    if (c->inject_blocks > 0) {
+        hipLaunchKernelGGL(k_inject, dim3(c->inject_blocks), dim3(MCL_BLOCK), 0, c->stream, c->field_tab,
+                           c->nlev - 1, (const double *)c->levels.back().T);
         HIPCHK(c, hipGetLastError());
     }
     return 0;
@@ -1426,11 +1438,8 @@ extern "C" int mcl_buoyancy_force(mcl_ctx *c)
     for (auto &L : c->levels) {
         // the mixed path's coarse levels carry only K (their F is not used)
         if (c->ctl.precision == MCL_PREC_MIXED && &L != &c->levels.back()) continue;
-        if (L.bnent > 0)
-            hipLaunchKernelGGL(k_buoy_terms, dim3(grid_for(c, L.bnent)), dim3(MCL_BLOCK), 0, c->stream, L.bnent, L.nno,
-                               L.brow_e, L.brow_xi, L.brow_eta, L.dev.ienl, L.nel, L.T, c->ctl.Ra, L.bterms);
-        hipLaunchKernelGGL(k_buoy_rows, dim3((L.gnoz + MCL_BLOCK - 1) / MCL_BLOCK), dim3(MCL_BLOCK), 0, c->stream,
-                           L.gnoz, L.gnox, L.brow_ptr, (const double *)L.bterms, L.avg);
+        hipLaunchKernelGGL(k_buoy_rows, dim3(L.gnoz), dim3(MCL_BUOY), 0, c->stream, L.gnox, L.nno, L.brow_ptr, L.brow_e,
+                           L.brow_xi, L.brow_eta, L.dev.ienl, L.nel, L.T, c->ctl.Ra, L.avg);
         HIPCHK(c, hipGetLastError());
         hipLaunchKernelGGL(k_buoy_apply, dim3(grid_for(c, L.nno)), dim3(MCL_BLOCK), 0, c->stream, L.nno, L.gnoz,
                            L.dev.node, L.T, c->ctl.Ra, L.avg, L.buoy);
@@ -1447,7 +1456,7 @@ extern "C" int mcl_velocity_pressure_KGF_matrix(mcl_ctx *c)
     if (rc) return rc;
     HIPCHK(c, hipSetDevice(c->device));
     if (c->asm_blocks > 0) {
-        hipLaunchKernelGGL(k_assemble_K, dim3(c->asm_blocks), dim3(MCL_BLOCK), 0, c->stream,
+        hipLaunchKernelGGL(k_assemble_K, dim3(c->asm_blocks), dim3(MCL_ASM_BLOCK), 0, c->stream,
                            (const AsmLevel *)c->asm_tab, c->nlev);
         HIPCHK(c, hipGetLastError());
     }
@@ -1604,15 +1613,15 @@ static int mixed_prepare(mcl_ctx *c, bool by_kernel)
         hipLaunchKernelGGL(k_al_rows, dim3(c->al_rblocks), dim3(MCL_BLOCK), 0, c->stream, c->al_tab, c->prep_n);
         HIPCHK(c, hipGetLastError());
     }
-    if (c->prep_blocks > 0) {
-        hipLaunchKernelGGL(k_prepare_fp32, dim3(c->prep_blocks), dim3(MCL_BLOCK), 0, c->stream,
-                           (const PrepLevel *)c->prep_tab, c->prep_n);
-        HIPCHK(c, hipGetLastError());
-    }
+    CoarseInv ci{0, -1, nullptr, nullptr, nullptr, nullptr};
     if (c->have_mg) {
-        Level &C0 = c->levels[0];
-        hipLaunchKernelGGL(k_coarse_inverse, dim3(1), dim3(MCL_BLOCK), 0, c->stream, C0.neq, C0.WK, C0.dev.Kcol,
-                           C0.dev.Kncol, (const double *)(c->al_gamma > 0 ? C0.kval_al : C0.dev.Kval), c->cinv);
+        const Level &C0 = c->levels[0];
+        ci = CoarseInv{C0.neq, c->prep_blocks, C0.dev.Kcol, C0.dev.Kncol,
+                       c->al_gamma > 0 ? C0.kval_al : C0.dev.Kval, c->cinv};
+    }
+    if (c->prep_blocks > 0 || c->have_mg) {
+        hipLaunchKernelGGL(k_prepare_fp32, dim3(c->prep_blocks + (c->have_mg ? 1 : 0)), dim3(MCL_BLOCK), 0, c->stream,
+                           (const PrepLevel *)c->prep_tab, c->prep_n, ci);
         HIPCHK(c, hipGetLastError());
     }
     c->mixed_ready = true;
@@ -2411,7 +2420,7 @@ static int batch_capture(mcl_batch *b, int i)
     int rc = mcl_buoyancy_force(c);
     if (!rc) rc = mcl_viscosity(c);
     if (!rc && c->asm_blocks > 0) {
-        hipLaunchKernelGGL(k_assemble_K, dim3(c->asm_blocks), dim3(MCL_BLOCK), 0, c->stream,
+        hipLaunchKernelGGL(k_assemble_K, dim3(c->asm_blocks), dim3(MCL_ASM_BLOCK), 0, c->stream,
                            (const AsmLevel *)c->asm_tab, c->nlev);
         if (hipGetLastError() != hipSuccess) rc = fail(c, MCL_E_DEVICE, "assembly launch");
     }

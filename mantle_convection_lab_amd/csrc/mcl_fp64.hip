@@ -27,15 +27,38 @@ extern "C" hipError_t mcl_upload_shape(const ShapeTables *s)
 
 // ------------------------------------------------------------------ physics
 
-// Viscosity.c:3-24: eta = exp(A (refT - T)), times lm_jump below z = 0.77.
-__global__ void k_viscosity(int nno, const double *__restrict__ T, const double *__restrict__ X,
-                            double A, double refT, double lm_jump, double *__restrict__ vis)
+// The level of a workgroup in a launch over all levels (lv[k].blk0: the first
+// workgroup of level k).
+template <typename T>
+__device__ __forceinline__ const T &block_level(const T *__restrict__ lv, int nlev)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nno; i += gridDim.x * blockDim.x) {
-        double v = exp(A * (refT - T[i]));
-        if (X[nno + i] < 0.77) v *= lm_jump;
-        vis[i] = v;
-    }
+    int k = 0;
+    while (k + 1 < nlev && (int)blockIdx.x >= lv[k + 1].blk0) k++;
+    return lv[k];
+}
+
+// Viscosity.c:3-24: eta = exp(A (refT - T)), times lm_jump below z = 0.77; one
+// thread a node of every level.  (A launch for each level cost 4.5 us, seven
+// of them at 256x256; one 5 us.)
+__global__ void __launch_bounds__(MCL_BLOCK) k_viscosity(const FieldLevel *__restrict__ lv, int nlev, double A,
+                                                         double refT, double lm_jump)
+{
+    const FieldLevel &F = block_level(lv, nlev);
+    const int i = ((int)blockIdx.x - F.blk0) * MCL_BLOCK + (int)threadIdx.x;
+    if (i >= F.nno) return;
+    double v = exp(A * (refT - F.T[i]));
+    if (F.X[F.nno + i] < 0.77) v *= lm_jump;
+    F.vis[i] = v;
+}
+
+// coarse_n = fine_{c2f(n)}: the finest temperature on the nodes of every
+// coarser level
+__global__ void __launch_bounds__(MCL_BLOCK) k_inject(const FieldLevel *__restrict__ lv, int nlev,
+                                                      const double *__restrict__ fine)
+{
+    const FieldLevel &F = block_level(lv, nlev);
+    const int i = ((int)blockIdx.x - F.blk0) * MCL_BLOCK + (int)threadIdx.x;
+    if (i < F.nno) F.T[i] = fine[F.c2f[i]];
 }
 
 // Buoyancy.c:3-22 with get_node_horiz_avg (Parallel.c:354-437): one thread per
@@ -43,58 +66,65 @@ __global__ void k_viscosity(int nno, const double *__restrict__ T, const double 
 // (elements ascending; within an element the interior points, then the top
 // row or right column points, then the corner node).  Each entry adds
 // N_a(xi, eta) * data[node_a] for a = 0..3 separately, as the reference does.
-// Row averages in two passes.  k_buoy_terms evaluates every term of every
-// row's ordered contribution list in parallel (the products are the
-// reference's, independent of the running sum); k_buoy_rows then adds each
-// row's terms in list order, one thread per row, with its loads unrolled, so
-// the sum rounds exactly as the reference's sequential loop.  Entries with a
-// negative element contribute one term (Ra T of the last node) and three
-// +0.0 terms, which leave the sum unchanged.
-__global__ void k_buoy_terms(int nent, int nno, const int *__restrict__ ent_e, const signed char *__restrict__ ent_xi,
-                             const signed char *__restrict__ ent_eta, const int *__restrict__ ienl, int nel,
-                             const double *__restrict__ T, double Ra, double *__restrict__ terms)
+// A workgroup takes one row: its threads evaluate the terms of MCL_BUOY entries
+// into LDS (the products are the reference's, independent of the running sum),
+// then thread 0 adds them in list order, so the sum rounds exactly as the
+// reference's sequential loop; what bounds it is that chain of additions.
+// (One thread a row, reading the terms from memory, took 59 us for the 1028
+// terms a row of 256x256; this 11 us.)  Entries with a negative element
+// contribute one term (Ra T of the last node) and three +0.0 terms, which
+// leave the sum unchanged.
+__global__ void __launch_bounds__(MCL_BUOY) k_buoy_rows(int gnox, int nno, const int *__restrict__ ptr,
+                                                        const int *__restrict__ ent_e,
+                                                        const signed char *__restrict__ ent_xi,
+                                                        const signed char *__restrict__ ent_eta,
+                                                        const int *__restrict__ ienl, int nel,
+                                                        const double *__restrict__ T, double Ra,
+                                                        double *__restrict__ avg)
 {
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nent; t += gridDim.x * blockDim.x) {
-        int e = ent_e[t];
-        double v0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
-        if (e < 0) {
-            v0 = Ra * T[nno - 1];
-        } else {
-            double xi = (double)ent_xi[t], eta = (double)ent_eta[t];
-            // Na values of Shape_function.c:180-197
-            double n0 = 0.25 * (1.0 - xi) * (1.0 - eta);
-            double n1 = 0.25 * (1.0 - xi) * (1.0 + eta);
-            double n2 = 0.25 * (1.0 + xi) * (1.0 + eta);
-            double n3 = 0.25 * (1.0 + xi) * (1.0 - eta);
-            v0 = n0 * (Ra * T[ienl[e]]);
-            v1 = n1 * (Ra * T[ienl[nel + e]]);
-            v2 = n2 * (Ra * T[ienl[2 * nel + e]]);
-            v3 = n3 * (Ra * T[ienl[3 * nel + e]]);
-        }
-        terms[4 * (size_t)t] = v0;
-        terms[4 * (size_t)t + 1] = v1;
-        terms[4 * (size_t)t + 2] = v2;
-        terms[4 * (size_t)t + 3] = v3;
-    }
-}
-
-__global__ void k_buoy_rows(int gnoz, int gnox, const int *__restrict__ ptr, const double *__restrict__ terms,
-                            double *__restrict__ avg)
-{
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= gnoz) return;
-    const int t0 = 4 * ptr[k], t1 = 4 * ptr[k + 1];
+    __shared__ __attribute__((aligned(16))) double terms[4 * MCL_BUOY];
+    const int t0 = ptr[blockIdx.x], t1 = ptr[blockIdx.x + 1];
     double s = 0.0;
-    int t = t0;
-    for (; t + 8 <= t1; t += 8) {
-        double v[8];
+    for (int b = t0; b < t1; b += MCL_BUOY) {
+        const int t = b + (int)threadIdx.x;
+        if (t < t1) {
+            const int e = ent_e[t];
+            double v0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
+            if (e < 0) {
+                v0 = Ra * T[nno - 1];
+            } else {
+                double xi = (double)ent_xi[t], eta = (double)ent_eta[t];
+                // Na values of Shape_function.c:180-197
+                double n0 = 0.25 * (1.0 - xi) * (1.0 - eta);
+                double n1 = 0.25 * (1.0 - xi) * (1.0 + eta);
+                double n2 = 0.25 * (1.0 + xi) * (1.0 + eta);
+                double n3 = 0.25 * (1.0 + xi) * (1.0 - eta);
+                v0 = n0 * (Ra * T[ienl[e]]);
+                v1 = n1 * (Ra * T[ienl[nel + e]]);
+                v2 = n2 * (Ra * T[ienl[2 * nel + e]]);
+                v3 = n3 * (Ra * T[ienl[3 * nel + e]]);
+            }
+            terms[4 * threadIdx.x] = v0;
+            terms[4 * threadIdx.x + 1] = v1;
+            terms[4 * threadIdx.x + 2] = v2;
+            terms[4 * threadIdx.x + 3] = v3;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int n = 4 * min(MCL_BUOY, t1 - b);
+            int u = 0;
+            for (; u + 32 <= n; u += 32) {
+                double v[32];
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = terms[t + u];
+                for (int k = 0; k < 32; k++) v[k] = terms[u + k];
 #pragma unroll
-        for (int u = 0; u < 8; u++) s += v[u];
+                for (int k = 0; k < 32; k++) s += v[k];
+            }
+            for (; u < n; u++) s += terms[u];
+        }
+        __syncthreads();
     }
-    for (; t < t1; t++) s += terms[t];
-    avg[k] = s / gnox;
+    if (threadIdx.x == 0) avg[blockIdx.x] = s / gnox;
 }
 
 __global__ void k_buoy_apply(int nno, int gnoz, const int *__restrict__ node, const double *__restrict__ T,
@@ -109,56 +139,32 @@ __global__ void k_buoy_apply(int nno, int gnoz, const int *__restrict__ node, co
 
 // ------------------------------------------------------------ Stokes assembly
 
-// Upper-triangle element stiffness entry of get_element_K (Build_matrix.c:
-// 192-271) for row dof (a,i) and column dof (b,j) with 2a+i <= 2b+j; eta_g is
-// the linearly interpolated viscosity at the four Gauss points.
-__device__ __forceinline__ double ke_upper(int a, int i, int b, int j, const double eta_g[4], double dxdxi,
-                                           double dzdeta, double jac)
-{
-    const double dzdxi = 0.0, dxdeta = 0.0;
-    double K = 0.0;
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        double eta = eta_g[g];
-        double D00 = 2.0 * eta, D11 = 2.0 * eta, D22 = eta;
-        const double D01 = 0.0, D02 = 0.0, D10 = 0.0, D12 = 0.0, D20 = 0.0, D21 = 0.0;
-        double ax = c_shape.dxi[a][g] * dzdeta - c_shape.deta[a][g] * dzdxi;
-        double az = c_shape.deta[a][g] * dxdxi - c_shape.dxi[a][g] * dxdeta;
-        double bx = c_shape.dxi[b][g] * dzdeta - c_shape.deta[b][g] * dzdxi;
-        double bz = c_shape.deta[b][g] * dxdxi - c_shape.dxi[b][g] * dxdeta;
-        if (i == 0 && j == 0)
-            K += ((ax * D00 + az * D20) * bx + (ax * D02 + az * D22) * bz);
-        else if (i == 1 && j == 0)
-            K += ((az * D10 + ax * D20) * bx + (az * D12 + ax * D22) * bz);
-        else if (i == 0 && j == 1)
-            K += ((ax * D01 + az * D21) * bz + (ax * D02 + az * D22) * bx);
-        else
-            K += ((az * D11 + ax * D21) * bz + (az * D12 + ax * D22) * bx);
-    }
-    return K / jac;
-}
+// A row of the element stiffness matrix of get_element_K (Build_matrix.c:
+// 192-271) after the reference's mirror step: entry (p, q) is the value of the
+// upper entry (min(p, q), max(p, q)), a sum over the four Gauss points.  With u
+// and w the upper entry's first dof's shape derivative along and across its
+// direction, s and t the second's, and D = 2 eta for equal directions, else 0,
+// the four cases of the reference are one expression, (u D) s + (w eta) t (its
+// terms with a zero in the elasticity matrix add signed zeros, which leave the
+// sum as it is).  Both orders are summed and one is taken: fewer instructions
+// than choosing the operands.
+struct KeRow {
+    double u[4], w[4], we[4], eta[4];     // of the row's dof
+    double D[2][4], uD[2][4];             // with column dofs along x, z
+};
 
-// Element entry K_e[p][q] after the reference's mirror step: the value of the
-// upper entry (min(p,q), max(p,q)).
-__device__ __forceinline__ double ke_entry(int p, int q, const double eta_g[4], double dxdxi, double dzdeta,
+__device__ __forceinline__ double ke_entry(const KeRow &r, int p, int q, const double (&bx)[4], const double (&bz)[4],
                                            double jac)
 {
-    int lo = p < q ? p : q, hi = p < q ? q : p;
-    return ke_upper(lo >> 1, lo & 1, hi >> 1, hi & 1, eta_g, dxdxi, dzdeta, jac);
-}
-
-__device__ __forceinline__ void elem_eta(const LevelDev &L, int e, const double *__restrict__ vis, double eta_g[4])
-{
-    double vn[4];
-#pragma unroll
-    for (int d = 0; d < 4; d++) vn[d] = vis[L.ienl[d * L.nel + e]];
+    const bool jq = q & 1;
+    double Kr = 0.0, Kq = 0.0;   // the row's dof first, the column's
 #pragma unroll
     for (int g = 0; g < 4; g++) {
-        double s = 0.0;
-#pragma unroll
-        for (int d = 0; d < 4; d++) s += c_shape.N[d][g] * vn[d];
-        eta_g[g] = s;
+        const double s = jq ? bz[g] : bx[g], t = jq ? bx[g] : bz[g];
+        Kr += r.uD[jq][g] * s + r.we[g] * t;
+        Kq += (s * r.D[jq][g]) * r.u[g] + (t * r.eta[g]) * r.w[g];
     }
+    return (q < p ? Kq : Kr) / jac;
 }
 
 // One thread per velocity row P: K row slots (element-ascending sums, the
@@ -168,98 +174,146 @@ __device__ __forceinline__ void elem_eta(const LevelDev &L, int e, const double 
 // thread's own LDS column for rows of at most 18 slots (written to HBM once at
 // the end), else in place in HBM; the additions to each slot come in the same
 // order either way.  One launch assembles every level: each workgroup takes
-// MCL_BLOCK rows of one level (lv[k].blk0 gives the first workgroup of level
-// k), so the short levels run side by side instead of one launch each.
+// MCL_ASM_BLOCK rows of one level (lv[k].blk0 gives the first workgroup of level
+// k), so the short levels run side by side instead of one launch each.  What
+// bounds it is FP64 instruction issue (about 3000 a row): workgroups of 256
+// threads spread the rows more evenly than 512.  At 256x256 about 50 us, 112 with
+// the operands chosen per entry and every element's loads behind the last's.
 #define MCL_ASM_LDS_SLOTS 18
-__global__ void __launch_bounds__(MCL_BLOCK) k_assemble_K(const AsmLevel *__restrict__ lv, int nlev)
+__global__ void __launch_bounds__(MCL_ASM_BLOCK) k_assemble_K(const AsmLevel *__restrict__ lv, int nlev)
 {
-    __shared__ double kacc[MCL_ASM_LDS_SLOTS * MCL_BLOCK];
-    double *acc = kacc + threadIdx.x;  // slot u at acc[u * MCL_BLOCK]
-    int lk = 0;
-    while (lk + 1 < nlev && (int)blockIdx.x >= lv[lk + 1].blk0) lk++;
-    const LevelDev &L = lv[lk].L;
-    const double *__restrict__ vis = lv[lk].vis;
-    const double *__restrict__ buoy = lv[lk].buoy;
+    __shared__ double kacc[MCL_ASM_LDS_SLOTS * MCL_ASM_BLOCK];
+    __shared__ double sh[3][16];   // dN/dxi, dN/deta, N of (node, Gauss point)
+    if (threadIdx.x < 16) {
+        sh[0][threadIdx.x] = c_shape.dxi[threadIdx.x >> 2][threadIdx.x & 3];
+        sh[1][threadIdx.x] = c_shape.deta[threadIdx.x >> 2][threadIdx.x & 3];
+        sh[2][threadIdx.x] = c_shape.N[threadIdx.x >> 2][threadIdx.x & 3];
+    }
+    __syncthreads();
+    double *acc = kacc + threadIdx.x;  // slot u at acc[u * MCL_ASM_BLOCK]
+    const AsmLevel &lev = block_level(lv, nlev);
+    const LevelDev &L = lev.L;
+    const double *__restrict__ vis = lev.vis;
+    const double *__restrict__ buoy = lev.buoy;
     const bool inl = L.WK <= MCL_ASM_LDS_SLOTS;
     {
-        const int P = ((int)blockIdx.x - lv[lk].blk0) * MCL_BLOCK + (int)threadIdx.x;
+        const int P = ((int)blockIdx.x - lev.blk0) * MCL_ASM_BLOCK + (int)threadIdx.x;
         if (P >= L.neq) return;
         const int n = L.veq_node[P], ip = L.veq_dof[P];
         const int nadj = L.p2n_cnt[n];
-        const int nc = L.Kncol[P];
         if (inl)
-            for (int u = 0; u < L.WK; u++) acc[u * MCL_BLOCK] = 0.0;
+            for (int u = 0; u < L.WK; u++) acc[u * MCL_ASM_BLOCK] = 0.0;
         else
             for (int s = 0; s < L.WK; s++) L.Kval[s * L.neq + P] = 0.0;
+        // the elements at the row's node (a missing one reads the first's data)
+        int el[4], a[4], idx[4][4];
+        double dxdxi[4], dzdeta[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int kk = k < nadj ? k : 0;
+            el[k] = L.p2n_el[kk * L.nno + n];
+            a[k] = L.p2n_a[kk * L.nno + n];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int l = L.elev[el[k]];
+            dxdxi[k] = 0.5 * L.lvl_dx[l];
+            dzdeta[k] = 0.5 * L.lvl_dz[l];
+#pragma unroll
+            for (int d = 0; d < 4; d++) idx[k][d] = L.ienl[d * L.nel + el[k]];
+        }
         double F = 0.0;
-        for (int k = 0; k < nadj; k++) {
-            int e = L.p2n_el[k * L.nno + n], a = L.p2n_a[k * L.nno + n];
-            int lev = L.elev[e];
-            double dxdxi = 0.5 * L.lvl_dx[lev], dzdeta = 0.5 * L.lvl_dz[lev];
-            double jac = dxdxi * dzdeta - 0.0 * 0.0;
-            double eta_g[4];
-            elem_eta(L, e, vis, eta_g);
-            int p = 2 * a + ip;
-            for (int j = 0; j < 2; j++)
-                for (int b = 0; b < 4; b++) {
-                    int q = 2 * b + j;
-                    double kv = ke_entry(p, q, eta_g, dxdxi, dzdeta, jac);
-                    int slot = L.Kslot[(k * 8 + q) * L.neq + P];
-                    if (slot >= 0) {
-                        if (inl) acc[slot * MCL_BLOCK] += kv;
-                        else L.Kval[slot * L.neq + P] += kv;
-                    }
-                    int nb = L.ienl[b * L.nel + e];
-                    if (L.v_bc[j * L.nno + nb] == 'V') F -= kv * L.v_bc_val[j * L.nno + nb];
+        int sd = -1;   // the diagonal's slot
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (k >= nadj) break;
+            // keeps the next element's loads out of this one's registers
+            asm volatile("" ::: "memory");
+            const double jac = dxdxi[k] * dzdeta[k] - 0.0 * 0.0;
+            int slot[8];
+            char bc[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                slot[q] = L.Kslot[(k * 8 + q) * L.neq + P];
+                bc[q] = L.v_bc[(q & 1) * L.nno + idx[k][q >> 1]];
+            }
+            double vn[4];
+            KeRow row;
+#pragma unroll
+            for (int d = 0; d < 4; d++) vn[d] = vis[idx[k][d]];
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                double s = 0.0;
+#pragma unroll
+                for (int d = 0; d < 4; d++) s += c_shape.N[d][g] * vn[d];
+                const double ax = sh[0][4 * a[k] + g] * dzdeta[k], az = sh[1][4 * a[k] + g] * dxdxi[k];
+                row.eta[g] = s;
+                row.u[g] = ip ? az : ax;
+                row.w[g] = ip ? ax : az;
+                row.D[0][g] = ip ? 0.0 : 2.0 * s;
+                row.D[1][g] = ip ? 2.0 * s : 0.0;
+                row.uD[0][g] = row.u[g] * row.D[0][g];
+                row.uD[1][g] = row.u[g] * row.D[1][g];
+                row.we[g] = row.w[g] * s;
+            }
+            const int p = 2 * a[k] + ip;
+            // column dofs in the reference's order: j outer, b inner
+#pragma unroll
+            for (int jb = 0; jb < 8; jb++) {
+                const int j = jb >> 2, b = jb & 3, q = 2 * b + j;
+                double bx[4], bz[4];
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    bx[g] = c_shape.dxi[b][g] * dzdeta[k];
+                    bz[g] = c_shape.deta[b][g] * dxdxi[k];
                 }
+                const double kv = ke_entry(row, p, q, bx, bz, jac);
+                if (q == p) sd = slot[q];
+                if (slot[q] >= 0) {
+                    if (inl) acc[slot[q] * MCL_ASM_BLOCK] += kv;
+                    else L.Kval[slot[q] * L.neq + P] += kv;
+                }
+                if (bc[q] == 'V') F -= kv * L.v_bc_val[j * L.nno + idx[k][b]];
+            }
         }
         // element loads, get_element_F (Build_matrix.c:273-344)
-        for (int k = 0; k < nadj; k++) {
-            int e = L.p2n_el[k * L.nno + n], a = L.p2n_a[k * L.nno + n];
-            int lev = L.elev[e];
-            double dxdxi = 0.5 * L.lvl_dx[lev], dzdeta = 0.5 * L.lvl_dz[lev];
-            double jac = dxdxi * dzdeta - 0.0 * 0.0;
-            int idx[4];
 #pragma unroll
-            for (int d = 0; d < 4; d++) idx[d] = L.ienl[d * L.nel + e];
+        for (int k = 0; k < 4; k++) {
+            if (k >= nadj) break;
+            asm volatile("" ::: "memory");
+            const double jac = dxdxi[k] * dzdeta[k] - 0.0 * 0.0;
             double Fe = 0.0;
             if (ip == 1) {
-                double fg[4];
+                double fg[4], bn[4];
+#pragma unroll
+                for (int d = 0; d < 4; d++) bn[d] = buoy[idx[k][d]];
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
                     double s = 0.0;
 #pragma unroll
-                    for (int d = 0; d < 4; d++) s += c_shape.N[d][g] * buoy[idx[d]];
+                    for (int d = 0; d < 4; d++) s += c_shape.N[d][g] * bn[d];
                     fg[g] = s;
                 }
 #pragma unroll
-                for (int g = 0; g < 4; g++) Fe += c_shape.N[a][g] * fg[g];
+                for (int g = 0; g < 4; g++) Fe += sh[2][4 * a[k] + g] * fg[g];
                 Fe *= jac;
             }
             int nat = 0;
 #pragma unroll
             for (int d = 0; d < 4; d++)
-                if (L.v_bc[ip * L.nno + idx[d]] == 'S') nat += d;
+                if (L.v_bc[ip * L.nno + idx[k][d]] == 'S') nat += d;
             if (nat == 3) nat = 1;
             else if (nat == 1 || nat == 5) nat = 2;
             else if (nat == 0 || nat == 2) nat = 0;
             if (nat != 0) {
-                double Lx = L.X[ip * L.nno + idx[2]] - L.X[ip * L.nno + idx[0]];
-                Fe += 0.5 * Lx * L.v_bc_val[ip * L.nno + idx[a]];
+                double Lx = L.X[ip * L.nno + idx[k][2]] - L.X[ip * L.nno + idx[k][0]];
+                Fe += 0.5 * Lx * L.v_bc_val[ip * L.nno + L.ienl[a[k] * L.nel + el[k]]];
             }
             F += Fe;
         }
-        double diag = 0.0;
-        if (inl) {
-            for (int u = 0; u < L.WK; u++) {
-                const double v = acc[u * MCL_BLOCK];
-                L.Kval[u * L.neq + P] = v;
-                if (u < nc && L.Kcol[u * L.neq + P] == P) diag = v;
-            }
-        } else {
-            for (int s = 0; s < nc; s++)
-                if (L.Kcol[s * L.neq + P] == P) diag = L.Kval[s * L.neq + P];
-        }
+        if (inl)
+            for (int u = 0; u < L.WK; u++) L.Kval[u * L.neq + P] = acc[u * MCL_ASM_BLOCK];
+        const double diag = sd < 0 ? 0.0 : inl ? acc[sd * MCL_ASM_BLOCK] : L.Kval[sd * L.neq + P];
         L.F[P] = F;
         L.Kdiag[P] = diag;
     }

@@ -264,12 +264,19 @@ struct MixedParams {
 
 extern "C" hipError_t mcl_upload_shape(const ShapeTables *s);
 
-__global__ void k_viscosity(int nno, const double *T, const double *X, double A, double refT, double lm_jump,
-                            double *vis);
-__global__ void k_buoy_terms(int nent, int nno, const int *ent_e, const signed char *ent_xi,
-                             const signed char *ent_eta, const int *ienl, int nel, const double *T, double Ra,
-                             double *terms);
-__global__ void k_buoy_rows(int gnoz, int gnox, const int *ptr, const double *terms, double *avg);
+// A level's nodal fields in a launch over all levels (blk0: its first workgroup).
+struct FieldLevel {
+    int nno, blk0;
+    const int *c2f;      // [nno] the finest level's node of each node (coarser levels)
+    const double *X;
+    double *T, *vis;
+};
+__global__ void k_viscosity(const FieldLevel *lv, int nlev, double A, double refT, double lm_jump);
+__global__ void k_inject(const FieldLevel *lv, int nlev, const double *fine);
+#define MCL_BUOY 256   // threads of k_buoy_rows
+__global__ void k_buoy_rows(int gnox, int nno, const int *ptr, const int *ent_e, const signed char *ent_xi,
+                            const signed char *ent_eta, const int *ienl, int nel, const double *T, double Ra,
+                            double *avg);
 __global__ void k_buoy_apply(int nno, int gnoz, const int *node, const double *T, double Ra, const double *avg,
                              double *buoy);
 // One level of the all-levels assembly launch: its rows occupy the
@@ -279,6 +286,7 @@ struct AsmLevel {
     const double *vis, *buoy;
     int blk0;
 };
+#define MCL_ASM_BLOCK 256   // threads of k_assemble_K
 __global__ void k_assemble_K(const AsmLevel *lv, int nlev);
 // k_uzawa_fp64 for an inner solver (MCL_INNER_*)
 const void *mcl_uzawa_fp64_kernel(int solver);
@@ -299,7 +307,14 @@ struct PrepLevel {
     unsigned *bound;
     int blk0;
 };
-__global__ void k_prepare_fp32(const PrepLevel *lv, int nlev);
+// the coarsest level's K and where its dense inverse goes
+struct CoarseInv {
+    int n, blk;          // rows; the workgroup that computes it
+    const int *col, *ncol;
+    const double *val;
+    double *inv;
+};
+__global__ void k_prepare_fp32(const PrepLevel *lv, int nlev, CoarseInv ci);
 // One multigrid level of the augmented-Lagrangian launches: K_al = K +
 // gamma G W G^T (W = diag(w), w_e = 1 / sum_i G_ie^2 / K_ii, the BAB of the
 // plain K), same ELL pattern, gamma read from the device.  Elements occupy workgroups [eblk0, ...) of
@@ -318,6 +333,4 @@ __global__ void k_al_weights(const AlLevel *lv, int nlev);
 __global__ void k_extrapolate(int nv, int np, double *d, double *p, double *h, const double *ws,
                               const double *model_time, int after, double rmax);
 __global__ void k_al_rows(const AlLevel *lv, int nlev);
-__global__ void k_coarse_inverse(int n, int W, const int *col, const int *ncol, const double *val, double *inv);
-__global__ void k_inject(int nc, const int *c2f, const double *fine, double *coarse);
 __global__ void k_zero_words(unsigned *p, long long n);

@@ -40,12 +40,62 @@ __shared__ long long mcl_ph[MCL_PHASES + 1];
 
 // ------------------------------------------------------------ set-up kernels
 
+// Dense inverse of the coarsest K by in-place Gauss-Jordan elimination (K is
+// symmetric positive definite: no pivoting).  One workgroup, n <= 64.
+__device__ __forceinline__ void coarse_inverse(const CoarseInv &ci, double *A)
+{
+    __shared__ double rowk[64], colk[64];
+    const int n = ci.n;
+    for (int t = threadIdx.x; t < n * n; t += blockDim.x) A[t] = 0.0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += blockDim.x)
+        for (int s = 0; s < ci.ncol[i]; s++) A[i * n + ci.col[s * n + i]] = ci.val[s * n + i];
+    __syncthreads();
+    // this thread's entries (64 x 64 over MCL_BLOCK threads)
+    int ei[8], ej[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const int t = (int)threadIdx.x + u * MCL_BLOCK;
+        ei[u] = t < n * n ? t / n : -1;
+        ej[u] = t - (t / n) * n;
+    }
+    for (int k = 0; k < n; k++) {
+        if ((int)threadIdx.x < n) {
+            const int j = threadIdx.x;
+            const double piv = A[k * n + k];
+            rowk[j] = (j == k) ? 1.0 / piv : A[k * n + j] / piv;
+            colk[j] = A[j * n + k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int i = ei[u], j = ej[u], t = (int)threadIdx.x + u * MCL_BLOCK;
+            if (i < 0) continue;
+            if (i == k) {
+                A[t] = rowk[j];
+            } else {
+                double f = colk[i];
+                A[t] = (j == k) ? -f * rowk[k] : A[t] - f * rowk[j];
+            }
+        }
+        __syncthreads();
+    }
+    for (int t = threadIdx.x; t < n * n; t += blockDim.x) ci.inv[t] = A[t];
+}
+
 // FP32 copy of an FP64 ELL matrix, 1/diag, and the Gershgorin bound of D^-1 K
 // (max over rows of sum_j |K_ij| / K_ii), written as float bits with atomicMax
-// (positive floats order like their bit patterns).  One launch covers every
-// multigrid level: each workgroup takes MCL_BLOCK rows of one level.
-__global__ void __launch_bounds__(MCL_BLOCK) k_prepare_fp32(const PrepLevel *__restrict__ lv, int nlev)
+// (positive floats order like their bit patterns), one a workgroup: an atomic
+// of every wave on the level's one word took most of 39 us at 256x256 (11 so).
+// One launch covers every multigrid level: each workgroup takes MCL_BLOCK rows
+// of one level, one more inverts the coarsest K (26 us in a launch of its own).
+__global__ void __launch_bounds__(MCL_BLOCK) k_prepare_fp32(const PrepLevel *__restrict__ lv, int nlev, CoarseInv ci)
 {
+    __shared__ double lds[64 * 64];
+    if ((int)blockIdx.x == ci.blk) {
+        coarse_inverse(ci, lds);
+        return;
+    }
     int lk = 0;
     while (lk + 1 < nlev && (int)blockIdx.x >= lv[lk + 1].blk0) lk++;
     const PrepLevel &A = lv[lk];
@@ -53,18 +103,30 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_prepare_fp32(const PrepLevel *__r
     float m = 0.f;
     if (i < A.n) {
         double s = 0.0;
-        for (int k = 0; k < A.W; k += 2) {
-            const double v0 = A.val[k * A.n + i], v1 = k + 1 < A.W ? A.val[(k + 1) * A.n + i] : 0.0;
-            ((f2v *)A.val32)[(k >> 1) * A.n + i] = f2v{(float)v0, (float)v1};
-            s += fabs(v0);
-            s += fabs(v1);
+        for (int k0 = 0; k0 < A.W; k0 += 18) {
+            double v[18];
+#pragma unroll
+            for (int k = 0; k < 18; k++) v[k] = k0 + k < A.W ? A.val[(k0 + k) * A.n + i] : 0.0;
+#pragma unroll
+            for (int k = 0; k < 18; k += 2) {
+                if (k0 + k >= A.W) break;
+                ((f2v *)A.val32)[((k0 + k) >> 1) * A.n + i] = f2v{(float)v[k], (float)v[k + 1]};
+                s += fabs(v[k]);
+                s += fabs(v[k + 1]);
+            }
         }
         const double d = A.diag[i];
         A.dinv[i] = (float)(1.0 / d);
         m = (float)(s / d);
     }
     for (int o = MCL_WAVE / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, MCL_WAVE));
-    if ((threadIdx.x & (MCL_WAVE - 1)) == 0) atomicMax(A.bound, __float_as_uint(m));
+    float *wmax = (float *)lds;
+    if ((threadIdx.x & (MCL_WAVE - 1)) == 0) wmax[threadIdx.x / MCL_WAVE] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < MCL_BLOCK / MCL_WAVE; w++) m = fmaxf(m, wmax[w]);
+        atomicMax(A.bound, __float_as_uint(m));
+    }
 }
 
 // Augmented Lagrangian of the mixed solve: K_al = K + gamma G W G^T with W =
@@ -156,47 +218,6 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_extrapolate(int nv, int np, doubl
         if (ex) *x = x1 + r * (x1 - h[i]);
         h[i] = x1;
     }
-}
-
-// Dense inverse of the coarsest K by in-place Gauss-Jordan elimination (K is
-// symmetric positive definite: no pivoting).  One workgroup, n <= 64.
-__global__ void k_coarse_inverse(int n, int W, const int *__restrict__ col, const int *__restrict__ ncol,
-                                 const double *__restrict__ val, double *__restrict__ inv)
-{
-    __shared__ double A[64 * 64];
-    __shared__ double rowk[64], colk[64];
-    for (int t = threadIdx.x; t < n * n; t += blockDim.x) A[t] = 0.0;
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x)
-        for (int s = 0; s < ncol[i]; s++) A[i * n + col[s * n + i]] = val[s * n + i];
-    __syncthreads();
-    for (int k = 0; k < n; k++) {
-        double piv = A[k * n + k];
-        __syncthreads();
-        for (int j = threadIdx.x; j < n; j += blockDim.x) {
-            rowk[j] = (j == k) ? 1.0 / piv : A[k * n + j] / piv;
-            colk[j] = A[j * n + k];
-        }
-        __syncthreads();
-        for (int t = threadIdx.x; t < n * n; t += blockDim.x) {
-            int i = t / n, j = t - i * n;
-            if (i == k) {
-                A[t] = rowk[j];
-            } else {
-                double f = colk[i];
-                A[t] = (j == k) ? -f * rowk[k] : A[t] - f * rowk[j];
-            }
-        }
-        __syncthreads();
-    }
-    for (int t = threadIdx.x; t < n * n; t += blockDim.x) inv[t] = A[t];
-}
-
-// coarse[c] = fine[c2f[c]]: nodal values injected from the finest level.
-__global__ void k_inject(int nc, const int *__restrict__ c2f, const double *__restrict__ fine,
-                         double *__restrict__ coarse)
-{
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += gridDim.x * blockDim.x) coarse[c] = fine[c2f[c]];
 }
 
 // --------------------------------------------------------------- level ops
