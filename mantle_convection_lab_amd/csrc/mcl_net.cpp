@@ -33,6 +33,13 @@ struct ConvShape {
     int cs_in, ci_off;
     int cs_out, co_off;
 };
+struct NetLayer {
+    int off, nw, nb, Cin;
+    uint16_t *Wf, *Wd;
+};
+struct NetLayers {
+    NetLayer l[15];
+};
 __global__ void k_conv3_fwd(ConvShape s, const uint16_t *in, const uint16_t *Wf, const float *bias, uint16_t *out,
                             int relu);
 __global__ void k_conv3_dgrad(ConvShape s, const uint16_t *dout, const uint16_t *act, const uint16_t *Wd,
@@ -58,9 +65,9 @@ __global__ void k_up_bwd(int B, int H, int W, int C, const uint16_t *dout, int c
 __global__ void k_head_fwd(int M, const uint16_t *x, int cs, const float *Wh, const float *bh, float *y);
 __global__ void k_head_bwd(int M, const uint16_t *x, int cs, const float *Wh, const float *y, const float *tgt,
                            float scale, uint16_t *dx, float *dWh, float *dbh, float *loss);
-__global__ void k_adam(int n, float *w, const float *g, float *m1, float *m2, float lr, float b1, float b2, float eps,
-                       float c1, float c2);
-__global__ void k_weights_bf16(int Cout, int Cin, const float *w, uint16_t *Wf, uint16_t *Wd);
+template <bool STEP>
+__global__ void k_update_weights(NetLayers ls, float *w, const float *g, float *m1, float *m2, float lr, float b1,
+                                 float b2, float eps, float c1, float c2);
 __global__ void k_f32_to_bf16(size_t n, const float *x, uint16_t *y);
 __global__ void k_bf16_to_f32(size_t n, const uint16_t *x, float *y);
 
@@ -74,8 +81,7 @@ struct Act {           // one NHWC bf16 activation buffer and its gradient
 struct Conv {          // one 3x3 convolution layer
     int Cin = 0, Cout = 0;
     size_t nw = 0;     // Cout*9*Cin
-    float *w = nullptr, *b = nullptr, *dw = nullptr, *db = nullptr;
-    float *m1 = nullptr, *m2 = nullptr, *bm1 = nullptr, *bm2 = nullptr;
+    float *w = nullptr, *b = nullptr, *dw = nullptr, *db = nullptr;   // in mcl_net's params and grads
     uint16_t *Wf = nullptr, *Wd = nullptr;
 };
 
@@ -90,8 +96,14 @@ struct mcl_net {
     Act x0, e1a, cat1, p1, e2a, cat2, p2, e3a, cat3, p3, b1, b2, d3a, d3b, d2a, d2b, d1a, d1b;
     Conv enc1a, enc1b, enc2a, enc2b, enc3a, enc3b, bota, botb, dec3a, dec3b, dec2a, dec2b, dec1a, dec1b;
     // head (1x1, 32 -> 3, FP32)
-    float *wh = nullptr, *bh = nullptr, *dwh = nullptr, *dbh = nullptr, *hm1 = nullptr, *hm2 = nullptr,
-          *hbm1 = nullptr, *hbm2 = nullptr;
+    float *wh = nullptr, *bh = nullptr, *dwh = nullptr, *dbh = nullptr;
+    // Parameters, gradients and Adam moments, each one buffer in the flat order
+    // of mcl_net_get_params, so that clearing, reading and updating them is one
+    // call for the network; the loss lies behind the gradients and is cleared
+    // with them.
+    size_t np = 0;
+    float *params = nullptr, *grads = nullptr, *m1 = nullptr, *m2 = nullptr;
+    NetLayers layers{};
     float *y = nullptr, *tgt = nullptr, *xin = nullptr, *loss = nullptr;
     long long adam_t = 0;
     float out_scale[3] = {1.0f, 1.0f, 1.0f};   // per output channel (RMS of the training targets)
@@ -162,20 +174,19 @@ struct Normal {
     }
 };
 
-static int make_conv(mcl_net *n, Conv &c, int Cin, int Cout, std::mt19937_64 &rng)
+// Convolution i, its parameters at offset `off` of the flat order (moved past them).
+static int make_conv(mcl_net *n, int i, Conv &c, int Cin, int Cout, size_t &off)
 {
     c.Cin = Cin;
     c.Cout = Cout;
     c.nw = (size_t)Cout * 9 * Cin;
-    if (nalloc(n, &c.w, c.nw) || nalloc(n, &c.b, Cout) || nalloc(n, &c.dw, c.nw) || nalloc(n, &c.db, Cout) ||
-        nalloc(n, &c.m1, c.nw) || nalloc(n, &c.m2, c.nw) || nalloc(n, &c.bm1, Cout) || nalloc(n, &c.bm2, Cout) ||
-        nalloc(n, &c.Wf, c.nw) || nalloc(n, &c.Wd, c.nw))
-        return MCL_E_DEVICE;
-    // He initialisation for ReLU layers
-    Normal nd(std::sqrt(2.0f / (9.0f * (float)Cin)));
-    std::vector<float> w(c.nw);
-    for (auto &v : w) v = nd(rng);
-    NCHK(hipMemcpy(c.w, w.data(), c.nw * sizeof(float), hipMemcpyHostToDevice));
+    if (nalloc(n, &c.Wf, c.nw) || nalloc(n, &c.Wd, c.nw)) return MCL_E_DEVICE;
+    c.w = n->params + off;
+    c.b = c.w + c.nw;
+    c.dw = n->grads + off;
+    c.db = c.dw + c.nw;
+    n->layers.l[i] = {(int)off, (int)c.nw, Cout, Cin, c.Wf, c.Wd};
+    off += c.nw + Cout;
     return 0;
 }
 
@@ -279,17 +290,21 @@ static void conv_bwd(mcl_net *n, Conv &c, const Act &in, int ci_off, Act &out, i
     if (din) conv_product<true>(n, s, g, in_relu ? x : nullptr, c.Wd, nullptr, in.g, 0);
 }
 
-static void refresh_bf16(mcl_net *n, Conv &c)
-{
-    hipLaunchKernelGGL(k_weights_bf16, dim3(gblocks(c.nw)), dim3(256), 0, n->stream, c.Cout, c.Cin, (const float *)c.w,
-                       c.Wf, c.Wd);
-}
-
 static Conv *convs(mcl_net *n, int i)
 {
     Conv *all[] = {&n->enc1a, &n->enc1b, &n->enc2a, &n->enc2b, &n->enc3a, &n->enc3b, &n->bota,
                    &n->botb,  &n->dec3a, &n->dec3b, &n->dec2a, &n->dec2b, &n->dec1a, &n->dec1b};
     return i < 14 ? all[i] : nullptr;
+}
+
+// One row of workgroups for each layer: 256 of 256 threads cover the largest
+// (590 080 parameters) in nine rounds.
+static const dim3 update_grid(256, 15);
+
+static void weights_bf16(mcl_net *n)
+{
+    hipLaunchKernelGGL(k_update_weights<false>, update_grid, dim3(256), 0, n->stream, n->layers, n->params,
+                       (const float *)nullptr, (float *)nullptr, (float *)nullptr, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
 }
 
 int mcl_net_create(int H, int W, int batch, unsigned long long seed, mcl_net **out)
@@ -323,36 +338,42 @@ int mcl_net_create(int H, int W, int batch, unsigned long long seed, mcl_net **o
     rc |= make_act(n, n->d2b, H / 2, W / 2, 64);
     rc |= make_act(n, n->d1a, H, W, 32);
     rc |= make_act(n, n->d1b, H, W, 32);
-    rc |= make_conv(n, n->enc1a, 16, 32, rng);
-    rc |= make_conv(n, n->enc1b, 32, 32, rng);
-    rc |= make_conv(n, n->enc2a, 32, 64, rng);
-    rc |= make_conv(n, n->enc2b, 64, 64, rng);
-    rc |= make_conv(n, n->enc3a, 64, 128, rng);
-    rc |= make_conv(n, n->enc3b, 128, 128, rng);
-    rc |= make_conv(n, n->bota, 128, 256, rng);
-    rc |= make_conv(n, n->botb, 256, 256, rng);
-    rc |= make_conv(n, n->dec3a, 384, 128, rng);
-    rc |= make_conv(n, n->dec3b, 128, 128, rng);
-    rc |= make_conv(n, n->dec2a, 192, 64, rng);
-    rc |= make_conv(n, n->dec2b, 64, 64, rng);
-    rc |= make_conv(n, n->dec1a, 96, 32, rng);
-    rc |= make_conv(n, n->dec1b, 32, 32, rng);
+    static const int chan[14][2] = {{16, 32}, {32, 32}, {32, 64}, {64, 64}, {64, 128}, {128, 128}, {128, 256},
+                                    {256, 256}, {384, 128}, {128, 128}, {192, 64}, {64, 64}, {96, 32}, {32, 32}};
+    for (auto &c : chan) n->np += (size_t)c[1] * (9 * c[0] + 1);
+    n->np += 3 * 32 + 3;
+    rc |= nalloc(n, &n->params, n->np) | nalloc(n, &n->grads, n->np + 1) | nalloc(n, &n->m1, n->np) |
+          nalloc(n, &n->m2, n->np);
+    size_t off = 0;
+    for (int i = 0; i < 14 && !rc; i++) rc |= make_conv(n, i, *convs(n, i), chan[i][0], chan[i][1], off);
     size_t M = (size_t)batch * H * W;
-    rc |= nalloc(n, &n->wh, 3 * 32) | nalloc(n, &n->bh, 3) | nalloc(n, &n->dwh, 3 * 32) | nalloc(n, &n->dbh, 3);
-    rc |= nalloc(n, &n->hm1, 3 * 32) | nalloc(n, &n->hm2, 3 * 32) | nalloc(n, &n->hbm1, 3) | nalloc(n, &n->hbm2, 3);
-    rc |= nalloc(n, &n->y, 3 * M) | nalloc(n, &n->tgt, 3 * M) | nalloc(n, &n->xin, 2 * M) | nalloc(n, &n->loss, 4);
+    rc |= nalloc(n, &n->y, 3 * M) | nalloc(n, &n->tgt, 3 * M) | nalloc(n, &n->xin, 2 * M);
     if (rc) {
         mcl_net_destroy(n);
         return MCL_E_DEVICE;
     }
+    n->wh = n->params + off;
+    n->bh = n->wh + 3 * 32;
+    n->dwh = n->grads + off;
+    n->dbh = n->dwh + 3 * 32;
+    n->loss = n->grads + n->np;
+    n->layers.l[14] = {(int)off, 0, 3 * 32 + 3, 0, nullptr, nullptr};
+    // He initialisation for the ReLU layers, zero biases
+    std::vector<float> p(n->np, 0.f);
+    off = 0;
+    for (int i = 0; i < 14; i++) {
+        const Conv &c = *convs(n, i);
+        Normal nd(std::sqrt(2.0f / (9.0f * (float)c.Cin)));
+        for (size_t k = 0; k < c.nw; k++) p[off + k] = nd(rng);
+        off += c.nw + c.Cout;
+    }
     Normal nd(std::sqrt(1.0f / 32.0f));
-    std::vector<float> wh(96);
-    for (auto &v : wh) v = nd(rng);
-    if (hipMemcpy(n->wh, wh.data(), 96 * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) {
+    for (int k = 0; k < 96; k++) p[off + k] = nd(rng);
+    if (hipMemcpy(n->params, p.data(), n->np * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) {
         mcl_net_destroy(n);
         return MCL_E_DEVICE;
     }
-    for (int i = 0; i < 14; i++) refresh_bf16(n, *convs(n, i));
+    weights_bf16(n);
     *out = n;
     return 0;
 }
@@ -420,14 +441,7 @@ static void forward(mcl_net *n)
 
 static void zero_grads(mcl_net *n)
 {
-    for (int i = 0; i < 14; i++) {
-        Conv &c = *convs(n, i);
-        (void)hipMemsetAsync(c.dw, 0, c.nw * sizeof(float), n->stream);
-        (void)hipMemsetAsync(c.db, 0, c.Cout * sizeof(float), n->stream);
-    }
-    (void)hipMemsetAsync(n->dwh, 0, 96 * sizeof(float), n->stream);
-    (void)hipMemsetAsync(n->dbh, 0, 3 * sizeof(float), n->stream);
-    (void)hipMemsetAsync(n->loss, 0, sizeof(float), n->stream);
+    (void)hipMemsetAsync(n->grads, 0, (n->np + 1) * sizeof(float), n->stream);
 }
 
 static void backward(mcl_net *n)
@@ -471,18 +485,8 @@ static void adam_step(mcl_net *n, float lr)
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     n->adam_t++;
     float c1 = 1.0f - std::pow(b1, (float)n->adam_t), c2 = 1.0f - std::pow(b2, (float)n->adam_t);
-    for (int i = 0; i < 14; i++) {
-        Conv &c = *convs(n, i);
-        hipLaunchKernelGGL(k_adam, dim3(gblocks(c.nw)), dim3(256), 0, n->stream, (int)c.nw, c.w, (const float *)c.dw,
-                           c.m1, c.m2, lr, b1, b2, eps, c1, c2);
-        hipLaunchKernelGGL(k_adam, dim3(1), dim3(256), 0, n->stream, c.Cout, c.b, (const float *)c.db, c.bm1, c.bm2,
-                           lr, b1, b2, eps, c1, c2);
-        refresh_bf16(n, c);
-    }
-    hipLaunchKernelGGL(k_adam, dim3(1), dim3(256), 0, n->stream, 96, n->wh, (const float *)n->dwh, n->hm1, n->hm2, lr,
-                       b1, b2, eps, c1, c2);
-    hipLaunchKernelGGL(k_adam, dim3(1), dim3(256), 0, n->stream, 3, n->bh, (const float *)n->dbh, n->hbm1, n->hbm2, lr,
-                       b1, b2, eps, c1, c2);
+    hipLaunchKernelGGL(k_update_weights<true>, update_grid, dim3(256), 0, n->stream, n->layers, n->params,
+                       (const float *)n->grads, n->m1, n->m2, lr, b1, b2, eps, c1, c2);
 }
 
 int mcl_net_forward(mcl_net *n, const float *x_host, float *y_host)
@@ -517,41 +521,17 @@ int mcl_net_train_step(mcl_net *n, const float *x_host, const float *t_host, flo
 
 // Parameters in a flat FP32 vector: for each conv in order w[Cout][3][3][Cin]
 // then b[Cout]; then the head w[3][32], b[3].
-long long mcl_net_num_params(const mcl_net *n)
-{
-    long long s = 0;
-    for (int i = 0; i < 14; i++) {
-        Conv &c = *convs(const_cast<mcl_net *>(n), i);
-        s += (long long)c.nw + c.Cout;
-    }
-    return s + 96 + 3;
-}
+long long mcl_net_num_params(const mcl_net *n) { return (long long)n->np; }
 
 static int copy_params(mcl_net *n, float *host, bool get, bool grads)
 {
-    size_t off = 0;
-    for (int i = 0; i < 14; i++) {
-        Conv &c = *convs(n, i);
-        float *w = grads ? c.dw : c.w, *b = grads ? c.db : c.b;
-        if (get) {
-            NCHK(hipMemcpy(host + off, w, c.nw * sizeof(float), hipMemcpyDeviceToHost));
-            NCHK(hipMemcpy(host + off + c.nw, b, c.Cout * sizeof(float), hipMemcpyDeviceToHost));
-        } else {
-            NCHK(hipMemcpy(w, host + off, c.nw * sizeof(float), hipMemcpyHostToDevice));
-            NCHK(hipMemcpy(b, host + off + c.nw, c.Cout * sizeof(float), hipMemcpyHostToDevice));
-        }
-        off += c.nw + c.Cout;
-    }
-    float *wh = grads ? n->dwh : n->wh, *bh = grads ? n->dbh : n->bh;
     if (get) {
-        NCHK(hipMemcpy(host + off, wh, 96 * sizeof(float), hipMemcpyDeviceToHost));
-        NCHK(hipMemcpy(host + off + 96, bh, 3 * sizeof(float), hipMemcpyDeviceToHost));
-    } else {
-        NCHK(hipMemcpy(wh, host + off, 96 * sizeof(float), hipMemcpyHostToDevice));
-        NCHK(hipMemcpy(bh, host + off + 96, 3 * sizeof(float), hipMemcpyHostToDevice));
-        for (int i = 0; i < 14; i++) refresh_bf16(n, *convs(n, i));
-        NCHK(hipStreamSynchronize(n->stream));
+        NCHK(hipMemcpy(host, grads ? n->grads : n->params, n->np * sizeof(float), hipMemcpyDeviceToHost));
+        return 0;
     }
+    NCHK(hipMemcpy(n->params, host, n->np * sizeof(float), hipMemcpyHostToDevice));
+    weights_bf16(n);
+    NCHK(hipStreamSynchronize(n->stream));
     return 0;
 }
 

@@ -39,6 +39,15 @@ struct ConvShape {
     int cs_out, co_off;   // channel stride / offset of the output buffer
 };
 
+struct NetLayer {
+    int off, nw, nb;      // first parameter in the flat order, 3x3 weights, parameters after them (biases, the head)
+    int Cin;
+    uint16_t *Wf, *Wd;    // bf16 weights of a 3x3 layer
+};
+struct NetLayers {
+    NetLayer l[15];       // 14 convolutions, the head
+};
+
 // Load 4 consecutive bf16 channels (8-byte aligned) or zeros.
 __device__ __forceinline__ s4 load4(const uint16_t *p, bool valid)
 {
@@ -281,7 +290,7 @@ __global__ void __launch_bounds__(64 * WX * WY)
 }
 
 // The variants: large tiles where they fill the device, small ones where a
-// layer has few pixels (see conv_tile in mcl_net.cpp).
+// layer has few pixels (see conv_product in mcl_net.cpp).
 #define CONV3_TILE(MR, NB, WX, WY)                                                                              \
     template __global__ void k_conv3_tile<MR, NB, WX, WY, false>(ConvShape, const uint16_t *, const uint16_t *, \
                                                                  const uint16_t *, const float *, uint16_t *, int); \
@@ -873,31 +882,40 @@ __global__ void __launch_bounds__(256) k_head_bwd(int M, const uint16_t *__restr
 
 // ----------------------------------------------------------------- Adam etc.
 // Adam (Kingma & Ba 2015) on FP32 master weights; refreshes the bf16 copies.
-__global__ void k_adam(int n, float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m1,
-                       float *__restrict__ m2, float lr, float b1, float b2, float eps, float c1, float c2)
+// Adam step (STEP) and the bf16 weights of every layer from the FP32 masters
+// [co][tap][ci]: Wf ([co][tap][ci]) and Wd ([ci][tap][co]).  blockIdx.y is the
+// layer.  Bound by its launch: 7.8 MB of masters, moments and gradients a
+// buffer, where one launch a tensor for each of the two took 44.
+template <bool STEP>
+__global__ void __launch_bounds__(256)
+k_update_weights(NetLayers ls, float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m1,
+                 float *__restrict__ m2, float lr, float b1, float b2, float eps, float c1, float c2)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        float gi = g[i];
-        float a = b1 * m1[i] + (1.f - b1) * gi;
-        float b = b2 * m2[i] + (1.f - b2) * gi * gi;
-        m1[i] = a;
-        m2[i] = b;
-        w[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+    const NetLayer l = ls.l[blockIdx.y];
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < l.nw + l.nb; i += gridDim.x * blockDim.x) {
+        const int j = l.off + i;
+        float wi = w[j];
+        if (STEP) {
+            float gi = g[j];
+            float a = b1 * m1[j] + (1.f - b1) * gi;
+            float b = b2 * m2[j] + (1.f - b2) * gi * gi;
+            m1[j] = a;
+            m2[j] = b;
+            wi -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+            w[j] = wi;
+        }
+        if (i < l.nw) {
+            const int ci = i % l.Cin, tap = (i / l.Cin) % 9, co = i / (9 * l.Cin);
+            const uint16_t v = f2bf(wi);
+            l.Wf[i] = v;
+            l.Wd[((size_t)ci * 9 + tap) * l.nb + co] = v;
+        }
     }
 }
-
-// Wf (bf16, [co][tap][ci]) and Wd (bf16, [ci][tap][co]) from the FP32 master [co][tap][ci].
-__global__ void k_weights_bf16(int Cout, int Cin, const float *__restrict__ w, uint16_t *__restrict__ Wf,
-                               uint16_t *__restrict__ Wd)
-{
-    int n = Cout * 9 * Cin;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        int ci = i % Cin, tap = (i / Cin) % 9, co = i / (9 * Cin);
-        uint16_t v = f2bf(w[i]);
-        Wf[i] = v;
-        Wd[((size_t)ci * 9 + tap) * Cout + co] = v;
-    }
-}
+template __global__ void k_update_weights<true>(NetLayers, float *, const float *, float *, float *, float, float,
+                                                float, float, float, float);
+template __global__ void k_update_weights<false>(NetLayers, float *, const float *, float *, float *, float, float,
+                                                 float, float, float, float);
 
 __global__ void k_f32_to_bf16(size_t n, const float *__restrict__ x, uint16_t *__restrict__ y)
 {
