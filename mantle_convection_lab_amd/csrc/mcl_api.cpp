@@ -370,39 +370,46 @@ static int build_level(mcl_ctx *c, const mcl_mesh_view &v, Level &Lv)
             for (int a = 0; a < 4; a++)
                 if (v.lm[(d * 4 + a) * (size_t)nel + e] != v.id[d * nno + ienl[a * (size_t)nel + e]])
                     return fail(c, MCL_E_ARG, "lm inconsistent with id at element %d", e);
-    // velocity row patterns: sorted unique columns over the node's elements
-    std::vector<std::vector<int>> rows(neq);
+    // velocity row patterns: the sorted unique columns over the node's at most
+    // four elements, the same for both equations of a node
+    auto columns = [](int *r, int m) {
+        std::sort(r, r + m);
+        return (int)(std::unique(r, r + m) - r);
+    };
+    std::vector<int> pat_ptr(nno + 1, 0), pat;
+    pat.reserve(18 * (size_t)nno);
     int WK = 0;
-    for (int P = 0; P < neq; P++) {
-        int n = veq_node[P];
-        auto &r = rows[P];
-        for (int k = 0; k < cnt[n]; k++) {
-            int e = p2n_el[k * (size_t)nno + n];
-            for (int q = 0; q < 8; q++) {
-                int Q = v.lm[((q & 1) * 4 + (q >> 1)) * (size_t)nel + e];
-                if (Q >= 0) r.push_back(Q);
+    for (int n = 0; n < nno; n++) {
+        if (v.id[n] >= 0 || v.id[nno + n] >= 0) {
+            int r[32], m = 0;
+            for (int k = 0; k < cnt[n]; k++) {
+                const int e = p2n_el[k * (size_t)nno + n];
+                for (int q = 0; q < 8; q++) {
+                    const int Q = v.lm[q * (size_t)nel + e];
+                    if (Q >= 0) r[m++] = Q;
+                }
             }
+            m = columns(r, m);
+            WK = std::max(WK, m);
+            pat.insert(pat.end(), r, r + m);
         }
-        std::sort(r.begin(), r.end());
-        r.erase(std::unique(r.begin(), r.end()), r.end());
-        WK = std::max<int>(WK, (int)r.size());
+        pat_ptr[n + 1] = (int)pat.size();
     }
     if (WK > 127) return fail(c, MCL_E_ARG, "velocity row too long (%d)", WK);
     std::vector<int> Kcol((size_t)std::max(WK, 1) * std::max(neq, 1), 0), Kncol(std::max(neq, 1), 0);
     std::vector<signed char> Kslot(32 * (size_t)std::max(neq, 1), -1);
     for (int P = 0; P < neq; P++) {
-        auto &r = rows[P];
-        Kncol[P] = (int)r.size();
-        for (size_t s = 0; s < r.size(); s++) Kcol[s * neq + P] = r[s];
-        for (size_t s = r.size(); s < (size_t)WK; s++) Kcol[s * neq + P] = P;  // padding reads x[P] * 0
-        int n = veq_node[P];
+        const int n = veq_node[P], m = pat_ptr[n + 1] - pat_ptr[n];
+        const int *r = pat.data() + pat_ptr[n];
+        Kncol[P] = m;
+        for (int s = 0; s < m; s++) Kcol[s * (size_t)neq + P] = r[s];
+        for (int s = m; s < WK; s++) Kcol[s * (size_t)neq + P] = P;  // padding reads x[P] * 0
         for (int k = 0; k < cnt[n]; k++) {
             int e = p2n_el[k * (size_t)nno + n];
             for (int q = 0; q < 8; q++) {
                 int Q = v.lm[((q & 1) * 4 + (q >> 1)) * (size_t)nel + e];
                 if (Q < 0) continue;
-                int s = (int)(std::lower_bound(r.begin(), r.end(), Q) - r.begin());
-                Kslot[(k * 8 + q) * (size_t)neq + P] = (signed char)s;
+                Kslot[(k * 8 + q) * (size_t)neq + P] = (signed char)(std::lower_bound(r, r + m, Q) - r);
             }
         }
     }
@@ -413,46 +420,50 @@ static int build_level(mcl_ctx *c, const mcl_mesh_view &v, Level &Lv)
     std::vector<int> gt_row(8 * (size_t)nel, -1);
     std::vector<signed char> gt_p(8 * (size_t)nel, 0);
     for (int e = 0; e < nel; e++) {
-        std::vector<std::pair<int, int>> rp;
+        std::pair<int, int> rp[8];
+        int m = 0;
         for (int d = 0; d < 2; d++)
             for (int a = 0; a < 4; a++) {
                 int P = v.lm[(d * 4 + a) * (size_t)nel + e];
-                if (P >= 0) rp.push_back({P, 2 * a + d});
+                if (P >= 0) rp[m++] = {P, 2 * a + d};
             }
-        std::sort(rp.begin(), rp.end());
-        for (size_t t = 0; t < rp.size(); t++) {
+        std::sort(rp, rp + m);
+        for (int t = 0; t < m; t++) {
             gt_row[t * nel + e] = rp[t].first;
             gt_p[t * nel + e] = (signed char)rp[t].second;
         }
     }
     // heat row patterns
-    std::vector<std::vector<int>> hrows(neqT);
+    std::vector<int> hpat_ptr(neqT + 1, 0), hpat;
+    hpat.reserve(9 * (size_t)neqT);
     int WT = 0;
     for (int P = 0; P < neqT; P++) {
-        int n = heq_node[P];
-        auto &r = hrows[P];
+        const int n = heq_node[P];
+        int r[16], m = 0;
         for (int k = 0; k < cnt[n]; k++) {
             int e = p2n_el[k * (size_t)nno + n];
             for (int b = 0; b < 4; b++) {
                 int Q = v.heat_lm[b * (size_t)nel + e];
-                if (Q >= 0) r.push_back(Q);
+                if (Q >= 0) r[m++] = Q;
             }
         }
-        std::sort(r.begin(), r.end());
-        r.erase(std::unique(r.begin(), r.end()), r.end());
-        WT = std::max<int>(WT, (int)r.size());
+        m = columns(r, m);
+        WT = std::max(WT, m);
+        hpat.insert(hpat.end(), r, r + m);
+        hpat_ptr[P + 1] = (int)hpat.size();
     }
     std::vector<int> Tcol((size_t)std::max(WT, 1) * std::max(neqT, 1), 0), Tncol(std::max(neqT, 1), 0),
         Tdiag(std::max(neqT, 1), 0);
     std::vector<signed char> Tslot(16 * (size_t)std::max(neqT, 1), -1);
     for (int P = 0; P < neqT; P++) {
-        auto &r = hrows[P];
-        Tncol[P] = (int)r.size();
-        for (size_t s = 0; s < r.size(); s++) Tcol[s * neqT + P] = r[s];
-        for (size_t s = r.size(); s < (size_t)WT; s++) Tcol[s * neqT + P] = P;
-        auto it = std::lower_bound(r.begin(), r.end(), P);
-        if (it == r.end() || *it != P) return fail(c, MCL_E_ARG, "heat row %d has no diagonal", P);
-        Tdiag[P] = (int)(it - r.begin());
+        const int m = hpat_ptr[P + 1] - hpat_ptr[P];
+        const int *r = hpat.data() + hpat_ptr[P];
+        Tncol[P] = m;
+        for (int s = 0; s < m; s++) Tcol[s * (size_t)neqT + P] = r[s];
+        for (int s = m; s < WT; s++) Tcol[s * (size_t)neqT + P] = P;
+        const int *it = std::lower_bound(r, r + m, P);
+        if (it == r + m || *it != P) return fail(c, MCL_E_ARG, "heat row %d has no diagonal", P);
+        Tdiag[P] = (int)(it - r);
         int n = heq_node[P];
         for (int k = 0; k < cnt[n]; k++) {
             int e = p2n_el[k * (size_t)nno + n];
@@ -460,7 +471,7 @@ static int build_level(mcl_ctx *c, const mcl_mesh_view &v, Level &Lv)
                 int Q = v.heat_lm[b * (size_t)nel + e];
                 if (Q < 0) continue;
                 Tslot[(k * 4 + b) * (size_t)neqT + P] =
-                    (signed char)(std::lower_bound(r.begin(), r.end(), Q) - r.begin());
+                    (signed char)(std::lower_bound(r, r + m, Q) - r);
             }
         }
     }
@@ -831,23 +842,24 @@ static int build_multigrid(mcl_ctx *c)
             mg[k].pn = F.pn;
             mg[k].pcol = F.pcol;
             // restriction = transpose, rows of the coarse level
-            std::vector<std::vector<std::pair<int, float>>> rows(std::max(nc, 1));
-            for (int u = 0; u < nf; u++) {
-                int m = F.interp_n[u];
-                for (int a = 0; a < m; a++) {
-                    int l = F.interp_eq[a * (size_t)nf + u];
-                    if (l >= 0) rows[l].push_back({u, 1.0f / (float)m});
-                }
-            }
-            int rw = 1;
-            for (auto &r : rows) rw = std::max<int>(rw, (int)r.size());
+            std::vector<int> have(std::max(nc, 1), 0);
+            auto each = [&](auto &&f) {
+                for (int u = 0; u < nf; u++)
+                    for (int a = 0; a < F.interp_n[u]; a++) {
+                        const int l = F.interp_eq[a * (size_t)nf + u];
+                        if (l >= 0) f(l, u);
+                    }
+            };
+            each([&](int l, int) { have[l]++; });
+            const int rw = std::max(1, *std::max_element(have.begin(), have.end()));
             std::vector<int> rcol((size_t)rw * std::max(nc, 1), -1);
             std::vector<float> rval((size_t)rw * std::max(nc, 1), 0.f);
-            for (int l = 0; l < nc; l++)
-                for (size_t t = 0; t < rows[l].size(); t++) {
-                    rcol[t * nc + l] = rows[l][t].first;
-                    rval[t * nc + l] = rows[l][t].second;
-                }
+            std::fill(have.begin(), have.end(), 0);
+            each([&](int l, int u) {
+                const size_t at = (size_t)have[l]++ * nc + l;
+                rcol[at] = u;
+                rval[at] = 1.0f / (float)F.interp_n[u];
+            });
             const float *fp;
             if (dev_upload(c, C.owned, &cp, rcol)) return MCL_E_DEVICE;
             C.rcol = (int *)cp;
@@ -1468,9 +1480,10 @@ extern "C" int mcl_velocity_pressure_KGF_matrix(mcl_ctx *c)
 // Workgroups of a persistent solve: one per rows_per_block rows, at most what
 // fits co-resident; the environment variable `knob` (MCL_FP64_BLOCKS for the
 // FP64 Uzawa and heat kernels, MCL_MIXED_BLOCKS for the mixed solve), if set,
-// replaces the count (still capped at co-residency).  The FP64 solvers take two rows per thread
-// (their phases are grid barriers, whose cost grows with the workgroup
-// count); the mixed solve takes at most 128 rows per workgroup (its V-cycle
+// replaces the count (still capped at co-residency).  The FP64 solvers take one
+// row per thread, which keeps the row in registers over the whole solve (an
+// inner iteration at 128x128 8.2 us; two rows a thread, re-read after fenced
+// barriers, 29); the mixed solve takes at most 128 rows per workgroup (its V-cycle
 // waits are mostly point-to-point, and more workgroups keep more loads in
 // flight: at 256x256 and above every CU has one workgroup).
 #define MCL_FP64_ROWS_PER_THREAD 1
@@ -1676,13 +1689,23 @@ static int build_halos(mcl_ctx *c, int nb, Add &add)
     if (fuse_level <= 0) return 0;
     const long long cap = MCL_HALO_LDS;
     std::vector<MgLevelDev> mg = c->mg_host;
-    auto sorted_unique = [](std::vector<int> &v) {
-        std::sort(v.begin(), v.end());
-        v.erase(std::unique(v.begin(), v.end()), v.end());
+    // Lists are collected and looked up through a place for every row of the
+    // level (-1: in no list, LISTED: collected, else its local index), taken
+    // back list by list.  (Sorting every column and searching the lists for it
+    // was 85 % of a mesh's set-up.)
+    const int LISTED = -2;
+    auto collect = [&](std::vector<int> &at, std::vector<int> &v, int j) {
+        if (at[j] != -1) return;
+        at[j] = LISTED;
+        v.push_back(j);
     };
-    auto pos = [](const std::vector<int> &v, int j) {
-        auto it = std::lower_bound(v.begin(), v.end(), j);
-        return (it != v.end() && *it == j) ? (int)(it - v.begin()) : -1;
+    auto index = [](std::vector<int> &at, std::vector<int> &v, int first) {
+        std::sort(v.begin(), v.end());
+        for (size_t t = 0; t < v.size(); t++) at[v[t]] = first + (int)t;
+    };
+    auto clear = [](std::vector<int> &at, std::vector<int> &v) {
+        for (int j : v) at[j] = -1;
+        v.clear();
     };
     for (int l = lb + 1; l <= top; l++) {
         MgLevelDev &M = mg[l];
@@ -1712,35 +1735,27 @@ static int build_halos(mcl_ctx *c, int nb, Add &add)
         std::vector<short> rl((size_t)std::max(rw, 1) * std::max(nc, 1), -1);
         bool up1 = true, up2 = fuse_level >= 2, dn1 = coarse_grid && (int)C.rcol_h.size() == rw * nc && nc > 0;
         bool dn2 = dn1 && fuse_level >= 2;
-        std::vector<int> H1, H2, F, Th, Uh;
+        std::vector<int> H1, H2, F, Th, Uh, atV(n, -1), atF(n, -1), atU(n, -1);
         for (int g = 0; g < nb; g++) {
             const int b0 = g * R, e0 = std::min(b0 + R, n);
             auto own = [&](int j) { return j >= b0 && j < e0; };
             // up: H1, H2
-            H1.clear();
+            clear(atV, H1);
+            clear(atV, H2);
             for (int s = 0; s < WK; s++)
                 for (int i = b0; i < e0; i++)
-                    if (!own(kcol(i, s))) H1.push_back(kcol(i, s));
-            sorted_unique(H1);
-            H2.clear();
+                    if (!own(kcol(i, s))) collect(atV, H1, kcol(i, s));
+            index(atV, H1, R);
             for (int s = 0; s < WK; s++)
-                for (int j : H1) {
-                    const int q = kcol(j, s);
-                    if (!own(q) && pos(H1, q) < 0) H2.push_back(q);
-                }
-            sorted_unique(H2);
+                for (int j : H1)
+                    if (!own(kcol(j, s))) collect(atV, H2, kcol(j, s));
+            index(atV, H2, R + (int)H1.size());
             const long long nW = R + (long long)H1.size(), nV = nW + (long long)H2.size();
             if (nW > cap) up1 = false;
             if (nV + nW > cap) up2 = false;
             // local index in V (-1: missing, which the construction excludes;
             // checked so that no LDS index can leave its list)
-            auto locV = [&](int j) {
-                if (own(j)) return j - b0;
-                const int p1 = pos(H1, j);
-                if (p1 >= 0) return R + p1;
-                const int p2 = pos(H2, j);
-                return p2 >= 0 ? R + (int)H1.size() + p2 : -1;
-            };
+            auto locV = [&](int j) { return own(j) ? j - b0 : atV[j]; };
             for (int s = 0; s < 2 * W2; s++)
                 for (int i = b0; i < e0; i++) {
                     const int q = locV(s < WK ? kcol(i, s) : i);
@@ -1776,45 +1791,35 @@ static int build_halos(mcl_ctx *c, int nb, Add &add)
             }
             // down: F, Th, Uh
             const int c0 = g * Rc, c1 = std::min(c0 + Rc, nc);
-            F.clear();
+            clear(atF, F);
             for (int k = 0; k < rw; k++)
                 for (int cc = c0; cc < c1; cc++) {
                     const int u = C.rcol_h[(size_t)k * nc + cc];
-                    if (u >= 0) F.push_back(u);
+                    if (u >= 0) collect(atF, F, u);
                 }
-            sorted_unique(F);
+            index(atF, F, 0);
             if ((long long)F.size() > cap) dn1 = false;
             for (int k = 0; k < rw; k++)
                 for (int cc = c0; cc < c1; cc++) {
                     const int u = C.rcol_h[(size_t)k * nc + cc];
-                    if (u >= 0) rl[(size_t)k * nc + cc] = (short)pos(F, u);
+                    if (u >= 0) rl[(size_t)k * nc + cc] = (short)atF[u];
                 }
-            Th.clear();
+            clear(atU, Th);
+            clear(atU, Uh);
             for (int s = 0; s < WK; s++)
                 for (int u : F)
-                    if (!own(kcol(u, s))) Th.push_back(kcol(u, s));
-            sorted_unique(Th);
-            Uh.clear();
+                    if (!own(kcol(u, s))) collect(atU, Th, kcol(u, s));
+            index(atU, Th, R);
             for (int s = 0; s < WK; s++) {
-                for (int i = b0; i < e0; i++) {
-                    const int q = kcol(i, s);
-                    if (!own(q) && pos(Th, q) < 0) Uh.push_back(q);
-                }
-                for (int j : Th) {
-                    const int q = kcol(j, s);
-                    if (!own(q) && pos(Th, q) < 0) Uh.push_back(q);
-                }
+                for (int i = b0; i < e0; i++)
+                    if (!own(kcol(i, s))) collect(atU, Uh, kcol(i, s));
+                for (int j : Th)
+                    if (!own(kcol(j, s))) collect(atU, Uh, kcol(j, s));
             }
-            sorted_unique(Uh);
+            index(atU, Uh, R + (int)Th.size());
             const long long nT = R + (long long)Th.size(), nU = nT + (long long)Uh.size();
             if (nU + nT + (long long)F.size() > cap) dn2 = false;
-            auto locU = [&](int j) {
-                if (own(j)) return j - b0;
-                const int pt = pos(Th, j);
-                if (pt >= 0) return R + pt;
-                const int pu = pos(Uh, j);
-                return pu >= 0 ? R + (int)Th.size() + pu : -1;
-            };
+            auto locU = [&](int j) { return own(j) ? j - b0 : atU[j]; };
             // mt: T rows (O padded to R, then Th) -> U, pair-major in the block
             const size_t mt0 = mt.size();
             mt.resize(mt0 + (size_t)W2 * nT, 0);
@@ -1843,8 +1848,9 @@ static int build_halos(mcl_ctx *c, int nb, Add &add)
             // down dependencies: the residual reads b and x on F's K columns
             // (one-sweep form); the two-sweep form reads x_1 on U
             for (int u : F) {
-                add(g, u / R);
-                for (int s2 = 0; s2 < WK; s2++) add(g, kcol(u, s2) / R);
+                if (!own(u)) add(g, u / R);
+                for (int s2 = 0; s2 < WK; s2++)
+                    if (!own(kcol(u, s2))) add(g, kcol(u, s2) / R);
             }
             if (dn2)
                 for (int j : Uh) add(g, j / R);
@@ -1903,8 +1909,14 @@ static int build_neighbours(mcl_ctx *c, int nb)
         const int n = A.neq;
         if (n == 0) continue;
         const int R = (n + nb - 1) / nb;
-        for (int s = 0; s < A.WK; s++)
-            for (int i = 0; i < n; i++) add(i / R, A.Kcol_h[(size_t)s * n + i] / R);
+        for (int g = 0; g < nb; g++) {
+            const int b0 = g * R, e0 = std::min(b0 + R, n);
+            for (int s = 0; s < A.WK; s++)
+                for (int i = b0; i < e0; i++) {
+                    const int q = A.Kcol_h[(size_t)s * n + i];
+                    if (q < b0 || q >= e0) add(g, q / R);
+                }
+        }
         if (l - 1 > lb) {
             Level &C = c->levels[l - 1];
             const int Rc = (C.neq + nb - 1) / nb;
