@@ -40,6 +40,7 @@ struct Level {
     int WK = 0, WT = 0;
     double Llast0 = 0, Llast1 = 0, diff_dt = 0;
     LevelDev dev{};
+    int win_v = 0, win_t = 0;                 // widest window of MCL_BLOCK consecutive rows (velocity, temperature)
     // device fields
     double *T = nullptr, *vis = nullptr, *buoy = nullptr, *V = nullptr, *d = nullptr, *p = nullptr;
     double *stress = nullptr, *es = nullptr, *area = nullptr, *avg = nullptr;
@@ -396,6 +397,26 @@ static int build_level(mcl_ctx *c, const mcl_mesh_view &v, Level &Lv)
         pat_ptr[n + 1] = (int)pat.size();
     }
     if (WK > 127) return fail(c, MCL_E_ARG, "velocity row too long (%d)", WK);
+    // vector entries that MCL_BLOCK consecutive rows (a workgroup's) span,
+    // themselves included: the most of any
+    auto widest = [](int n, auto first, auto last) {
+        int most = 0;
+        for (int b = 0; b < n; b += MCL_BLOCK) {
+            int lo = b, hi = b;
+            for (int i = b; i < std::min(b + MCL_BLOCK, n); i++) {
+                lo = std::min(lo, std::min(i, first(i)));
+                hi = std::max(hi, std::max(i, last(i)));
+            }
+            most = std::max(most, hi - lo + 1);
+        }
+        return most;
+    };
+    // (a row without columns spans itself)
+    auto pat_end = [&](const std::vector<int> &ptr, const std::vector<int> &p, int r, int i, bool back) {
+        return ptr[r] == ptr[r + 1] ? i : p[back ? ptr[r + 1] - 1 : ptr[r]];
+    };
+    Lv.win_v = widest(neq, [&](int i) { return pat_end(pat_ptr, pat, veq_node[i], i, false); },
+                      [&](int i) { return pat_end(pat_ptr, pat, veq_node[i], i, true); });
     std::vector<int> Kcol((size_t)std::max(WK, 1) * std::max(neq, 1), 0), Kncol(std::max(neq, 1), 0);
     std::vector<signed char> Kslot(32 * (size_t)std::max(neq, 1), -1);
     for (int P = 0; P < neq; P++) {
@@ -452,6 +473,8 @@ static int build_level(mcl_ctx *c, const mcl_mesh_view &v, Level &Lv)
         hpat.insert(hpat.end(), r, r + m);
         hpat_ptr[P + 1] = (int)hpat.size();
     }
+    Lv.win_t = widest(neqT, [&](int i) { return pat_end(hpat_ptr, hpat, i, i, false); },
+                      [&](int i) { return pat_end(hpat_ptr, hpat, i, i, true); });
     std::vector<int> Tcol((size_t)std::max(WT, 1) * std::max(neqT, 1), 0), Tncol(std::max(neqT, 1), 0),
         Tdiag(std::max(neqT, 1), 0);
     std::vector<signed char> Tslot(16 * (size_t)std::max(neqT, 1), -1);
@@ -1561,6 +1584,16 @@ static int reset_sync_if_aborted(mcl_ctx *c, const DevStats &st, const SolveWork
     return 0;
 }
 
+// Whether a solve over n rows of `slots` slots keeps one row a thread in
+// registers (at most `held` slots) with its vector in the LDS window.  One
+// answer for the grid, from its widest window: the two forms wait differently
+// where there are hanging nodes, and in a tall box (16 x 3072) some workgroups'
+// windows fit and some do not.
+static int rows_fit(int n, int slots, int held, int window, unsigned nblocks)
+{
+    return slots <= held && n <= (long long)nblocks * MCL_BLOCK && window <= MCL_WINDOW;
+}
+
 // Uzawa kernel parameters for the finest level's (d, p) and the work space.
 static UzawaParams uzawa_params(mcl_ctx *c, double accuracy, const SolveWork &W)
 {
@@ -1611,6 +1644,7 @@ static UzawaParams uzawa_params(mcl_ctx *c, double accuracy, const SolveWork &W)
     // Gauss-Seidel sweeps and the multigrid V-cycle are sequential in the
     // row order: the whole solve runs in one workgroup
     if (k.solver == MCL_SOLVER_GS || k.solver == MCL_SOLVER_MG) P.gs.nblocks = 1;
+    P.rows_fit = rows_fit(L.neq, L.WK, MCL_ROW_V, L.win_v, P.gs.nblocks);
     return P;
 }
 
@@ -2321,6 +2355,7 @@ static int heat_enqueue(mcl_ctx *c, EnqMode mode, EventPair *ev)
     H.cg_precondition = k.cg_precondition;
     H.exact_dots = k.exact_dots;
     H.gs.nblocks = coop_blocks(c, std::max(L.neqT, L.nel), MCL_FP64_ROWS_PER_THREAD * MCL_BLOCK, "MCL_FP64_BLOCKS");
+    H.rows_fit = rows_fit(L.neqT, L.WT, MCL_ROW_T, L.win_t, H.gs.nblocks);
     if (ev) HIPCHK(c, hipEventRecord(ev->a, c->stream));
     void *args[] = {&H};
     HIPCHK(c, launch_persistent(c, (const void *)k_heat_fp64, H.gs.nblocks, args, mode == ENQ_GRAPH));

@@ -505,7 +505,7 @@ __device__ __forceinline__ int pcg_persistent(const LevelDev &L, const EllMat &A
 // sweep at 32x32 takes 2.4 us (14.5 us with a fenced barrier, its maxima
 // collected in a second pass and every column's load waiting for the last).
 // The caller's x must be complete; it is complete on return.
-__device__ __forceinline__ int jacobi_grid(const EllMat &A, const RowReg<18> &row, const Window &win, double diag,
+__device__ __forceinline__ int jacobi_grid(const EllMat &A, const RowReg<MCL_ROW_V> &row, const Window &win, double diag,
                                            const double *__restrict__ b, double *x, double *xt, double accu,
                                            int max_cycle, const GridSync &gs, WaitState &ws, bool &ok,
                                            long long &spmv)
@@ -518,7 +518,7 @@ __device__ __forceinline__ int jacobi_grid(const EllMat &A, const RowReg<18> &ro
     if (win.fits && mine) {
         bi = b[gtid];
 #pragma unroll
-        for (int u = 0; u < 18; u++)
+        for (int u = 0; u < MCL_ROW_V; u++)
             if (u < row.n && row.off[u] == 8u * (unsigned)(gtid - win.w0)) dslot = u;
     }
     double *src = x, *dst = xt;
@@ -669,12 +669,12 @@ __device__ int mg_block(const GsLevelDev *lv, int nl, const double *b, double *x
 // that is complete or, with x_zero, just zeroed; x is complete on return.
 template <int SOLVER>
 __device__ __forceinline__ int inner_solve(const UzawaParams &P, const LevelDev &L, const EllMat &K,
-                                           const RowReg<18> &row, const Window &win, double diag, const double *b,
+                                           const RowReg<MCL_ROW_V> &row, const Window &win, double diag, const double *b,
                                            double *x, bool x_zero, CgVecs cv, WaitState &ws, double *ldsm, bool &ok,
                                            long long &spmv)
 {
     if constexpr (SOLVER == MCL_INNER_CG) {
-        return pcg_persistent<18>(L, K, row, win, diag, b, x, x_zero, P.accuracy, P.max_cg_cycle, P.cg_precondition, 0,
+        return pcg_persistent<MCL_ROW_V>(L, K, row, win, diag, b, x, x_zero, P.accuracy, P.max_cg_cycle, P.cg_precondition, 0,
                                   cv, P.gs, ws, ok, spmv, P.exact_dots != 0);
     } else if constexpr (SOLVER == MCL_INNER_JC) {
         if (x_zero) ok = ok && grid_wait(P.gs, ws);
@@ -711,14 +711,14 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_uzawa_fp64(UzawaParams P)
     WaitState ws;
     bool ok = sync_begin(P.gs, ws);
     long long spmv = 0, inner = 0;
-    EllMat K{L.Kcol, L.Kncol, L.Kval, L.Kdiag, nullptr, neq, L.WK};
+    EllMat K{L.Kcol, L.Kncol, L.Kval, L.Kdiag, nullptr, neq};
     CgVecs cv{P.cg_r, P.cg_s, P.cg_d, P.cg_q, P.cg_d2};
-    RowReg<18> row;
+    RowReg<MCL_ROW_V> row;
     Window win{nullptr, 0, 0, false};
     double diag = 1.0;
     if constexpr (SOLVER == MCL_INNER_CG || SOLVER == MCL_INNER_JC) {
         __shared__ double buf[MCL_WINDOW];
-        win = row_window(row, K.col, K.ncol, K.val, K.width, neq, buf);
+        win = row_window(row, K.col, K.ncol, K.val, neq, buf, P.rows_fit != 0);
         if (gtid < neq) diag = K.diag[gtid];
     }
     for (int e = gtid; e < nel; e += gsize) P.BAB[e] = bab_elem(L, e);
@@ -1113,19 +1113,19 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_heat_fp64(HeatParams H)
     // the waits are those of the vectors that the products gather
     for (int P = gtid; P < n; P += gsize)
         heat_assemble_row(L, H, S, P, lds + threadIdx.x, lds + MCL_HEAT_LDS_SLOTS * MCL_BLOCK + threadIdx.x);
-    EllMat Ch{L.Tcol, L.Tncol, H.hC, nullptr, L.Tdiag_slot, n, L.WT};
-    EllMat Ah{L.Tcol, L.Tncol, H.hA, nullptr, L.Tdiag_slot, n, L.WT};
+    EllMat Ch{L.Tcol, L.Tncol, H.hC, nullptr, L.Tdiag_slot, n};
+    EllMat Ah{L.Tcol, L.Tncol, H.hA, nullptr, L.Tdiag_slot, n};
     CgVecs cv{H.cg_r, H.cg_s, H.cg_d, H.cg_q, H.cg_d2};
     auto hd = [&](int j) { return ald(H.hd + j); };
     // one of the two matrices at a time in registers; the LDS columns of the
     // assembly become the window
     static_assert(2 * MCL_HEAT_LDS_SLOTS * MCL_BLOCK >= MCL_WINDOW, "the window lies in the assembly's LDS");
-    RowReg<9> row;
+    RowReg<MCL_ROW_T> row;
     auto cg = [&](const EllMat &A, double *x, bool x_zero, int max_cycle) __attribute__((always_inline)) {
         __syncthreads();
-        const Window win = row_window(row, A.col, A.ncol, A.val, A.width, n, lds);
+        const Window win = row_window(row, A.col, A.ncol, A.val, n, lds, H.rows_fit != 0);
         const double diag = gtid < n ? ell_diag(A, gtid) : 1.0;
-        return pcg_persistent<9>(L, A, row, win, diag, H.B, x, x_zero, 1e-3, max_cycle, H.cg_precondition, 1, cv, H.gs,
+        return pcg_persistent<MCL_ROW_T>(L, A, row, win, diag, H.B, x, x_zero, 1e-3, max_cycle, H.cg_precondition, 1, cv, H.gs,
                                  ws, ok, spmv, H.exact_dots != 0);
     };
     int init_cycles = 0;

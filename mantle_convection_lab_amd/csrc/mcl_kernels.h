@@ -101,6 +101,12 @@ struct GsLevelDev {
 #define MCL_INNER_CG 2
 #define MCL_INNER_MG 3
 
+// One row a thread (mcl_ops.h): doubles of the LDS window, and the slots of a
+// velocity and of a temperature row that registers hold.
+#define MCL_WINDOW 6144
+#define MCL_ROW_V 18
+#define MCL_ROW_T 9
+
 struct UzawaParams {
     LevelDev L;
     GridSync gs;
@@ -112,6 +118,7 @@ struct UzawaParams {
     double accuracy, citcom_accu;
     int max_citcom_cycle, max_cg_cycle, cg_precondition, check_v_only, schur;
     int exact_dots;          // dot products in the reference's sequential order
+    int rows_fit;            // one row a thread, its vector through the LDS window (all workgroups)
     // inner solver (MCL_INNER_*): Jacobi runs on the whole grid; Gauss-Seidel
     // and multigrid need a launch of one workgroup
     int solver, mg_cycle, mg_finest_iteration, mg_coarse_iteration;
@@ -131,6 +138,7 @@ struct HeatParams {
     double *model_time;
     double accuracy, theta, Q, Llast0, Llast1, diff_dt;
     int first_call, cg_precondition;
+    int rows_fit;            // as UzawaParams
     int exact_dots;
 };
 

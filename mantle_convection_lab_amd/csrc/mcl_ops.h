@@ -72,8 +72,8 @@ __device__ __forceinline__ double ell_row(const int *__restrict__ col, const dou
 // lines), which is read once, in order, into LDS; the row itself -- offsets
 // into the window and values -- stays in registers over the whole solve.
 // Gathering through agent-scope loads instead moves every entry up to 18 times
-// past the L2.
-#define MCL_WINDOW 6144   // doubles of LDS
+// past the L2.  Both forms of a solve pass different waits, so all workgroups
+// take the same one: the host decides (fits) from the widest window of the mesh.
 struct Window {
     double *buf;    // LDS
     int w0, n;      // vector entries [w0, w0 + n)
@@ -117,17 +117,17 @@ struct RowReg {
     }
 };
 
-// This thread's row of a matrix (row < rows: col, val slot-major, wk slots)
-// and the workgroup's window; fits = false: more slots than W, more rows than
-// threads, or a wider window than the LDS holds.
+// This thread's row of a matrix (row < rows: col, val slot-major) and the
+// workgroup's window.  fits = false (more slots than W, more rows than threads,
+// or a window of some workgroup wider than the LDS buffer): neither is used.
 template <int W>
 __device__ __forceinline__ Window row_window(RowReg<W> &r, const int *__restrict__ col, const int *__restrict__ ncol,
-                                             const double *__restrict__ val, int wk, int rows, double *buf)
+                                             const double *__restrict__ val, int rows, double *buf, bool fits)
 {
     __shared__ int lo, hi;
     const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    Window w{buf, 0, 0, wk <= W && rows <= (int)(gridDim.x * blockDim.x)};
-    if (!w.fits) return w;
+    Window w{buf, 0, 0, fits};
+    if (!fits) return w;
     if (threadIdx.x == 0) {
         lo = 0x7fffffff;
         hi = -1;
@@ -151,7 +151,6 @@ __device__ __forceinline__ Window row_window(RowReg<W> &r, const int *__restrict
     __syncthreads();
     w.w0 = hi < 0 ? 0 : lo;
     w.n = hi < 0 ? 0 : hi - lo + 1;
-    w.fits = w.n <= MCL_WINDOW;
 #pragma unroll
     for (int u = 0; u < W; u++) r.off[u] = 8u * (unsigned)(u < r.n ? c[u] - w.w0 : 0);
     return w;
@@ -294,7 +293,7 @@ struct EllMat {
     const double *val;
     const double *diag;      // diagonal values, or NULL to use diag_slot
     const int *diag_slot;
-    int n, width;            // rows; slots per row
+    int n;                   // rows
 };
 
 __device__ __forceinline__ double ell_diag(const EllMat &A, int i)
