@@ -339,8 +339,10 @@ static int build_level(mcl_ctx *c, const mcl_mesh_view &v, Level &Lv)
         }
     }
     Lv.ienl = ienl;
-    // node -> elements (ascending), corner index
-    std::vector<int> cnt(nno, 0), p2n_el(4 * (size_t)nno, -1), p2n_a(4 * (size_t)nno, -1);
+    // node -> elements (ascending), corner index; element 0, corner 0 where a
+    // node has none (k_assemble_K loads a first element before it looks at the
+    // count)
+    std::vector<int> cnt(nno, 0), p2n_el(4 * (size_t)nno, 0), p2n_a(4 * (size_t)nno, 0);
     for (int e = 0; e < nel; e++)
         for (int a = 0; a < 4; a++) {
             int n = ienl[a * (size_t)nel + e];

@@ -144,7 +144,7 @@ __device__ __forceinline__ Window row_window(RowReg<W> &r, const int *__restrict
             h = max(h, c[u]);
         }
     }
-    if (r.n > 0) {
+    if (row < rows) {
         atomicMin(&lo, min(l, row));
         atomicMax(&hi, max(h, row));
     }
