@@ -1076,23 +1076,19 @@ static int build_stationary(mcl_ctx *c)
     return 0;
 }
 
-extern "C" int mcl_mesh_upload(mcl_ctx *c, const mcl_mesh_view *levels, int nlev)
+static void drop_levels(mcl_ctx *c)
 {
-    if (!c) return MCL_E_ARG;
-    if (!levels || nlev <= 0 || nlev > MCL_MAX_LEVELS) return fail(c, MCL_E_ARG, "bad level list");
-    HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     for (auto &L : c->levels) free_all(L.owned);
     c->levels.clear();
+    c->nlev = 0;
+}
+
+static int upload_levels(mcl_ctx *c, const mcl_mesh_view *levels, int nlev)
+{
     c->levels.resize(nlev);
     for (int l = 0; l < nlev; l++) {
         int rc = build_level(c, levels[l], c->levels[l]);
-        if (rc) {
-            for (auto &L : c->levels) free_all(L.owned);
-            c->levels.clear();
-            c->nlev = 0;
-            return rc;
-        }
+        if (rc) return rc;
     }
     c->nlev = nlev;
     {
@@ -1255,6 +1251,21 @@ extern "C" int mcl_mesh_upload(mcl_ctx *c, const mcl_mesh_view *levels, int nlev
     c->first_heat = true;
     c->been_here_dp = false;
     return 0;
+}
+
+// After a failure at any point the context has no mesh: the tables over all
+// levels (assembly, fields, preparation) would still be those of the levels
+// that were freed.
+extern "C" int mcl_mesh_upload(mcl_ctx *c, const mcl_mesh_view *levels, int nlev)
+{
+    if (!c) return MCL_E_ARG;
+    if (!levels || nlev <= 0 || nlev > MCL_MAX_LEVELS) return fail(c, MCL_E_ARG, "bad level list");
+    HIPCHK(c, hipSetDevice(c->device));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    drop_levels(c);
+    int rc = upload_levels(c, levels, nlev);
+    if (rc) drop_levels(c);
+    return rc;
 }
 
 extern "C" int mcl_set_control(mcl_ctx *c, const mcl_control *ctl)

@@ -54,3 +54,40 @@ def test_equation_at_a_node_without_elements():
     with pytest.raises(MclError, match="NaN"):
         c.solve_velocity_pressure()
     c.close()
+
+
+def test_no_mesh_after_a_failed_upload():
+    """A list of levels that do not nest is refused once its levels are built;
+    the context then has no mesh, not the tables of the one before, and takes
+    the next upload."""
+    from mantle_convection_lab_amd import Model
+    from mantle_convection_lab_amd import _native as N
+    from mantle_convection_lab_amd.model import MclError
+    inp, mesh = _mesh(3)
+    finer = _mesh(4)[1]
+    m, ref = Model(inp, mesh=mesh), Model(inp, mesh=mesh)
+    want = ref.step()
+    c = m.ctx
+    good = mesh.views()
+    bad = (N.MeshView * 2)(finer.views()[finer.nlev - 1], good[mesh.nlev - 1])
+    print("[upload] a coarser level with nodes that the finest has not", flush=True)
+    assert c.L.mcl_mesh_upload(c.h, bad, 2) == 1
+    for call in (c.viscosity, c.buoyancy_force, c.velocity_pressure_KGF_matrix, c.solve_velocity_pressure,
+                 c.update_temperature):
+        with pytest.raises(MclError, match="no mesh"):
+            call()
+    with pytest.raises(MclError):
+        c.get_field(m.finest, "T")
+    m.ctx.close()
+    m = Model(inp, mesh=mesh)
+    c = m.ctx
+    assert c.L.mcl_mesh_upload(c.h, bad, 2) == 1
+    c.upload(good, c.levels)
+    for k in range(mesh.nlev):
+        c.set_field(mesh.level_struct(k).lev, "T", mesh.initial_temperature(k))
+    c.set_model_time(0.0)
+    got = m.step()
+    assert (got["uzawa"], got["inner"]) == (want["uzawa"], want["inner"])
+    assert all(np.array_equal(m.field(f), ref.field(f)) for f in ("D", "P", "T"))
+    m.ctx.close()
+    ref.ctx.close()
