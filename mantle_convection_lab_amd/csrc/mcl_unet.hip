@@ -669,6 +669,110 @@ template __global__ void k_conv3_wgrad_tile<64, 4>(ConvShape, const uint16_t *, 
 template __global__ void k_conv3_wgrad_tile<32, 8>(ConvShape, const uint16_t *, const uint16_t *, float *, float *, int);
 template __global__ void k_conv3_wgrad_tile<32, 4>(ConvShape, const uint16_t *, const uint16_t *, float *, float *, int);
 
+// The same for the levels that k_conv3_wgrad_tile has no tile for: 8 or 16
+// pixels wide, or 32 and 64 with a height that 4 does not divide.  A workgroup
+// owns 64 output channels n, 32 input channels c and all nine taps (waves: 16 n
+// each, 18 tiles of 16 x 16), and sums over tiles_per_split runs of 64 pixels
+// (TH x TW rectangles of one image, as k_conv3_mm).  Per run it stages G
+// transposed (channel-major, 64 pixels a row) and three copies of the X patch
+// shifted by -1, 0, +1 columns, channel-major, so that every operand fragment --
+// 8 consecutive pixels of one channel -- is one 16-byte LDS read; what bounds it
+// is that staging by 2-byte writes.  Requires TW % 8 == 0 (the host checks the
+// shapes).  A training step with these levels on the
+// unstaged kernel and on this one: 64 x 64, batch 32, 3.1 and 1.13 ms; 256 x 64,
+// batch 4, 2.6 and 0.89 ms; 512 x 16, batch 8, 7.1 and 3.0 ms.
+constexpr int WG_XP = 72;   // bf16 words per staged G row (64 pixels + pad)
+
+__global__ void __launch_bounds__(256) k_conv3_wgrad_mm(ConvShape s, const uint16_t *__restrict__ dout,
+                                                        const uint16_t *__restrict__ in, float *__restrict__ dW,
+                                                        float *__restrict__ db, int tiles_per_split)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t gt[64 * WG_XP];
+    __shared__ __attribute__((aligned(16))) uint16_t xs[3 * 32 * 3 * 72];   // largest: TW = 64, TH + 2 = 3
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int TW = s.W < 64 ? s.W : 64, TH = 64 / TW, PR = TH + 2, XP = TW + 8;
+    const int n0 = blockIdx.x * 64, c0 = blockIdx.y * 32;
+    const int ntiles = s.B * s.H * s.W / 64;
+    const int tb = blockIdx.z * tiles_per_split, te = min(ntiles, tb + tiles_per_split);
+    const bool active = n0 + 16 * wave < s.Cout;
+    const bool bias = blockIdx.y == 0;
+    float bsum = 0.f;   // this lane's share of sum_m G[m, n] for n = n0 + 16 wave + lane % 16
+    f4 acc[9][2];
+    for (int t = 0; t < 9; t++)
+        for (int b = 0; b < 2; b++) acc[t][b] = f4{0, 0, 0, 0};
+    const int kq = 8 * (lane >> 4);
+    for (int tile = tb; tile < te; tile++) {
+        const int m0 = tile * 64;
+        const int img = m0 / (s.H * s.W), r0 = m0 - img * s.H * s.W;
+        const int h0 = r0 / s.W, w0 = r0 - h0 * s.W;
+        __syncthreads();   // the previous tile's products are done with the LDS
+        // G^T: 64 pixels x 64 channels (8 channels per 16-byte load)
+        for (int t = threadIdx.x; t < 64 * 8; t += 256) {
+            const int p = t >> 3, q = t & 7, n = n0 + 8 * q;
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (n < s.Cout) v = *(const uint4 *)(dout + (size_t)(m0 + p) * s.cs_out + s.co_off + n);
+            const uint16_t *e = (const uint16_t *)&v;
+#pragma unroll
+            for (int k = 0; k < 8; k++) gt[(8 * q + k) * WG_XP + p] = e[k];
+        }
+        // X patch (PR rows x TW + 2 columns) into the three shifted copies
+        const int pw = TW + 2;
+        for (int t = threadIdx.x; t < PR * pw * 4; t += 256) {
+            const int pp = t >> 2, q = t & 3, c = c0 + 8 * q;
+            const int prow = pp / pw, pcol = pp - prow * pw;
+            const int hh = h0 - 1 + prow, ww = w0 - 1 + pcol;
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (c < s.Cin && hh >= 0 && hh < s.H && ww >= 0 && ww < s.W)
+                v = *(const uint4 *)(in + ((size_t)(img * s.H + hh) * s.W + ww) * s.cs_in + s.ci_off + c);
+            const uint16_t *e = (const uint16_t *)&v;
+            // copy sh holds X at column col + sh - 1 of the tile: col = pcol - sh
+#pragma unroll
+            for (int sh = 0; sh < 3; sh++) {
+                const int col = pcol - sh;
+                if (col < 0 || col >= TW) continue;
+#pragma unroll
+                for (int k = 0; k < 8; k++) xs[((sh * 32 + 8 * q + k) * PR + prow) * XP + col] = e[k];
+            }
+        }
+        __syncthreads();
+        if (!active) continue;
+        for (int kk = 0; kk < 64; kk += 32) {
+            const bf8 A = *(const bf8 *)(gt + (16 * wave + (lane & 15)) * WG_XP + kk + kq);
+            if (bias) {
+                const uint4 a4 = *(const uint4 *)(gt + (16 * wave + (lane & 15)) * WG_XP + kk + kq);
+                const uint16_t *e = (const uint16_t *)&a4;
+#pragma unroll
+                for (int k = 0; k < 8; k++) bsum += bf2f(e[k]);
+            }
+            const int p = kk + kq, py = p / TW, px = p - py * TW;
+            for (int tap = 0; tap < 9; tap++) {
+                const int dh = tap / 3 - 1, sh = tap % 3;
+                for (int b = 0; b < 2; b++) {
+                    const bf8 B = *(const bf8 *)(xs + ((sh * 32 + 16 * b + (lane & 15)) * PR + py + dh + 1) * XP + px);
+                    acc[tap][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[tap][b], 0, 0, 0);
+                }
+            }
+        }
+    }
+    if (!active) return;
+    if (bias) {
+        bsum += __shfl_xor(bsum, 16, 64);
+        bsum += __shfl_xor(bsum, 32, 64);
+        const int n = n0 + 16 * wave + lane;
+        if (lane < 16 && n < s.Cout) atomicAdd(&db[n], bsum);
+    }
+    const int NC = 9 * s.Cin;
+    for (int tap = 0; tap < 9; tap++)
+        for (int b = 0; b < 2; b++) {
+            const int c = c0 + 16 * b + (lane & 15);
+            if (c >= s.Cin) continue;
+            for (int e = 0; e < 4; e++) {
+                const int n = n0 + 16 * wave + (lane >> 4) * 4 + e;
+                if (n < s.Cout) atomicAdd(&dW[(size_t)n * NC + tap * s.Cin + c], acc[tap][b][e]);
+            }
+        }
+}
+
 // db[co] += sum_m dout[m, co]
 __global__ void k_bias_grad(int M, int Cout, int cs, int coff, const uint16_t *__restrict__ dout,
                             float *__restrict__ db)
