@@ -276,7 +276,6 @@ extern "C" int mcl_create(int device, mcl_ctx **out)
     c->gs.abort = sync + 32;
     c->gs.arrive = sync + 64;
     if (dev_alloc(c, c->owned, &c->rb.part, (size_t)MCL_RED_SLOTS * MCL_MAX_WG) ||
-        dev_alloc(c, c->owned, &c->rb.pmax, (size_t)MCL_RED_SLOTS * MCL_MAX_WG) ||
         dev_alloc(c, c->owned, &c->stats, 1) || dev_alloc(c, c->owned, &c->model_time, 1) ||
         dev_alloc(c, c->owned, &c->resid, 4)) {
         free_all(c->owned);
@@ -2174,8 +2173,7 @@ static int solve_enqueue(mcl_ctx *c, const SolveWork &W, EnqMode mode, EventPair
     HIPCHK(c, hipGetLastError());
     hipLaunchKernelGGL(k_residuals, dim3(grid_for(c, L.neq)), dim3(MCL_BLOCK), 0, c->stream, L.dev, W.rb,
                        (const double *)L.d, (const double *)L.p, k.precision == MCL_PREC_MIXED ? 1 : 0);
-    hipLaunchKernelGGL(k_collect3, dim3(1), dim3(MCL_BLOCK), 0, c->stream, W.rb, 12, (int)grid_for(c, L.neq),
-                       W.resid);
+    hipLaunchKernelGGL(k_collect3, dim3(1), dim3(MCL_BLOCK), 0, c->stream, W.rb, (int)grid_for(c, L.neq), W.resid);
     HIPCHK(c, hipGetLastError());
     return 0;
 }
@@ -2225,8 +2223,8 @@ static int solve_run(mcl_ctx *c, mcl_stokes_stats *out, const SolveWork &W, bool
         // Solver.c:41-51: accuracy = citcom_accu * sqrt(F.F / neq)
         hipLaunchKernelGGL(k_residuals, dim3(grid_for(c, L.neq)), dim3(MCL_BLOCK), 0, c->stream, L.dev, W.rb,
                            (const double *)L.d, (const double *)L.p, 0);
-        hipLaunchKernelGGL(k_collect3, dim3(1), dim3(MCL_BLOCK), 0, c->stream, W.rb, 12,
-                           (int)grid_for(c, L.neq), W.resid);
+        hipLaunchKernelGGL(k_collect3, dim3(1), dim3(MCL_BLOCK), 0, c->stream, W.rb, (int)grid_for(c, L.neq),
+                           W.resid);
         double r[3];
         HIPCHK(c, hipMemcpyAsync(r, W.resid, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -2274,7 +2272,7 @@ extern "C" int mcl_solve_velocity_pressure(mcl_ctx *c, mcl_stokes_stats *out)
 // Byte offsets of the allocation-free solve's buffers in the scratch array
 // (each 256-aligned); total = bytes needed.
 struct ScratchLayout {
-    size_t sync, stats, resid, part, pmax, work, total;
+    size_t sync, stats, resid, part, work, total;
 };
 
 static ScratchLayout scratch_layout(size_t nv, size_t np)
@@ -2286,7 +2284,6 @@ static ScratchLayout scratch_layout(size_t nv, size_t np)
     S.stats = o; o = up(o + sizeof(DevStats));
     S.resid = o; o = up(o + 4 * sizeof(double));
     S.part = o; o = up(o + (size_t)MCL_RED_SLOTS * MCL_MAX_WG * sizeof(dd));
-    S.pmax = o; o = up(o + (size_t)MCL_RED_SLOTS * MCL_MAX_WG * sizeof(double));
     S.work = o; o = up(o + (6 * nv + 9 * np) * sizeof(double));
     S.total = o;
     return S;
@@ -2322,7 +2319,6 @@ extern "C" int mcl_solve_velocity_pressure_noalloc(mcl_ctx *c, mcl_stokes_stats 
     W.stats = (DevStats *)(base + S.stats);
     W.resid = (double *)(base + S.resid);
     W.rb.part = (dd *)(base + S.part);
-    W.rb.pmax = (double *)(base + S.pmax);
     W.work = (double *)(base + S.work);
     return solve_run(c, out, W, true);
 }

@@ -12,6 +12,7 @@
 #define MCL_WAVE 64
 #define MCL_MAX_LEVELS 20
 #define MCL_MAX_WG 2048
+#define MCL_RED_SLOTS 3     // sums a launch hands to the next (RedBuf)
 // most workgroups of a persistent kernel (they are all resident at once)
 #define MCL_SYNC_WG 512
 // A line of the synchronisation block: 128 bytes, written by one workgroup
@@ -451,26 +452,25 @@ __device__ __forceinline__ bool grid_sync(const GridSync &gs, WaitState &w)
 // Partial sums between two launches: every workgroup of the first writes its
 // partials, one workgroup of the second reduces them in a fixed order.
 struct RedBuf {
-    dd *part;      // [slot][MCL_MAX_WG]
-    double *pmax;  // [slot][MCL_MAX_WG]
+    dd *part;      // [MCL_RED_SLOTS][MCL_MAX_WG]
 };
 
 template <int NR>
-__device__ __forceinline__ void reduce_publish(const RedBuf &rb, int slot0, dd (&v)[NR],
-                                               dd (*lds)[MCL_BLOCK / MCL_WAVE])
+__device__ __forceinline__ void reduce_publish(const RedBuf &rb, dd (&v)[NR], dd (*lds)[MCL_BLOCK / MCL_WAVE])
 {
+    static_assert(NR <= MCL_RED_SLOTS, "the partials have MCL_RED_SLOTS slots");
     block_reduce_dd<NR>(v, lds);
     if (threadIdx.x == 0)
 #pragma unroll
         for (int r = 0; r < NR; r++) {
-            dd *p = rb.part + (slot0 + r) * MCL_MAX_WG + blockIdx.x;
+            dd *p = rb.part + r * MCL_MAX_WG + blockIdx.x;
             __hip_atomic_store(&p->hi, v[r].hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&p->lo, v[r].lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
 }
 
 template <int NR>
-__device__ __forceinline__ void reduce_collect(const RedBuf &rb, int slot0, int nblocks, double (&out)[NR],
+__device__ __forceinline__ void reduce_collect(const RedBuf &rb, int nblocks, double (&out)[NR],
                                                dd (*lds)[MCL_BLOCK / MCL_WAVE])
 {
     dd v[NR];
@@ -479,7 +479,7 @@ __device__ __forceinline__ void reduce_collect(const RedBuf &rb, int slot0, int 
     for (int b = threadIdx.x; b < nblocks; b += MCL_BLOCK)
 #pragma unroll
         for (int r = 0; r < NR; r++) {
-            const dd *p = rb.part + (slot0 + r) * MCL_MAX_WG + b;
+            const dd *p = rb.part + r * MCL_MAX_WG + b;
             const dd t{__hip_atomic_load(&p->hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
                        __hip_atomic_load(&p->lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
             v[r] = dd_add(v[r], t);

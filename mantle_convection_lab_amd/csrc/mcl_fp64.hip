@@ -943,14 +943,14 @@ __global__ void k_residuals(LevelDev L, RedBuf rb, const double *__restrict__ d,
         double c = gt_elem(L, e, d);
         acc[1] = dd_add_prod(acc[1], c, c);
     }
-    reduce_publish<3>(rb, 12, acc, lds);
+    reduce_publish<3>(rb, acc, lds);
 }
 
-__global__ void k_collect3(RedBuf rb, int slot0, int nblocks, double *out)
+__global__ void k_collect3(RedBuf rb, int nblocks, double *out)
 {
     __shared__ dd lds[MCL_RED_ROWS][MCL_BLOCK / MCL_WAVE];
     double o[3];
-    reduce_collect<3>(rb, slot0, nblocks, o, lds);
+    reduce_collect<3>(rb, nblocks, o, lds);
     if (threadIdx.x == 0)
         for (int r = 0; r < 3; r++) out[r] = o[r];
 }
