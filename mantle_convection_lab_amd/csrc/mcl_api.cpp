@@ -1614,7 +1614,6 @@ static UzawaParams uzawa_params(mcl_ctx *c, double accuracy, const SolveWork &W)
     UzawaParams P{};
     P.L = L.dev;
     P.gs = W.gs;
-    P.rb = W.rb;
     P.stats = W.stats;
     P.d = L.d;
     P.p = L.p;
@@ -2333,7 +2332,6 @@ static int heat_enqueue(mcl_ctx *c, EnqMode mode, EventPair *ev)
     HeatParams H{};
     H.L = L.dev;
     H.gs = c->gs;
-    H.rb = c->rb;
     H.stats = c->stats;
     H.V = L.V;
     H.T = L.T;

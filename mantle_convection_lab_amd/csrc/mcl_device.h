@@ -500,15 +500,3 @@ __device__ __forceinline__ double block_max(double v, double *lds)
     for (int w = 1; w < MCL_BLOCK / MCL_WAVE; w++) t = fmax(t, lds[w]);
     return t;
 }
-
-__device__ __forceinline__ double block_min(double v, double *lds)
-{
-    const int lane = threadIdx.x & (MCL_WAVE - 1), wave = threadIdx.x / MCL_WAVE;
-    for (int m = MCL_WAVE / 2; m > 0; m >>= 1) v = fmin(v, __shfl_xor(v, m, MCL_WAVE));
-    __syncthreads();
-    if (lane == 0) lds[wave] = v;
-    __syncthreads();
-    double t = lds[0];
-    for (int w = 1; w < MCL_BLOCK / MCL_WAVE; w++) t = fmin(t, lds[w]);
-    return t;
-}

@@ -110,7 +110,6 @@ struct GsLevelDev {
 struct UzawaParams {
     LevelDev L;
     GridSync gs;
-    RedBuf rb;
     DevStats *stats;
     double *d, *p, *u1, *Ahv, *Ahp, *BAB;
     double *r0, *r1, *r2, *z0, *z1, *s1, *s2;
@@ -130,7 +129,6 @@ struct UzawaParams {
 struct HeatParams {
     LevelDev L;
     GridSync gs;
-    RedBuf rb;
     DevStats *stats;
     const double *V;
     double *T, *tau, *hK, *hC, *hA, *hF, *hd, *hdd, *d0, *B;

@@ -266,7 +266,8 @@ static void conv_bwd(mcl_net *n, Conv &c, const Act &in, int ci_off, Act &out, i
     const int TW = in.W < 64 ? in.W : 64;
     const bool staged = !conv_direct() && c.Cin % 8 == 0 && in.C % 8 == 0 && ci_off % 8 == 0 && out.C % 8 == 0 &&
                         co_off % 8 == 0;
-    if (staged && in.W % 32 == 0 && in.H % 4 == 0 && c.Cout % 32 == 0) {
+    // (32 output channels: the full-resolution layers, whose height 8 divides)
+    if (staged && in.W % 32 == 0 && c.Cout % 32 == 0 && in.H % (c.Cout % 64 == 0 ? 4 : 8) == 0) {
         // tiles of 32 x 8 pixels (32 x 4 on lower images), about 512
         // workgroups, each summing at least two tiles where there are that many
         const int th = in.H % 8 == 0 ? 8 : 4, tiles = M / (32 * th), nblk = c.Cout % 64 == 0 ? 64 : 32;
@@ -279,8 +280,7 @@ static void conv_bwd(mcl_net *n, Conv &c, const Act &in, int ci_off, Act &out, i
     hipLaunchKernelGGL((k_conv3_wgrad_tile<NBLK, TH>), grid, dim3(256), 0, n->stream, s, g, x, c.dw, c.db, tps)
         if (nblk == 64 && th == 8) WGRAD_TILE(64, 8);
         else if (nblk == 64) WGRAD_TILE(64, 4);
-        else if (th == 8) WGRAD_TILE(32, 8);
-        else WGRAD_TILE(32, 4);
+        else WGRAD_TILE(32, 8);
 #undef WGRAD_TILE
     } else if (staged && TW % 8 == 0 && in.W % TW == 0 && 64 % TW == 0 && in.H % (64 / TW) == 0) {
         // narrow and low levels: workgroups of 64 x 32 x 9 taps, about 512 in

@@ -667,7 +667,6 @@ __global__ void __launch_bounds__(256) k_conv3_wgrad_tile(ConvShape s, const uin
 template __global__ void k_conv3_wgrad_tile<64, 8>(ConvShape, const uint16_t *, const uint16_t *, float *, float *, int);
 template __global__ void k_conv3_wgrad_tile<64, 4>(ConvShape, const uint16_t *, const uint16_t *, float *, float *, int);
 template __global__ void k_conv3_wgrad_tile<32, 8>(ConvShape, const uint16_t *, const uint16_t *, float *, float *, int);
-template __global__ void k_conv3_wgrad_tile<32, 4>(ConvShape, const uint16_t *, const uint16_t *, float *, float *, int);
 
 // The same for the levels that k_conv3_wgrad_tile has no tile for: 8 or 16
 // pixels wide, or 32 and 64 with a height that 4 does not divide.  A workgroup
