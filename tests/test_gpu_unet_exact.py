@@ -79,6 +79,28 @@ def test_gradients_exact_narrow_levels(H, W, B):
     _check(H, W, B)
 
 
+# five tiles in three splits; 32 x 4 tiles below; an odd tile count over many
+# workgroups; three tiles a split at the 64-wide level
+@pytest.mark.parametrize("H,W,B", [(40, 32, 1), (48, 96, 1), (128, 256, 3), (256, 256, 3)])
+def test_gradients_exact_tiles(H, W, B):
+    _check(H, W, B)
+
+
+@pytest.mark.parametrize("H,W,B", [(32, 256, 15), (64, 128, 9), (256, 256, 4)])
+def test_forward_bytes_do_not_depend_on_the_tile(H, W, B):
+    """An image alone takes smaller tiles than in a batch; every output is the
+    same chain of products."""
+    print(f"[gpu-unet-exact] forward {H} x {W}, batch {B} and alone", flush=True)
+    from mantle_convection_lab_amd.learn import Net
+    x = np.random.default_rng(H + W).normal(size=(B, H, W, 2)).astype(np.float32)
+    batch, one = Net(H, W, B, seed=3), Net(H, W, 1, seed=3)
+    y = batch.forward(x)
+    for b in range(B):
+        assert y[b].tobytes() == one.forward(x[b: b + 1])[0].tobytes(), b
+    batch.close()
+    one.close()
+
+
 def _check(H, W, B):
     print(f"[gpu-unet-exact] {H} x {W}, batch {B}", flush=True)
     p, x, t, want = _case(H, W, B)
