@@ -94,13 +94,27 @@ def level_sizes(model):
 
 
 def fp64_bytes(rec, sizes, w=8, iw=4):
-    """Algorithmic bytes of k_uzawa_fp64 for one solve: per inner Jacobi-PCG
-    iteration nnz_K (w+iw) + 11 n_v w; per Uzawa iteration
+    """Algorithmic bytes of the FP64 solve where the matrix streams: per inner
+    Jacobi-PCG iteration nnz_K (w+iw) + 11 n_v w; per Uzawa iteration
     2 nnz_G (w+iw) + 7 n_v w + 12 n_p w with nnz_G = 4 n_v."""
     n_v, nnz, n_p = sizes[-1]
     b_cg = nnz * (w + iw) + 11 * n_v * w
     b_uz = 2 * (4 * n_v) * (w + iw) + 7 * n_v * w + 12 * n_p * w
     return rec["inner"] * b_cg + rec["uzawa"] * b_uz
+
+
+# rows that k_uzawa_fp64 keeps in registers: one a thread, 256 workgroups of 512
+FP64_HELD_ROWS = 256 * 512
+
+
+def fp64_held_bytes(rec, sizes, w=8, iw=4):
+    """Bytes k_uzawa_fp64 cannot do without for one solve where every thread
+    holds its row: K once, nnz_K (w+iw); per inner iteration s and d read, d, x
+    and s written, 5 n_v w (r, q and the row stay with their thread); the Uzawa
+    iterations as in fp64_bytes."""
+    n_v, nnz, _ = sizes[-1]
+    per_uzawa = fp64_bytes(dict(rec, inner=0), sizes, w, iw)
+    return nnz * (w + iw) + rec["inner"] * 5 * n_v * w + per_uzawa
 
 
 def mixed_bytes(rec, sizes, pre=MG_SWEEPS):
@@ -297,7 +311,9 @@ def summary(res, steps):
 
 def roofline(res, kernel):
     recs = res["recs"]
-    fn = fp64_bytes if kernel == "k_uzawa_fp64" else mixed_bytes
+    fn = mixed_bytes
+    if kernel == "k_uzawa_fp64":
+        fn = fp64_held_bytes if res["sizes"][-1][0] <= FP64_HELD_ROWS else fp64_bytes
     bytes_per = [fn(r, res["sizes"]) for r in recs]
     ms = [r["solve_ms"] for r in recs]
     if not ms:
