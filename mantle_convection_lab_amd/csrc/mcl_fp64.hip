@@ -355,6 +355,14 @@ __device__ double seq_dot(const double *__restrict__ x, const double *__restrict
     return res;
 }
 
+// How a conjugate-gradient solve reads the vector of its product, one form for
+// the whole grid (pcg_persistent):
+//   CG_ROWS    one row a thread, the vector through the LDS window (row_window)
+//   CG_GATHER  s + beta d gathered entry by entry with agent-scope loads
+//   CG_CACHED  d stored by its row's thread, a fenced wait, then plain loads,
+//              which the L1 and L2 serve to the rows that share an entry
+enum CgForm { CG_ROWS, CG_GATHER, CG_CACHED };
+
 // Conj_Grad (Solver.c:1589-1797) / Conj_Grad_heat (Update_temperature.c:
 // 1140-1354) inside a persistent kernel.  All workgroups execute the same
 // control flow: the scalars come from the grid waits, identical everywhere.
@@ -366,8 +374,9 @@ __device__ double seq_dot(const double *__restrict__ x, const double *__restrict
 //       wait for x), s = r / diag, with r.s and max |alpha r|
 // s, d and x cross workgroups with agent-scope accesses, so the waits need no
 // cache maintenance and the matrix stays in the L2; r and q belong to the row's
-// thread.
-// ROWS: every thread owns at most one row (row_window): the row, r, q, d and x
+// thread.  (CG_CACHED: one wait more, between d and the product; only d and x
+// cross.)
+// CG_ROWS: every thread owns at most one row (row_window): the row, r, q, d and x
 // stay in registers and the gathered vector comes through the window; what is
 // left of an iteration is the two waits and one round trip of loads.
 // Measured per inner iteration (three fenced barriers, the matrix re-read after
@@ -376,7 +385,7 @@ __device__ double seq_dot(const double *__restrict__ x, const double *__restrict
 // The caller's phase may write b on this thread's rows (grid stride) right
 // before the call; a non-zero x must be complete.  x is complete on return.
 // Returns the iteration count; ok is cleared if a wait gave up.
-template <int W, bool ROWS>
+template <int W, CgForm FORM>
 __device__ __forceinline__ int pcg_rows(const LevelDev &L, const EllMat &A, const RowReg<W> &row, const Window &win,
                                         double diag, const double *__restrict__ b, double *x, bool x_zero, double accu,
                                         int max_cycle, int precond, int kind, CgVecs v, const GridSync &gs,
@@ -384,6 +393,7 @@ __device__ __forceinline__ int pcg_rows(const LevelDev &L, const EllMat &A, cons
 {
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsize = gridDim.x * blockDim.x;
     const int n = A.n;
+    constexpr bool ROWS = FORM == CG_ROWS, cached = FORM == CG_CACHED;
     double rr = 0.0, rq = 0.0, rd = 0.0, rx = 0.0;
     if (ROWS && !x_zero && gtid < n) rx = ald(x + gtid);
     // row i times the vector value(j): the window's entries were filled before
@@ -392,12 +402,19 @@ __device__ __forceinline__ int pcg_rows(const LevelDev &L, const EllMat &A, cons
         else return ell_row_ld(A.col, A.val, A.ncol[i], n, i, value);
     };
     auto xat = [&](int j) { return ald(x + j); };
+    // CG_CACHED: r, s and q are read by their row's thread alone (by all of
+    // them in an exact dot product)
+    auto put = [&](double *p, double y) {
+        if (cached && !exact) *p = y;
+        else ast(p, y);
+    };
+    auto get = [&](const double *p) { return cached && !exact ? *p : ald(p); };
     // r of row i and s = M r, with r.s
     auto residual = [&](int i, double r, dd &acc) {
         const double s = precond ? r / (ROWS ? diag : ell_diag(A, i)) : r;
         if (ROWS) rr = r;
-        if (!ROWS || exact) ast(v.r + i, r);
-        ast(v.s + i, s);
+        if (!ROWS || exact) put(v.r + i, r);
+        put(v.s + i, s);
         acc = dd_add_prod(acc, r, s);
     };
     double delta_new;
@@ -419,14 +436,28 @@ __device__ __forceinline__ int pcg_rows(const LevelDev &L, const EllMat &A, cons
             auto dat = [&](int j) { return cycle == 0 ? ald(v.s + j) : ald(v.s + j) + beta * ald(dold + j); };
             dd acc[1] = {dd_zero()};
             if (ROWS) win.fill(dat);
+            if constexpr (cached) {
+                for (int i = gtid; i < n; i += gsize) {
+                    const double s = get(v.s + i);
+                    dnew[i] = cycle == 0 ? s : s + beta * dold[i];
+                }
+                ok = ok && grid_sync(gs, ws);
+            }
             for (int i = gtid; i < n; i += gsize) {
-                const double d = ROWS ? win.buf[i - win.w0] : dat(i), q = times(i, dat);
-                ast(dnew + i, d);
+                double d, q;
+                if constexpr (cached) {
+                    d = dnew[i];
+                    q = ell_row(A.col, A.val, A.ncol[i], n, i, dnew);
+                } else {
+                    d = ROWS ? win.buf[i - win.w0] : dat(i);
+                    q = times(i, dat);
+                    ast(dnew + i, d);
+                }
                 if (ROWS) {
                     rd = d;
                     rq = q;
                 }
-                if (!ROWS || exact) ast(v.q + i, q);
+                if (!ROWS || exact) put(v.q + i, q);
                 acc[0] = dd_add_prod(acc[0], d, q);
             }
             spmv++;
@@ -436,7 +467,7 @@ __device__ __forceinline__ int pcg_rows(const LevelDev &L, const EllMat &A, cons
         }
         const double alpha = delta_new / t1;
         for (int i = gtid; i < n; i += gsize) {
-            rx = (ROWS ? rx : ald(x + i)) + alpha * (ROWS ? rd : ald(dnew + i));
+            rx = (ROWS ? rx : ald(x + i)) + alpha * (ROWS ? rd : cached ? dnew[i] : ald(dnew + i));
             ast(x + i, rx);
         }
         if (L.nh > 0) {
@@ -458,7 +489,7 @@ __device__ __forceinline__ int pcg_rows(const LevelDev &L, const EllMat &A, cons
             for (int i = gtid; i < n; i += gsize) {
                 double r;
                 if (recompute) r = b[i] - times(i, xat);
-                else r = (ROWS ? rr : ald(v.r + i)) - alpha * (ROWS ? rq : ald(v.q + i));
+                else r = (ROWS ? rr : get(v.r + i)) - alpha * (ROWS ? rq : get(v.q + i));
                 residual(i, r, acc[0]);
                 mx[0] = fmax(mx[0], fabs(alpha * r));
             }
@@ -479,6 +510,13 @@ __device__ __forceinline__ int pcg_rows(const LevelDev &L, const EllMat &A, cons
     return cycle;
 }
 
+// The form of a solve that does not keep its rows (more rows than threads, or
+// hanging nodes).  The fenced wait of CG_CACHED pays once a thread has more than
+// one velocity row of 18 slots, or more than two temperature rows of 9.  us an
+// inner iteration, CG_GATHER / CG_CACHED: 128x128 on 32 workgroups (two rows a
+// thread) 22.8 / 18.1, on 8 74.9 / 46.5, on one 575 / 333; 512x512 on 256 (four
+// rows) 51.0 / 46.0; an adapted mesh of 43 390 equations with one row a thread
+// 20.7 / 21.5; temperature at 512x512 (two rows a thread) 49 / 55.
 template <int W>
 __device__ __forceinline__ int pcg_persistent(const LevelDev &L, const EllMat &A, const RowReg<W> &row,
                                               const Window &win, double diag, const double *__restrict__ b, double *x,
@@ -486,10 +524,13 @@ __device__ __forceinline__ int pcg_persistent(const LevelDev &L, const EllMat &A
                                               const GridSync &gs, WaitState &ws, bool &ok, long long &spmv, bool exact)
 {
     if (win.fits)
-        return pcg_rows<W, true>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws, ok,
-                                 spmv, exact);
-    return pcg_rows<W, false>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws, ok, spmv,
-                              exact);
+        return pcg_rows<W, CG_ROWS>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws, ok,
+                                    spmv, exact);
+    if (A.n <= (kind + 1) * (int)(gridDim.x * blockDim.x))
+        return pcg_rows<W, CG_GATHER>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws,
+                                      ok, spmv, exact);
+    return pcg_rows<W, CG_CACHED>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws, ok,
+                                  spmv, exact);
 }
 
 // ------------------------------------------------ stationary inner solvers
@@ -503,7 +544,9 @@ __device__ __forceinline__ int pcg_persistent(const LevelDev &L, const EllMat &A
 // the wait that ends a sweep carries its maximum.  With one row a thread
 // (row_window) the row stays in registers and x comes through the window: a
 // sweep at 32x32 takes 2.4 us (14.5 us with a fenced barrier, its maxima
-// collected in a second pass and every column's load waiting for the last).
+// collected in a second pass and every column's load waiting for the last);
+// with more rows the loads of nine slots go together (128x128 on 4 workgroups, 16
+// rows a thread: 68 us a sweep, 126 one column after the other).
 // The caller's x must be complete; it is complete on return.
 __device__ __forceinline__ int jacobi_grid(const EllMat &A, const RowReg<MCL_ROW_V> &row, const Window &win, double diag,
                                            const double *__restrict__ b, double *x, double *xt, double accu,
@@ -523,6 +566,32 @@ __device__ __forceinline__ int jacobi_grid(const EllMat &A, const RowReg<MCL_ROW
     }
     double *src = x, *dst = xt;
     int cycle = 0;
+    // this thread's rows of a sweep, their loads issued nine slots at a time
+    auto sweep = [&](double &mx) {
+        for (int i = gtid; i < n; i += gsize) {
+            double prod = 0.0, dg = 1.0;
+            const int nc = A.ncol[i];
+            for (int j = 0; j < nc; j += 9) {
+                int c[9];
+                double v[9], xv[9];
+#pragma unroll
+                for (int u = 0; u < 9; u++) {
+                    c[u] = j + u < nc ? A.col[(j + u) * n + i] : -1;
+                    v[u] = j + u < nc ? A.val[(j + u) * n + i] : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < 9; u++) xv[u] = c[u] >= 0 ? ald(src + c[u]) : 0.0;
+#pragma unroll
+                for (int u = 0; u < 9; u++) {
+                    if (c[u] == i) dg = v[u];
+                    else if (c[u] >= 0) prod += v[u] * xv[u];
+                }
+            }
+            const double xn = (b[i] - prod) / dg;
+            ast(dst + i, xn);
+            mx = fmax(mx, fabs(xn - ald(src + i)));
+        }
+    };
     while (ok && cycle < max_cycle) {
         double mx[1] = {0.0}, o[1] = {0.0};
         if (win.fits) {
@@ -533,19 +602,7 @@ __device__ __forceinline__ int jacobi_grid(const EllMat &A, const RowReg<MCL_ROW
                 mx[0] = fabs(xn - win.buf[gtid - win.w0]);
             }
         } else {
-            for (int i = gtid; i < n; i += gsize) {
-                double prod = 0.0, dg = 1.0;
-                const int nc = A.ncol[i];
-                for (int j = 0; j < nc; j++) {
-                    const int c = A.col[j * n + i];
-                    const double v = A.val[j * n + i];
-                    if (c != i) prod += v * ald(src + c);
-                    else dg = v;
-                }
-                const double xn = (b[i] - prod) / dg;
-                ast(dst + i, xn);
-                mx[0] = fmax(mx[0], fabs(xn - ald(src + i)));
-            }
+            sweep(mx[0]);
         }
         spmv++;
         dd none[1] = {dd_zero()};
