@@ -210,7 +210,7 @@ static void shape_tables(ShapeTables *s)
 
 // ------------------------------------------------------------ static scratch
 // Work space of mcl_solve_velocity_pressure_noalloc: the FP64 Uzawa solve's
-// grid-barrier words, statistics, residual norms, reduction partials and work
+// synchronisation words, statistics, residual norms, their partials and work
 // vectors, in one file-scope device array per GPU (each GPU the library runs
 // on holds its copy until the process ends).  Host code never uses the array's
 // name as an address: each device's copy is located once, with that device
@@ -269,7 +269,7 @@ extern "C" int mcl_create(int device, mcl_ctx **out)
     hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_m, (const void *)k_uzawa_mixed, MCL_BLOCK, 0);
     int per_cu = std::min(std::min(per_cu_u, per_cu_h), per_cu_m);
     c->max_coop_blocks = std::min(std::max(1, per_cu) * c->num_cu, MCL_SYNC_WG);
-    // grid barrier and reduction buffers
+    // synchronisation block and partial sums
     unsigned *sync = nullptr;
     if (dev_alloc(c, c->owned, &sync, MCL_SYNC_WORDS)) { delete c; return MCL_E_DEVICE; }
     c->gs.gen = sync;
@@ -1534,10 +1534,12 @@ static unsigned coop_blocks(mcl_ctx *c, long long n, int rows_per_block, const c
 }
 
 // Device buffers a Stokes solve works in besides the mesh and the fields:
-// grid-barrier words, reduction partials, the kernel's statistics, the
+// synchronisation words, the residuals' partials, the kernel's statistics, the
 // residual norms and the Uzawa / CG work vectors (6 n_v + 9 n_p doubles).
 // The context's own (allocated at set-up), or carved from the static scratch
-// array by the allocation-free solve.
+// array by the allocation-free solve.  Two more vectors of n_v (xt, xt2) are the
+// context's in either case: the second direction buffer of conjugate gradients
+// is one of them.
 struct SolveWork {
     GridSync gs;
     RedBuf rb;
@@ -1571,7 +1573,7 @@ static int zero_async(mcl_ctx *c, void *p, size_t bytes, bool by_kernel)
 // the device's cooperative-launch resources (a second process on the same
 // GPU), and then the same grid is launched plainly: with the CUs free every
 // workgroup is dispatched at once, and a workgroup kept waiting longer than the
-// barriers' spin limit ends the solve with MCL_E_DEVICE instead of a hang.
+// waits' spin limit ends the solve with MCL_E_DEVICE instead of a hang.
 static hipError_t launch_persistent(mcl_ctx *c, const void *fn, unsigned nb, void **args, bool plain = false)
 {
     // a batch's captured graphs launch plainly: their grids are capped so that
@@ -2135,7 +2137,7 @@ static int solve_enqueue(mcl_ctx *c, const SolveWork &W, EnqMode mode, EventPair
     }
     c->been_here_dp = true;
     if (mode == ENQ_NOALLOC) {
-        // barrier words (the kernel starts from generation 0)
+        // synchronisation words (the kernel starts from generation 0)
         rc = zero_async(c, W.gs.gen, MCL_SYNC_WORDS * sizeof(unsigned), true);
         if (rc) return rc;
     }

@@ -14,7 +14,8 @@
 //             ELL products, G p, CG vector updates
 //   elements  BAB, G^T d, pressure-space updates, SUPG tau, element stress
 // The Uzawa solve and the heat step each run as one persistent kernel launched
-// cooperatively; phases are separated by grid barriers (mcl_device.h).
+// cooperatively; its phases are separated by grid-wide waits that carry their
+// reductions (mcl_device.h).
 #include "mcl_kernels.h"
 #include "mcl_ops.h"
 
@@ -61,8 +62,8 @@ __global__ void __launch_bounds__(MCL_BLOCK) k_inject(const FieldLevel *__restri
     if (i < F.nno) F.T[i] = fine[F.c2f[i]];
 }
 
-// Buoyancy.c:3-22 with get_node_horiz_avg (Parallel.c:354-437): one thread per
-// node row k walks the row's contribution list in the reference's order
+// Buoyancy.c:3-22 with get_node_horiz_avg (Parallel.c:354-437): a node row's
+// average is the sum over its contribution list in the reference's order
 // (elements ascending; within an element the interior points, then the top
 // row or right column points, then the corner node).  Each entry adds
 // N_a(xi, eta) * data[node_a] for a = 0..3 separately, as the reference does.

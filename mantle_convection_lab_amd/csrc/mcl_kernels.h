@@ -121,7 +121,11 @@ struct UzawaParams {
     // inner solver (MCL_INNER_*): Jacobi runs on the whole grid; Gauss-Seidel
     // and multigrid need a launch of one workgroup
     int solver, mg_cycle, mg_finest_iteration, mg_coarse_iteration;
-    double *xt, *xt2;        // [n_v] previous iterates (Jacobi ping-pong, sweep and V-cycle differences)
+    // [n_v] each, the context's also where the work space is not: previous
+    // iterates (Jacobi ping-pong, sweep and V-cycle differences); with conjugate
+    // gradients xt is cg_d2, and the mixed solve keeps K v of its constrained
+    // product in xt2
+    double *xt, *xt2;
     const GsLevelDev *gsl;   // [ngsl] levels, coarsest first (device memory)
     int ngsl;
 };
@@ -173,7 +177,7 @@ struct MgLevelDev {
     // The FP32 matrix and every column map hold two slots of a row together
     // (WK2 = (WK + 1) / 2 pairs, [pair][row]; an odd row length is padded with
     // the row itself and 0): half the loads of one slot each, and their address
-    // registers (28 spilled registers before, 10 so; a solve at 32x32 3.81 ms
+    // registers (28 spilled registers before, 7 so; a solve at 32x32 3.81 ms
     // before, 3.72).  Maps into lists of at most 65 535 rows pack a pair into
     // one word.
     int WK2;

@@ -8,8 +8,9 @@
 // reference's interp maps, dense inverse on the coarsest grid); Jacobi when
 // there is a single level.  The preconditioner is symmetric (equal pre- and
 // post-sweeps, R = P^T), so plain CG applies; FP32 only perturbs it.
-// Levels small enough for one workgroup are processed by workgroup 0 alone with
-// workgroup barriers; larger levels use the whole grid and grid barriers.
+// Levels whose matrix fits a workgroup's LDS are processed by every workgroup
+// alike, with workgroup barriers only; larger levels are spread over the grid,
+// whose workgroups wait for their neighbours, and for all at the reductions.
 #include "mcl_kernels.h"
 #include "mcl_ops.h"
 
@@ -17,8 +18,8 @@ typedef float f2v __attribute__((ext_vector_type(2)));
 
 // Optional phase timers (build with -DMCL_PHASE_TIMERS=1): thread 0 of
 // workgroup 0 charges the 100 MHz wall clock since its previous stamp to a
-// phase; grid barriers keep every workgroup in step, so workgroup 0's split
-// is the grid's.  Phases: 0 d'/q pass, 1 x/r update (+ start), 2 V-cycle down
+// phase; the waits keep the workgroups in step, so workgroup 0's split is
+// about the grid's.  Phases: 0 d'/q pass, 1 x/r update (+ start), 2 V-cycle down
 // (grid levels), 7 restriction into the LDS levels, 8 LDS levels down,
 // 9 coarsest solve, 3 LDS levels up, 4 V-cycle up (grid levels), 5 last
 // sweep + r.z, 6 Uzawa outer work.
@@ -360,7 +361,7 @@ __device__ __forceinline__ auto sweep_buf(const LV &A, int k)
 }
 
 // the workgroup's LDS blocks: level descriptors, Gershgorin bounds (both read
-// in every phase, so kept out of the grid barriers' cache invalidations), and
+// in every phase, so kept out of the fenced waits' cache invalidations), and
 // the coarse levels' vectors and matrices
 struct MgLds {
     const MCL_L MgLevelDev *lev;
@@ -1617,7 +1618,7 @@ __device__ __forceinline__ void uzawa_mixed(const MixedParams &P)
 {
     __shared__ __attribute__((aligned(16))) float mg_pool[MCL_MG_POOL];
     // level descriptors and Gershgorin bounds (read in every phase; LDS keeps
-    // them out of the grid barriers' cache invalidations)
+    // them out of the fenced waits' cache invalidations)
     __shared__ MgLevelDev mg_lev[MCL_MG_MAX_LEVELS];
     __shared__ float mg_lam[MCL_MG_MAX_LEVELS];
     __shared__ float mg_halo[MCL_HALO_LDS];

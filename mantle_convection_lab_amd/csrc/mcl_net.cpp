@@ -204,14 +204,14 @@ static bool conv_direct()
 // One 3x3 product of `dg` = false: the forward pass, true: the data gradient.
 // Tiles of whole 16-pixel runs (k_conv3_tile) need a width that is a multiple
 // of 16 and 16-byte aligned pixels of the summed buffer; the tile is the
-// largest that leaves at least a workgroup a CU (the large ones stage less and
-// read less LDS per MFMA; a layer with few pixels is bound by the latency of
-// its chunks, which only more workgroups hide).  A forward pass of 15 images of
-// 32 x 256 takes 362 us with that line at one workgroup a CU, 371 at two, 384
-// at four; the 14 products of one 256 x 256 image take 119 us (280 us as 64
-// pixels x 64 channels a workgroup throughout).  Narrower layers whose 64
-// consecutive pixels form a rectangle of one image take k_conv3_mm, the rest
-// the unstaged kernels.
+// largest that leaves a workgroup for each of the 256 CUs (the large ones stage
+// less and read less LDS per MFMA; a layer with few pixels is bound by the
+// latency of its chunks, which only more workgroups hide).  A forward pass of 15
+// images of 32 x 256 takes 362 us with that line at one workgroup a CU, 371 at
+// two, 384 at four; the 14 products of one 256 x 256 image take 119 us (280 us as
+// 64 pixels x 64 channels a workgroup throughout).  Narrower layers whose 64
+// consecutive pixels form a rectangle of one image take k_conv3_mm, the rest the
+// unstaged kernels.
 template <bool DG>
 static void conv_product(mcl_net *n, const ConvShape &s, const uint16_t *X, const uint16_t *act, const uint16_t *Wt,
                          const float *bias, uint16_t *Y, int relu)
@@ -311,7 +311,7 @@ static Conv *convs(mcl_net *n, int i)
 }
 
 // One row of workgroups for each layer: 256 of 256 threads cover the largest
-// (590 080 parameters) in nine rounds.
+// (589 824 weights and 256 biases) in ten rounds, the last for the biases.
 static const dim3 update_grid(256, 15);
 
 static void weights_bf16(mcl_net *n)

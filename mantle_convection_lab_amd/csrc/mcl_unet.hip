@@ -533,8 +533,9 @@ __global__ void __launch_bounds__(256) k_conv3_wgrad(ConvShape s, const uint16_t
 // c x 9 taps (18 accumulators); it walks down the tile's rows and keeps the
 // fragments of three rows, so that a row costs 10 transposing reads for 18
 // MFMAs.  (Before, G was transposed and X copied three times with 2-byte LDS
-// writes: 399 us a layer at 256 x 256, batch 32, now 110.)  With NBLK = 32 two of the waves take the lower half of
-// the rows.  The next tile's loads are in flight while the products run.
+// writes: 399 us a layer at 256 x 256, batch 32, now 110.)  With NBLK = 32 two of
+// the waves take the lower half of the rows.  The next tile's loads are in flight
+// while the products run.
 typedef short bs4 __attribute__((ext_vector_type(4)));
 
 template <int ROWB>
@@ -676,10 +677,10 @@ template __global__ void k_conv3_wgrad_tile<32, 8>(ConvShape, const uint16_t *, 
 // transposed (channel-major, 64 pixels a row) and three copies of the X patch
 // shifted by -1, 0, +1 columns, channel-major, so that every operand fragment --
 // 8 consecutive pixels of one channel -- is one 16-byte LDS read; what bounds it
-// is that staging by 2-byte writes.  Requires TW % 8 == 0 (the host checks the
-// shapes).  A training step with these levels on the
-// unstaged kernel and on this one: 64 x 64, batch 32, 3.1 and 1.13 ms; 256 x 64,
-// batch 4, 2.6 and 0.89 ms; 512 x 16, batch 8, 7.1 and 3.0 ms.
+// is that staging by 2-byte writes (39 us a launch in a 64 x 64 network, batch
+// 32).  Requires TW % 8 == 0 (the host checks the shapes).  A training step with
+// these levels on the unstaged kernel and on this one: 64 x 64, batch 32, 3.1 and
+// 1.13 ms; 256 x 64, batch 4, 2.6 and 0.89 ms; 512 x 16, batch 8, 7.1 and 3.0 ms.
 constexpr int WG_XP = 72;   // bf16 words per staged G row (64 pixels + pad)
 
 __global__ void __launch_bounds__(256) k_conv3_wgrad_mm(ConvShape s, const uint16_t *__restrict__ dout,
@@ -984,11 +985,11 @@ __global__ void __launch_bounds__(256) k_head_bwd(int M, const uint16_t *__restr
 }
 
 // ----------------------------------------------------------------- Adam etc.
-// Adam (Kingma & Ba 2015) on FP32 master weights; refreshes the bf16 copies.
-// Adam step (STEP) and the bf16 weights of every layer from the FP32 masters
-// [co][tap][ci]: Wf ([co][tap][ci]) and Wd ([ci][tap][co]).  blockIdx.y is the
-// layer.  Bound by its launch: 7.8 MB of masters, moments and gradients a
-// buffer, where one launch a tensor for each of the two took 44.
+// Adam step (STEP; Kingma & Ba 2015) on the FP32 master weights [co][tap][ci],
+// and the bf16 weights of every layer from them: Wf ([co][tap][ci]) and Wd
+// ([ci][tap][co]).  blockIdx.y is the layer; one launch, where one a tensor for
+// each of the two took 44.  What bounds it is the rounds of the largest layer:
+// 24 to 35 us with the step, 28 without.
 template <bool STEP>
 __global__ void __launch_bounds__(256)
 k_update_weights(NetLayers ls, float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m1,
