@@ -513,11 +513,12 @@ __device__ __forceinline__ int pcg_rows(const LevelDev &L, const EllMat &A, cons
 
 // The form of a solve that does not keep its rows (more rows than threads, or
 // hanging nodes).  The fenced wait of CG_CACHED pays once a thread has more than
-// one velocity row of 18 slots, or more than two temperature rows of 9.  us an
+// one velocity row of 18 slots, or more than four temperature rows of 9.  us an
 // inner iteration, CG_GATHER / CG_CACHED: 128x128 on 32 workgroups (two rows a
 // thread) 22.8 / 18.1, on 8 74.9 / 46.5, on one 575 / 333; 512x512 on 256 (four
 // rows) 51.0 / 46.0; an adapted mesh of 43 390 equations with one row a thread
-// 20.7 / 21.5; temperature at 512x512 (two rows a thread) 49 / 55.
+// 20.7 / 21.5.  Temperature: 1024x512 on 256 workgroups (four rows a thread), a
+// step 294 / 302 us; that adapted mesh on 5 (eight rows), an iteration 133 / 115.
 template <int W>
 __device__ __forceinline__ int pcg_persistent(const LevelDev &L, const EllMat &A, const RowReg<W> &row,
                                               const Window &win, double diag, const double *__restrict__ b, double *x,
@@ -527,7 +528,7 @@ __device__ __forceinline__ int pcg_persistent(const LevelDev &L, const EllMat &A
     if (win.fits)
         return pcg_rows<W, CG_ROWS>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws, ok,
                                     spmv, exact);
-    if (A.n <= (kind + 1) * (int)(gridDim.x * blockDim.x))
+    if (A.n <= (kind == 0 ? 1 : 4) * (int)(gridDim.x * blockDim.x))
         return pcg_rows<W, CG_GATHER>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws,
                                       ok, spmv, exact);
     return pcg_rows<W, CG_CACHED>(L, A, row, win, diag, b, x, x_zero, accu, max_cycle, precond, kind, v, gs, ws, ok,
