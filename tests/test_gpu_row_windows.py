@@ -71,7 +71,7 @@ def _run(side, nproz, cap, **over):
 @pytest.mark.gpu
 @pytest.mark.parametrize("side,nproz,cap,over", [
     (32, 1, 1, {}),
-    (64, 1, 1, {}),
+    (64, 1, 1, dict(max_citcom_cycle=8)),
     (32, 1, 2, dict(exact_dots=1, max_citcom_cycle=10)),
     (16, 192, 60, dict(max_citcom_cycle=3, max_cg_cycle=60)),
 ])
